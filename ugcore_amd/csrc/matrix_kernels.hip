@@ -5,9 +5,9 @@
 //     rows list their entries by ascending source row, which is what the
 //     reference's row-by-row insertion into sorted rows produces;
 //   * the transposed product dest = a1*v1 + b1*A^T*w1 (axpy_transposed,
-//     sparsematrix_impl.h:341-370) over a cached transpose, one thread per
-//     transposed row accumulating in ascending source row as the reference's
-//     row loop does, skipping zero entries as the reference does;
+//     sparsematrix_impl.h:341-370) over a cached transpose, every transposed
+//     row accumulated in ascending source row as the reference's row loop
+//     does, skipping zero entries as the reference does;
 //   * Dirichlet rows (SetDirichletRow, algebra_common/sparsematrix_util.h:850-861);
 //   * value scaling.
 //
@@ -75,22 +75,65 @@ __global__ __launch_bounds__(256) void k_transpose_gather(int64_t n, const int32
 
 // dest[c] = a1*v1[c] (v1_is_dest: dest[c]*a1; a1 == 0: 0), then for the
 // entries of transposed row c in ascending source row r: dest[c] += (b1*a)*w[r]
-// for a != 0
+// for a != 0.
+// A workgroup owns kTRows consecutive rows, whose entries are one contiguous
+// run: all 256 threads bring the run into LDS (coefficient and gathered w
+// value, kTChunk at a time, coalesced, four loads in flight per thread), then
+// one thread per row adds its part in order, so the sums are those of a plain
+// row loop. Bound by the gathers of w. With one thread per row walking the
+// arrays directly the loads of a wave were spread over 64 rows: 400,003 rows of
+// about 16 entries, band 6000: 228 -> 46 us on one MI355X.
+constexpr int kTRows = 64, kTChunk = 1024;
+
 __global__ __launch_bounds__(256) void k_axpy_transposed(int64_t n, const int32_t* __restrict__ rp,
                                                          const int32_t* __restrict__ cl, const double* __restrict__ vl,
                                                          double a1, const double* v1, int v1_is_dest, double b1,
-                                                         const double* __restrict__ w, double* dest) {
-    const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (c >= n) return;
-    double d;
-    if (a1 == 0.0) d = 0.0;
-    else if (v1_is_dest) d = a1 == 1.0 ? dest[c] : dest[c] * a1;
-    else d = a1 * v1[c];
-    for (int32_t k = rp[c]; k < rp[c + 1]; ++k) {
-        const double a = vl[k];
-        if (a != 0.0) d = d + (b1 * a) * w[cl[k]];
+                                                         const double* __restrict__ w, double* dest, int64_t per_xcd) {
+    __shared__ double as[kTChunk], ws[kTChunk];
+    __shared__ int32_t rps[kTRows + 1];
+    // consecutive row blocks on one XCD: neighbouring rows read the same part of w
+    const int64_t lb = per_xcd ? (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
+    const int64_t c0 = lb * kTRows;
+    if (c0 >= n) return;
+    const int t = threadIdx.x;
+    if (t <= kTRows) rps[t] = rp[c0 + t < n ? c0 + t : n];
+    __syncthreads();
+    const int32_t begin = rps[0], end = rps[kTRows];
+    const int64_t c = c0 + t;
+    const bool owner = t < kTRows && c < n;
+    double d = 0.0;
+    if (owner && a1 != 0.0) {
+        if (v1_is_dest) d = a1 == 1.0 ? dest[c] : dest[c] * a1;
+        else d = a1 * v1[c];
     }
-    dest[c] = d;
+    const int32_t mine = owner ? rps[t] : 0, stop = owner ? rps[t + 1] : 0;
+    for (int64_t base = begin; base < end; base += kTChunk) {
+        constexpr int U = kTChunk / 256;
+        double a[U], x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t k = base + t + u * 256;
+            const bool in = k < end;
+            a[u] = in ? vl[k] : 0.0;
+            x[u] = in ? w[cl[k]] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            as[t + u * 256] = a[u];
+            ws[t + u * 256] = x[u];
+        }
+        __syncthreads();
+        if (owner) {
+            const int lo = (int)((mine > base ? mine : base) - base);
+            const int hi = (int)((stop < base + kTChunk ? stop : base + kTChunk) - base);
+            for (int k = lo; k < hi; ++k) {
+                const double av = as[k];
+                if (av != 0.0) d = d + (b1 * av) * ws[k];
+            }
+        }
+        __syncthreads();
+    }
+    if (owner) dest[c] = d;
 }
 
 // SetDirichletRow for every listed row: all entries 0, the diagonal 1 (the
@@ -164,8 +207,10 @@ int transpose_gather(int64_t n, const int32_t* idx_sorted, const int32_t* row_of
 int axpy_transposed(int64_t n, const int32_t* rp, const int32_t* cl, const double* vl, double a1, const double* v1,
                     bool v1_is_dest, double b1, const double* w, double* dest, hipStream_t s) {
     if (n <= 0) return 0;
-    hipLaunchKernelGGL(k_axpy_transposed, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, rp, cl, vl, a1, v1,
-                       v1_is_dest ? 1 : 0, b1, w, dest);
+    const int64_t nb = blocks_for(n, kTRows);
+    const int64_t per = nb >= 64 ? (nb + 7) / 8 : 0;
+    hipLaunchKernelGGL(k_axpy_transposed, dim3((unsigned)(per ? 8 * per : nb)), dim3(256), 0, s, n, rp, cl, vl, a1, v1,
+                       v1_is_dest ? 1 : 0, b1, w, dest, per);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
