@@ -433,9 +433,11 @@ class BiCGStab : public ILinearOperatorInverse {
 // P1 tetrahedra with FV1 and optional full-upwind convection, Q1 hexahedra with
 // FE (2x2x2 Gauss); -div(k grad u) (+ div(v u)) = f, k per element, f constant
 // or per DoF (hexahedra: constant), homogeneous Dirichlet values on the listed
-// DoFs. The CSR pattern (every element coupling, rows sorted), the CSR slot of
-// every local entry and an element colouring are built once on the device;
-// every assembly is one launch per colour without atomics (elem_assembly.hip).
+// DoFs. The CSR pattern (every element coupling, rows sorted), the local
+// entries of every CSR entry (Q2: the slot of every local entry) and an element
+// colouring are built once on the device; an assembly forms the local matrices
+// and adds them up per entry, Q2 in one launch per colour; no atomics
+// (elem_assembly.hip).
 class ElementDiscretization {
    public:
     enum ElemType { TRIANGLE_FV1 = 0, TETRAHEDRON_FV1 = 1, HEXAHEDRON_Q1 = 2, HEXAHEDRON_Q2 = 3 };
@@ -481,14 +483,19 @@ class ElementDiscretization {
 
    private:
     void build();
-    void run(double* val, double* rhs, const double* u, double* d);
+    // val and vec (each may be null): the matrix values and the right-hand
+    // side, or with u the defect sum_e (A_e u_e - f_e)
+    void run(double* val, double* vec, const double* u);
     // hands the pattern to A (true: A still held it from the last assembly)
     bool give_pattern(GPUSparseMatrix& A);
     void finish_matrix(GPUSparseMatrix& A, bool kept);
     uint64_t asm_pattern_id_ = 0;
     int type_, nv_, dim_;
     int64_t ne_, ndofs_, nnz_ = 0;
-    DeviceBuffer<int32_t> dofs_, rowptr_, col_, order_, slot_, dir_;
+    DeviceBuffer<int32_t> dofs_, rowptr_, col_, dir_;
+    DeviceBuffer<int32_t> order_, slot_;                   // Q2: elements by colour, slots
+    DeviceBuffer<int32_t> eptr_, src_, inc_ptr_, inc_t_;   // others: lists of local entries / vertices
+    DeviceBuffer<double> ke_, fe_;                         // workspace: local matrices and vectors
     DeviceBuffer<double> coords_, kel_, kq_, f_dof_;
     std::vector<int64_t> colour_start_;
     double f_const_ = 0.0;

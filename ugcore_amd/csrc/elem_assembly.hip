@@ -12,13 +12,23 @@
 //     keys. Rows come out sorted by column and every coupling is stored, also
 //     one whose value is zero, as AddLocalMatrixToGlobal's insertion
 //     (local_algebra.h:766-789) leaves them;
-//   * the slot of every local entry (e, a, b) in that CSR;
+//   * for every CSR entry the list of local entries (e, a, b) that make it up
+//     (the sorted positions of its key, elements ascending), and for every DoF
+//     the list of local vertices (e, a);
 //   * a colouring of the elements such that no two elements of one colour
 //     share a DoF (Jones-Plassmann rounds over the DoF -> element incidence,
 //     each local maximum of a hashed priority taking the lowest colour its
-//     coloured neighbours leave free), and the elements sorted by colour.
-// Each assembly then runs one launch per colour, one element per thread: the
-// local matrix in registers, added to its slots without atomics.
+//     coloured neighbours leave free), and for Q2 hexahedra the elements sorted
+//     by colour with the slot of every local entry.
+// An assembly of the other element types is two launches without atomics: all
+// local matrices (one element per thread) into a workspace, then one thread
+// per CSR entry and per DoF adds up its list in ascending element order. The
+// workspace (8 nv^2 bytes per element) is written and read once, mostly within
+// the caches; one launch per colour instead leaves the chip idle (tetrahedra
+// need about 27 colours) and reads and writes every value once per element.
+// 263,958 tetrahedra (48,132 DoFs), matrix, load vector and defect on one
+// MI355X: 786 us in colours, 120 us. Q2 hexahedra have 5.8 KB local matrices
+// from the matrix cores and keep the launch per colour.
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
@@ -153,6 +163,15 @@ __global__ void k_colour_keys(int64_t ne, const int32_t* __restrict__ colour, ui
     idx[e] = (int32_t)e;
 }
 
+// eptr[i] = first sorted position of entry i, i = 0..nnz (run_incl as above)
+__global__ void k_entry_ptr(int64_t n, const int32_t* __restrict__ head, const int32_t* __restrict__ run_incl,
+                            int32_t* __restrict__ eptr) {
+    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (k > n) return;
+    if (k == n) eptr[n > 0 ? run_incl[n - 1] : 0] = (int32_t)n;
+    else if (head[k]) eptr[run_incl[k] - 1] = (int32_t)k;
+}
+
 // slot[ab * ne + pos] = slot of local entry ab of the element at colour-sorted position pos
 __global__ void k_slots_by_position(int64_t ne, int nv2, const int32_t* __restrict__ order,
                                     const int32_t* __restrict__ slot_local, int32_t* __restrict__ slot) {
@@ -162,58 +181,40 @@ __global__ void k_slots_by_position(int64_t ne, int nv2, const int32_t* __restri
     for (int ab = 0; ab < nv2; ++ab) slot[(int64_t)ab * ne + pos] = slot_local[e * nv2 + ab];
 }
 
-struct ElemArgs {
-    int64_t ne;
-    const int32_t* order;
-    const int32_t* dofs;
-    const double* coords;
-    const double* kel;      // diffusion per element (null: 1)
-    double f_const;
-    const double* f_dof;    // source per DoF (null: f_const)
-    double vel[3];
-    int conv;
-    const int32_t* slot;
-    double* val;            // matrix values (null: no matrix)
-    double* rhs;            // right-hand side (null: none)
-    const double* u;        // defect mode: d += A_e u_e - f_e
-    double* d;
-};
-
 template <int NV, int DIM>
-__device__ __forceinline__ void load_element(const ElemArgs& A, int64_t e, int32_t* dof, double (*X)[DIM]) {
+__device__ __forceinline__ void load_element(const ElemLaunch& A, int64_t e, int32_t* dof, double (*X)[DIM]) {
     for (int a = 0; a < NV; ++a) {
         dof[a] = A.dofs[e * NV + a];
         for (int c = 0; c < DIM; ++c) X[a][c] = A.coords[(int64_t)dof[a] * DIM + c];
     }
 }
 
+// the element's results: Ke row by row, and fe or (with u) A_e u_e - f_e
 template <int NV>
-__device__ __forceinline__ void scatter(const ElemArgs& A, int64_t pos, const int32_t* dof, const double (*Ke)[NV],
-                                        const double* fe) {
-    if (A.val) {
+__device__ __forceinline__ void store_element(const ElemLaunch& A, int64_t e, const int32_t* dof,
+                                              const double (*Ke)[NV], double* fe) {
+    if (A.ke) {
+        double* k = A.ke + e * (NV * NV);
         for (int a = 0; a < NV; ++a)
-            for (int b = 0; b < NV; ++b) {
-                const int32_t k = A.slot[(int64_t)(a * NV + b) * A.ne + pos];
-                A.val[k] += Ke[a][b];
-            }
+            for (int b = 0; b < NV; ++b) k[a * NV + b] = Ke[a][b];
     }
-    if (A.rhs)
-        for (int a = 0; a < NV; ++a) A.rhs[dof[a]] += fe[a];
-    if (A.d) {
+    if (!A.fe) return;
+    if (A.u) {
+        double ue[NV];
+        for (int b = 0; b < NV; ++b) ue[b] = A.u[dof[b]];
         for (int a = 0; a < NV; ++a) {
             double s = 0.0;
-            for (int b = 0; b < NV; ++b) s += Ke[a][b] * A.u[dof[b]];
-            A.d[dof[a]] += s - fe[a];
+            for (int b = 0; b < NV; ++b) s += Ke[a][b] * ue[b];
+            fe[a] = s - fe[a];
         }
     }
+    for (int a = 0; a < NV; ++a) A.fe[e * NV + a] = fe[a];
 }
 
 // P1 triangle, FV1; source per scv: f * area / 3 (f per DoF or constant)
-__global__ __launch_bounds__(128) void k_elem_tri_fv1(ElemArgs A, int64_t pos0, int64_t cnt) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= cnt) return;
-    const int64_t pos = pos0 + t;
-    const int64_t e = A.order[pos];
+__global__ __launch_bounds__(128) void k_elem_tri_fv1(ElemLaunch A) {
+    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (e >= A.ne) return;
     int32_t dof[3];
     double X[3][2];
     load_element<3, 2>(A, e, dof, X);
@@ -221,15 +222,13 @@ __global__ __launch_bounds__(128) void k_elem_tri_fv1(ElemArgs A, int64_t pos0, 
     double Ke[3][3], area, fe[3];
     fv1_tri_element_k(X, [=](const double*) { return k; }, Ke, area);
     for (int a = 0; a < 3; ++a) fe[a] = (A.f_dof ? A.f_dof[dof[a]] : A.f_const) * (area / 3.0);
-    scatter<3>(A, pos, dof, Ke, fe);
+    store_element<3>(A, e, dof, Ke, fe);
 }
 
 // P1 tetrahedron, FV1 with optional full-upwind convection; source f * |scv|
-__global__ __launch_bounds__(128) void k_elem_tet_fv1(ElemArgs A, int64_t pos0, int64_t cnt) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= cnt) return;
-    const int64_t pos = pos0 + t;
-    const int64_t e = A.order[pos];
+__global__ __launch_bounds__(128) void k_elem_tet_fv1(ElemLaunch A) {
+    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (e >= A.ne) return;
     int32_t dof[4];
     double X[4][3];
     load_element<4, 3>(A, e, dof, X);
@@ -238,22 +237,53 @@ __global__ __launch_bounds__(128) void k_elem_tet_fv1(ElemArgs A, int64_t pos0, 
     double Ke[4][4], vol[4], fe[4];
     fv1_tet_element(X, kip, A.vel, A.conv != 0, Ke, vol);
     for (int a = 0; a < 4; ++a) fe[a] = (A.f_dof ? A.f_dof[dof[a]] : A.f_const) * vol[a];
-    scatter<4>(A, pos, dof, Ke, fe);
+    store_element<4>(A, e, dof, Ke, fe);
 }
 
 // Q1 hexahedron, FE (2x2x2 Gauss); source f_const * int phi
-__global__ __launch_bounds__(128) void k_elem_hex_q1(ElemArgs A, int64_t pos0, int64_t cnt) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= cnt) return;
-    const int64_t pos = pos0 + t;
-    const int64_t e = A.order[pos];
+__global__ __launch_bounds__(128) void k_elem_hex_q1(ElemLaunch A) {
+    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (e >= A.ne) return;
     int32_t dof[8];
     double X[8][3];
     load_element<8, 3>(A, e, dof, X);
     const double k = A.kel ? A.kel[e] : 1.0;
     double Ke[8][8], fe[8];
     q1_hex_element_k(X, [=](const double*) { return k; }, A.f_const, Ke, fe);
-    scatter<8>(A, pos, dof, Ke, fe);
+    store_element<8>(A, e, dof, Ke, fe);
+}
+
+// sum of part[list[k]], k in [lo, hi), in order; four loads in flight
+__device__ __forceinline__ double list_sum(int32_t lo, int32_t hi, const int32_t* __restrict__ list,
+                                           const double* __restrict__ part) {
+    double s = 0.0;
+    int32_t k = lo;
+    for (; k + 4 <= hi; k += 4) {
+        double v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = part[list[k + q]];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += v[q];
+    }
+    for (; k < hi; ++k) s += part[list[k]];
+    return s;
+}
+
+// val[i] = sum of the local entries of CSR entry i (the first nb_entries
+// workgroups); vec[v] = sum of the local vector entries of DoF v (the others)
+__global__ __launch_bounds__(256) void k_elem_gather(int64_t nnz, const int32_t* __restrict__ eptr,
+                                                     const int32_t* __restrict__ src, const double* __restrict__ ke,
+                                                     double* __restrict__ val, int64_t nb_entries, int64_t ndofs,
+                                                     const int32_t* __restrict__ inc_ptr,
+                                                     const int32_t* __restrict__ inc_t,
+                                                     const double* __restrict__ fe, double* __restrict__ vec) {
+    if (blockIdx.x < nb_entries) {
+        const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+        if (i < nnz) val[i] = list_sum(eptr[i], eptr[i + 1], src, ke);
+    } else {
+        const int64_t v = (blockIdx.x - nb_entries) * (int64_t)256 + threadIdx.x;
+        if (v < ndofs) vec[v] = list_sum(inc_ptr[v], inc_ptr[v + 1], inc_t, fe);
+    }
 }
 
 __global__ void k_zero_listed(int64_t n, const int32_t* __restrict__ idx, double* __restrict__ x) {
@@ -387,11 +417,14 @@ int elem_pattern(int64_t ne, int nv, int64_t ndofs, const int32_t* dofs, uint64_
 }
 
 int elem_pattern_fill(int64_t ne, int nv, const uint64_t* key2, const int32_t* idx2, const int32_t* head,
-                      const int32_t* run_incl, int32_t* col, int32_t* slot_local, hipStream_t s) {
+                      const int32_t* run_incl, int32_t* col, int32_t* slot_local, int32_t* eptr, hipStream_t s) {
     const int64_t n = ne * nv * nv;
-    if (n == 0) return 0;
-    hipLaunchKernelGGL(k_pattern_cols, dim3(blocks(n, 256)), dim3(256), 0, s, n, key2, head, run_incl, col);
-    hipLaunchKernelGGL(k_slot_of_local, dim3(blocks(n, 256)), dim3(256), 0, s, n, idx2, run_incl, slot_local);
+    if (eptr) hipLaunchKernelGGL(k_entry_ptr, dim3(blocks(n + 1, 256)), dim3(256), 0, s, n, head, run_incl, eptr);
+    if (n > 0) {
+        hipLaunchKernelGGL(k_pattern_cols, dim3(blocks(n, 256)), dim3(256), 0, s, n, key2, head, run_incl, col);
+        if (slot_local)
+            hipLaunchKernelGGL(k_slot_of_local, dim3(blocks(n, 256)), dim3(256), 0, s, n, idx2, run_incl, slot_local);
+    }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -453,31 +486,25 @@ int elem_slots_by_position(int64_t ne, int nv, const int32_t* order, const int32
 
 // ---- assembly ---------------------------------------------------------------------
 
-int elem_assemble_colour(int elem_type, const ElemLaunch& L, int64_t pos0, int64_t cnt, hipStream_t s) {
-    if (cnt <= 0) return 0;
-    ElemArgs A;
-    A.ne = L.ne;
-    A.order = L.order;
-    A.dofs = L.dofs;
-    A.coords = L.coords;
-    A.kel = L.kel;
-    A.f_const = L.f_const;
-    A.f_dof = L.f_dof;
-    for (int c = 0; c < 3; ++c) A.vel[c] = L.vel[c];
-    A.conv = L.conv;
-    A.slot = L.slot;
-    A.val = L.val;
-    A.rhs = L.rhs;
-    A.u = L.u;
-    A.d = L.d;
+int elem_local(int elem_type, const ElemLaunch& L, hipStream_t s) {
+    if (L.ne <= 0) return 0;
     if (elem_type == 0)
-        hipLaunchKernelGGL(k_elem_tri_fv1, dim3(blocks(cnt, 128)), dim3(128), 0, s, A, pos0, cnt);
+        hipLaunchKernelGGL(k_elem_tri_fv1, dim3(blocks(L.ne, 128)), dim3(128), 0, s, L);
     else if (elem_type == 1)
-        hipLaunchKernelGGL(k_elem_tet_fv1, dim3(blocks(cnt, 128)), dim3(128), 0, s, A, pos0, cnt);
+        hipLaunchKernelGGL(k_elem_tet_fv1, dim3(blocks(L.ne, 128)), dim3(128), 0, s, L);
     else if (elem_type == 2)
-        hipLaunchKernelGGL(k_elem_hex_q1, dim3(blocks(cnt, 128)), dim3(128), 0, s, A, pos0, cnt);
+        hipLaunchKernelGGL(k_elem_hex_q1, dim3(blocks(L.ne, 128)), dim3(128), 0, s, L);
     else
         return -1;
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int elem_gather(int64_t nnz, const int32_t* eptr, const int32_t* src, const double* ke, double* val, int64_t ndofs,
+                const int32_t* inc_ptr, const int32_t* inc_t, const double* fe, double* vec, hipStream_t s) {
+    const int64_t nbe = val ? (nnz + 255) / 256 : 0, nbv = vec ? (ndofs + 255) / 256 : 0;
+    if (nbe + nbv == 0) return 0;
+    hipLaunchKernelGGL(k_elem_gather, dim3((unsigned)(nbe + nbv)), dim3(256), 0, s, nnz, eptr, src, ke, val, nbe, ndofs,
+                       inc_ptr, inc_t, fe, vec);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

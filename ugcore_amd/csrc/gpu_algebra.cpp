@@ -1252,7 +1252,8 @@ void ElementDiscretization::build() {
     if (elem_pattern_temp_bytes(ne_, nv_, ndofs_, &sort_b, &scan_b) != 0)
         throw UGError("ElementDiscretization: sort set-up failed");
     DeviceBuffer<uint64_t> key(n), key2(n);
-    DeviceBuffer<int32_t> idx(n), idx2(n), head(n), run(n), nnz_dev(1), slot_local(n);
+    const bool q2 = type_ == HEXAHEDRON_Q2;
+    DeviceBuffer<int32_t> idx(n), idx2(n), head(n), run(n), nnz_dev(1), slot_local(q2 ? n : 0);
     DeviceBuffer<uint8_t> temp((int64_t)std::max(sort_b, scan_b));
     rowptr_.resize(ndofs_ + 1);
     UGX_LAUNCH(elem_pattern(ne_, nv_, ndofs_, dofs_.get(), key.get(), key2.get(), idx.get(), idx2.get(), head.get(),
@@ -1261,8 +1262,10 @@ void ElementDiscretization::build() {
     nnz_dev.download(&nnz, 1);
     nnz_ = nnz;
     col_.resize(nnz_);
+    if (!q2) eptr_.resize(nnz_ + 1);
     UGX_LAUNCH(elem_pattern_fill(ne_, nv_, key2.get(), idx2.get(), head.get(), run.get(), col_.get(),
-                                 slot_local.get(), c.stream));
+                                 q2 ? slot_local.get() : nullptr, q2 ? nullptr : eptr_.get(), c.stream));
+    if (!q2) src_ = std::move(idx2);
     key.release();
     key2.release();
     head.release();
@@ -1275,7 +1278,7 @@ void ElementDiscretization::build() {
     if (elem_incidence_temp_bytes(ni, ndofs_, &inc_b) != 0 || elem_incidence_temp_bytes(ne_, 64, &sort_b) != 0)
         throw UGError("ElementDiscretization: sort set-up failed");
     DeviceBuffer<uint32_t> ikey(std::max(ni, ne_)), ikey2(std::max(ni, ne_));
-    DeviceBuffer<int32_t> iidx(std::max(ni, ne_)), inc_t(ni), inc_ptr(ndofs_ + 1), colour(ne_), flags(2);
+    DeviceBuffer<int32_t> iidx(std::max(ni, ne_)), inc_t(ni), inc_ptr(ndofs_ + 1), colour(ne_), flags(2), order(ne_);
     DeviceBuffer<uint8_t> itemp((int64_t)std::max(inc_b, sort_b));
     UGX_LAUNCH(elem_incidence(ne_, nv_, ndofs_, dofs_.get(), ikey.get(), ikey2.get(), iidx.get(), inc_t.get(),
                               itemp.get(), inc_b, inc_ptr.get(), c.stream));
@@ -1297,15 +1300,20 @@ void ElementDiscretization::build() {
         colour.download(col_h.data(), ne_);
         for (int32_t x : col_h) ncol = std::max(ncol, x + 1);
     }
-    order_.resize(ne_);
     DeviceBuffer<int32_t> colour_ptr(ncol + 1);
-    UGX_LAUNCH(elem_colour_order(ne_, ncol, colour.get(), ikey.get(), ikey2.get(), iidx.get(), order_.get(),
+    UGX_LAUNCH(elem_colour_order(ne_, ncol, colour.get(), ikey.get(), ikey2.get(), iidx.get(), order.get(),
                                  itemp.get(), sort_b, colour_ptr.get(), c.stream));
     std::vector<int32_t> cp(ncol + 1);
     colour_ptr.download(cp.data(), ncol + 1);
     colour_start_.assign(cp.begin(), cp.end());
-    slot_.resize(n);
-    UGX_LAUNCH(elem_slots_by_position(ne_, nv_, order_.get(), slot_local.get(), slot_.get(), c.stream));
+    if (q2) {
+        order_ = std::move(order);
+        slot_.resize(n);
+        UGX_LAUNCH(elem_slots_by_position(ne_, nv_, order_.get(), slot_local.get(), slot_.get(), c.stream));
+    } else {
+        inc_ptr_ = std::move(inc_ptr);
+        inc_t_ = std::move(inc_t);
+    }
     sync();
 }
 
@@ -1368,34 +1376,37 @@ void ElementDiscretization::set_dirichlet_device(const int32_t* dofs_dev, int64_
     ndir_ = n;
 }
 
-void ElementDiscretization::run(double* val, double* rhs, const double* u, double* d) {
+void ElementDiscretization::run(double* val, double* vec, const double* u) {
     auto& c = context();
-    ugamd::ElemLaunch L;
-    L.ne = ne_;
-    L.order = order_.get();
-    L.dofs = dofs_.get();
-    L.coords = coords_.get();
-    L.kel = has_k_ ? kel_.get() : nullptr;
-    L.f_const = f_const_;
-    L.f_dof = has_f_dof_ ? f_dof_.get() : nullptr;
-    for (int k = 0; k < 3; ++k) L.vel[k] = vel_[k];
-    L.conv = conv_ ? 1 : 0;
-    L.slot = slot_.get();
-    L.val = val;
-    L.rhs = rhs;
-    L.u = u;
-    L.d = d;
+    const double* kel = has_k_ ? kel_.get() : nullptr;
     if (type_ == HEXAHEDRON_Q2) {
+        // summed up in memory; written, not scaled: fresh memory may hold NaN
+        if (val && nnz_ > 0) UGX_LAUNCH(vec_set<double>(nnz_, val, 0.0, c.stream));
+        if (vec) UGX_LAUNCH(vec_set<double>(ndofs_, vec, 0.0, c.stream));
         for (int col = 0; col + 1 < (int)colour_start_.size(); ++col)
-            UGX_LAUNCH(elem_assemble_q2_colour(ne_, order_.get(), dofs_.get(), coords_.get(), L.kel,
-                                               has_kq_ ? kq_.get() : nullptr, f_const_, slot_.get(), val, rhs,
+            UGX_LAUNCH(elem_assemble_q2_colour(ne_, order_.get(), dofs_.get(), coords_.get(), kel,
+                                               has_kq_ ? kq_.get() : nullptr, f_const_, slot_.get(), val, vec,
                                                colour_start_[col], colour_start_[col + 1] - colour_start_[col],
                                                c.stream));
         return;
     }
-    for (int col = 0; col + 1 < (int)colour_start_.size(); ++col)
-        UGX_LAUNCH(elem_assemble_colour(type_, L, colour_start_[col], colour_start_[col + 1] - colour_start_[col],
-                                        c.stream));
+    if (val) ke_.resize(ne_ * nv_ * nv_);
+    if (vec) fe_.resize(ne_ * nv_);
+    ugamd::ElemLaunch L;
+    L.ne = ne_;
+    L.dofs = dofs_.get();
+    L.coords = coords_.get();
+    L.kel = kel;
+    L.f_const = f_const_;
+    L.f_dof = has_f_dof_ ? f_dof_.get() : nullptr;
+    for (int k = 0; k < 3; ++k) L.vel[k] = vel_[k];
+    L.conv = conv_ ? 1 : 0;
+    L.u = u;
+    L.ke = val ? ke_.get() : nullptr;
+    L.fe = vec ? fe_.get() : nullptr;
+    UGX_LAUNCH(elem_local(type_, L, c.stream));
+    UGX_LAUNCH(elem_gather(nnz_, eptr_.get(), src_.get(), ke_.get(), val, ndofs_, inc_ptr_.get(), inc_t_.get(),
+                           fe_.get(), vec, c.stream));
 }
 
 bool ElementDiscretization::give_pattern(GPUSparseMatrix& A) {
@@ -1417,21 +1428,19 @@ void ElementDiscretization::finish_matrix(GPUSparseMatrix& A, bool kept) {
     A.set_origin(this);
     if (kept) A.refresh_layout_values();
     else A.build_spmv_layout();
+    sync();   // the values are there for readers on other streams too
     asm_pattern_id_ = A.pattern_id();
 }
 
 void ElementDiscretization::assemble_linear(GPUSparseMatrix& A, GPUVector& b) {
     auto& c = context();
     const bool kept = give_pattern(A);
-    if (nnz_ > 0) UGX_LAUNCH(vec_set<double>(nnz_, A.val(), 0.0, c.stream));   // fresh memory may hold NaN
     b.resize(ndofs_);
-    b.set(0.0);
-    run(A.val(), b.data(), nullptr, nullptr);
+    run(A.val(), b.data(), nullptr);
     if (ndir_ > 0) {
         UGX_LAUNCH(dirichlet_rows(ndir_, dir_.get(), A.rowptr(), A.col(), A.val(), c.stream));
         UGX_LAUNCH(zero_listed(ndir_, dir_.get(), b.data(), c.stream));
     }
-    sync();
     finish_matrix(A, kept);
 }
 
@@ -1439,10 +1448,8 @@ void ElementDiscretization::assemble_jacobian(GPUSparseMatrix& J, const GPUVecto
     if (u.size() != ndofs_) throw UGError("ElementDiscretization::assemble_jacobian: size mismatch");
     auto& c = context();
     const bool kept = give_pattern(J);
-    if (nnz_ > 0) UGX_LAUNCH(vec_set<double>(nnz_, J.val(), 0.0, c.stream));   // fresh memory may hold NaN
-    run(J.val(), nullptr, nullptr, nullptr);
+    run(J.val(), nullptr, nullptr);
     if (ndir_ > 0) UGX_LAUNCH(dirichlet_rows(ndir_, dir_.get(), J.rowptr(), J.col(), J.val(), c.stream));
-    sync();
     finish_matrix(J, kept);
 }
 
@@ -1458,8 +1465,7 @@ void ElementDiscretization::assemble_defect(GPUVector& d, const GPUVector& u) {
         assemble_linear(T, b);
         T.axpy(d, -1.0, b, 1.0, u);
     } else {
-        d.set(0.0);
-        run(nullptr, nullptr, u.data(), d.data());
+        run(nullptr, d.data(), u.data());
     }
     if (ndir_ > 0) UGX_LAUNCH(zero_listed(ndir_, dir_.get(), d.data(), context().stream));
 }

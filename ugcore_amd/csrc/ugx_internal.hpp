@@ -273,9 +273,12 @@ int elem_pattern_temp_bytes(int64_t ne, int nv, int64_t ndofs, size_t* sort_byte
 int elem_pattern(int64_t ne, int nv, int64_t ndofs, const int32_t* dofs, uint64_t* key, uint64_t* key2, int32_t* idx,
                  int32_t* idx2, int32_t* head, int32_t* run_incl, void* temp, size_t sort_bytes, size_t scan_bytes,
                  int32_t* rowptr, int32_t* nnz_dev, hipStream_t s);
-// the columns (nnz) and the CSR slot of every local entry (ne*nv*nv, index e*nv*nv + a*nv + b)
+// the columns (nnz) and, each unless null, the CSR slot of every local entry
+// (ne*nv*nv, index e*nv*nv + a*nv + b) and the first sorted position of every
+// entry (nnz + 1): entry i is the sum of the local entries idx2[eptr[i] ..
+// eptr[i+1]-1], elements ascending
 int elem_pattern_fill(int64_t ne, int nv, const uint64_t* key2, const int32_t* idx2, const int32_t* head,
-                      const int32_t* run_incl, int32_t* col, int32_t* slot_local, hipStream_t s);
+                      const int32_t* run_incl, int32_t* col, int32_t* slot_local, int32_t* eptr, hipStream_t s);
 int elem_incidence_temp_bytes(int64_t n, int64_t maxkey, size_t* bytes);
 // DoF -> incidences (t = e*nv + a) sorted by DoF: inc_ptr (ndofs + 1), inc_t (ne*nv)
 int elem_incidence(int64_t ne, int nv, int64_t ndofs, const int32_t* dofs, uint32_t* key, uint32_t* key2, int32_t* idx,
@@ -290,23 +293,24 @@ int elem_slots_by_position(int64_t ne, int nv, const int32_t* order, const int32
                            hipStream_t s);
 struct ElemLaunch {
     int64_t ne = 0;
-    const int32_t* order = nullptr;
     const int32_t* dofs = nullptr;
     const double* coords = nullptr;
-    const double* kel = nullptr;
+    const double* kel = nullptr;     // diffusion per element (null: 1)
     double f_const = 0.0;
-    const double* f_dof = nullptr;
+    const double* f_dof = nullptr;   // source per DoF (null: f_const)
     double vel[3] = {0.0, 0.0, 0.0};
     int conv = 0;
-    const int32_t* slot = nullptr;
-    double* val = nullptr;
-    double* rhs = nullptr;
-    const double* u = nullptr;
-    double* d = nullptr;
+    const double* u = nullptr;       // defect mode: fe = A_e u_e - f_e
+    double* ke = nullptr;            // local matrices [ne][nv][nv] (null: none)
+    double* fe = nullptr;            // local vectors [ne][nv] (null: none)
 };
-// one colour's elements (positions pos0 .. pos0+cnt-1 of the colour order);
-// elem_type 0 P1 triangle FV1, 1 P1 tetrahedron FV1, 2 Q1 hexahedron FE
-int elem_assemble_colour(int elem_type, const ElemLaunch& L, int64_t pos0, int64_t cnt, hipStream_t s);
+// local matrices and vectors of every element; elem_type 0 P1 triangle FV1,
+// 1 P1 tetrahedron FV1, 2 Q1 hexahedron FE
+int elem_local(int elem_type, const ElemLaunch& L, hipStream_t s);
+// val[i] (null: none) = sum of ke over the list of entry i; vec[v] (null: none)
+// = sum of fe over the local vertices of DoF v; both in ascending element order
+int elem_gather(int64_t nnz, const int32_t* eptr, const int32_t* src, const double* ke, double* val, int64_t ndofs,
+                const int32_t* inc_ptr, const int32_t* inc_t, const double* fe, double* vec, hipStream_t s);
 int zero_listed(int64_t n, const int32_t* idx, double* x, hipStream_t s);
 // Q2 hexahedra (27 DoFs in the local shape order of LagrangeLSFS<Hexahedron,
 // 2>): one colour, one element per wavefront (q2_kernels.hip); the
