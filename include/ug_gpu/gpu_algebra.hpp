@@ -15,7 +15,7 @@
 //   AssembledMultiGridCycle     lib_disc/operator/linear_operator/multi_grid_solver/mg_solver.h:82-590
 //   DomainDiscretization        lib_disc/spatial_disc/domain_disc.h:77,649 (structured device assembly)
 //
-// Device memory is owned by the objects (hipMalloc at set-up, never inside
+// Device memory is owned by the objects (taken at set-up, never inside
 // an iteration); all work is ordered on one HIP stream per process.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -49,15 +49,26 @@ DeviceContext& context();            // initialises the device on first use
 DeviceContext* context_if_ready();   // nullptr before the first context() (allocates nothing)
 void sync();
 
+// Device memory of the library's objects, from a pool of released blocks
+// (gpu_algebra.cpp, BlockPool). Internal buffers are used on the library's
+// stream only. shared(): a buffer whose address callers can see and use on
+// streams of their own; it is only given memory on which no work is pending,
+// and its release waits for the device, as hipFree does.
 template <typename T>
 class DeviceBuffer {
    public:
     DeviceBuffer() = default;
     explicit DeviceBuffer(int64_t n) { resize(n); }
+    static DeviceBuffer shared() {
+        DeviceBuffer b;
+        b.shared_ = true;
+        return b;
+    }
     ~DeviceBuffer() { release(); }
     DeviceBuffer(const DeviceBuffer&) = delete;
     DeviceBuffer& operator=(const DeviceBuffer&) = delete;
-    DeviceBuffer(DeviceBuffer&& o) noexcept : p_(o.p_), n_(o.n_) { o.p_ = nullptr; o.n_ = 0; }
+    DeviceBuffer(DeviceBuffer&& o) noexcept : p_(o.p_), n_(o.n_), shared_(o.shared_) { o.p_ = nullptr; o.n_ = 0; }
+    // between two internal buffers (or two shared ones)
     DeviceBuffer& operator=(DeviceBuffer&& o) noexcept {
         if (this != &o) { release(); p_ = o.p_; n_ = o.n_; o.p_ = nullptr; o.n_ = 0; }
         return *this;
@@ -73,6 +84,7 @@ class DeviceBuffer {
    private:
     T* p_ = nullptr;
     int64_t n_ = 0;
+    bool shared_ = false;
 };
 
 // ---------------------------------------------------------------------------
@@ -102,7 +114,7 @@ class GPUVector {
 
    private:
     int64_t n_ = 0;
-    DeviceBuffer<double> buf_;
+    DeviceBuffer<double> buf_ = DeviceBuffer<double>::shared();
 };
 
 // VecScaleAdd (operations_vec.h:55-63, 162-175)
@@ -252,8 +264,8 @@ class GPUSparseMatrix {
     mutable int64_t t_nnz_ = 0;
     mutable DeviceBuffer<int32_t> t_rowptr_, t_col_;
     mutable DeviceBuffer<double> t_val_;
-    DeviceBuffer<int32_t> rowptr_, col_;
-    DeviceBuffer<double> val_;
+    DeviceBuffer<int32_t> rowptr_ = DeviceBuffer<int32_t>::shared(), col_ = DeviceBuffer<int32_t>::shared();
+    DeviceBuffer<double> val_ = DeviceBuffer<double>::shared();
     bool sell_enabled_ = true, sell_valid_ = false;
     const void* origin_ = nullptr;
     uint64_t version_ = 0;
