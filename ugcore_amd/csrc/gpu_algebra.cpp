@@ -1939,6 +1939,11 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
     bool rap = false;            // Galerkin coarse operators R A P below the top level
     bool graphs = true;          // replay the lattice cycle from captured HIP graphs
     bool fuse_smoothing = true;  // matrix-free top level of the lattice entry: fused smoothing passes
+    // the levels [base, coarse_top] as one kernel where they fit one workgroup
+    // (V-cycles; coarse_top == base: none do)
+    CoarseCycle<T> coarse;
+    DeviceBuffer<T> coarse_constants;
+    int coarse_top = 0;
     struct CycleGraph {
         const void* key[5];
         hipGraphExec_t exec;
@@ -2128,6 +2133,40 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
             UGX_HIP(hipMemcpy(&bad, c.flag, sizeof(int), hipMemcpyDeviceToHost));
             if (bad && lev > base) throw UGError("GMG: Jacobi found a zero diagonal");
         }
+        plan_coarse_cycle();
+    }
+
+    // the finest level below the top whose V-cycle fits one workgroup
+    void plan_coarse_cycle() {
+        coarse_top = base;
+        for (int lev = std::min(top - 1, base + kCoarseMaxLevels); lev > base; --lev) {
+            CoarseCycle<T> c;
+            c.nl = lev - base;
+            for (int k = 0; k < c.nl; ++k) {
+                GmgLevel<T>& l = L[lev - k];
+                if (l.N > kCoarseRows) break;
+                c.L[k].W = l.W;
+                c.L[k].N = (int)l.N;
+                c.L[k].A = sym_ok ? l.A.get() : l.Afull.get();
+                c.L[k].g_dinv = l.dinv;
+                c.L[k].pcode = tets ? disc->level(lev - k).pcode.get() : nullptr;
+            }
+            c.Wb = L[base].W;
+            c.lu_n = lu_n;
+            c.Linv = lu_linvT.get();
+            c.Uinv = lu_uinvT.get();
+            c.perm = lu_perm.get();
+            c.nu1 = nu1;
+            c.nu2 = nu2;
+            if (L[lev].N <= kCoarseRows && coarse_levels_fit<T>(disc->kind(), c)) {
+                coarse_constants.resize(c.pack_n);
+                UGX_LAUNCH(coarse_pack<T>(disc->kind(), c, coarse_constants.get(), context().stream));
+                c.pack = coarse_constants.get();
+                coarse = c;
+                coarse_top = lev;
+                return;
+            }
+        }
     }
 
     // The reference updates the top-level defect once more after the last
@@ -2254,6 +2293,13 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
     void lmgc(int lev, int type, bool last) {
         if (lev == base) {
             base_solve(top);
+            return;
+        }
+        // a V-cycle's levels from here down, on its last visit, in one kernel
+        if (lev == coarse_top && type == AssembledMultiGridCycle::_V_ && last && sym == sym_ok) {
+            coarse.sd = L[lev].sd;
+            coarse.sc = L[lev].sc;
+            UGX_LAUNCH(coarse_cycle<T>(disc->kind(), coarse, context().stream));
             return;
         }
         presmooth_and_restriction(lev);

@@ -162,6 +162,40 @@ int restrict_defect(int dim, int Wc, int Wf, int64_t n_c, const TV* sdf, const u
 template <typename TV>
 int lu_solve(int n, const double* LinvT, const double* UinvT, const int32_t* perm, const TV* b, TV* x, hipStream_t s);
 
+// ---- the V-cycle below the large levels as one kernel (coarse_cycle.hip) ----
+constexpr int kCoarseMaxLevels = 6, kCoarseRows = 2304;
+template <typename T>
+struct CoarseLevel {
+    int W = 0, N = 0;
+    const T* A = nullptr;              // tiled diagonals: symmetric storage (kinds 0, 1) or all 27 (kind 2)
+    const T* g_dinv = nullptr;
+    const uint8_t* pcode = nullptr;    // kind 2: parent-edge codes of this level
+    int halo = 0, x = 0, x1 = 0, sd = 0, sc = 0, dinv = 0, a = -1;   // places in LDS (coarse_plan)
+};
+template <typename T>
+struct CoarseCycle {
+    int nl = 0;                        // smoothed levels, finest first
+    CoarseLevel<T> L[kCoarseMaxLevels];
+    int Wb = 0, lu_n = 0;              // base level and its LU solve
+    const double *Linv = nullptr, *Uinv = nullptr;
+    const int32_t* perm = nullptr;
+    int nu1 = 0, nu2 = 0;
+    const T* sd = nullptr;             // defect of the finest of the levels
+    T* sc = nullptr;                   // its correction, read and written
+    const T* pack = nullptr;           // the constants of the LDS image (coarse_pack), 16-byte aligned
+    int pack_n = 0, vec_end = 0, base_sd = 0, base_sc = 0, lu_bytes = 0;
+};
+// whether one workgroup can run these levels (fills in the LDS places)
+template <typename T>
+bool coarse_levels_fit(int kind, CoarseCycle<T>& c);
+// fills the constants of a plan that fits (pack: pack_n entries)
+template <typename T>
+int coarse_pack(int kind, const CoarseCycle<T>& c, T* pack, hipStream_t s);
+// sc += the V-cycle's correction for the defect sd, including the finest
+// level's last correction update
+template <typename T>
+int coarse_cycle(int kind, const CoarseCycle<T>& c, hipStream_t s);
+
 int invert_map(int64_t n, const int32_t* dof_of_lat, int32_t* lat_of_dof, hipStream_t s);
 int pattern_count(int dim, int W, int64_t n, const int32_t* lat_of_dof, int32_t* cnt, hipStream_t s);
 template <typename TM>
