@@ -240,6 +240,16 @@ class GPUSparseMatrix {
         sell_enabled_ = layout >= 1;
         build_spmv_layout();
     }
+    // the dictionary layout in another numbering of rows and columns (map: row
+    // or column -> its number there, a device array): slots and dictionary
+    bool dictionary_ready() const { return dict_valid_ && rows_ == cols_; }
+    void renumber_dictionary(const int32_t* map, DeviceBuffer<int32_t>& order, DeviceBuffer<int32_t>& dict) const;
+    // y = A x in that numbering; out[0] = (y, u), out[1] = (y, y) (device),
+    // part: dictionary_partials() doubles
+    int64_t dictionary_partials() const;
+    template <typename T>
+    void dictionary_product(const DeviceBuffer<int32_t>& order, const DeviceBuffer<int32_t>& dict, const T* x,
+                            double* y, const double* u, double* part, double* out) const;
     bool has_row_order() const { return rows_ > 0 && row_order_.size() == rows_; }
     int lanes() const { return lanes_; }
     void set_lanes(int g) {
@@ -431,9 +441,21 @@ class BiCGStab : public ILinearOperatorInverse {
     }
     void set_min_orthogonality(double m) { min_ortho_ = m; }
 
+    ~BiCGStab() override;
+
    private:
+    // the same iteration on lattice-ordered vectors: the cycle starts from the
+    // defect that the vector update wrote in its precision and is replayed as
+    // a graph, the operator product sums its dot products, and the host reads
+    // two scalars per half step
+    template <typename T>
+    bool apply_lattice(GPUVector& x, GPUVector& b, AssembledMultiGridCycle& gmg);
     int num_restarts_ = 0;
     double min_ortho_ = 0.0;
+    // lattice-path work space, kept across solves
+    DeviceBuffer<double> ws_x_, ws_r_, ws_r0_, ws_p_, ws_v_, ws_s_, ws_t_, ws_partial_, ws_sc_;
+    DeviceBuffer<int32_t> ws_order_, ws_dict_;
+    void* event_ = nullptr;   // the scalars of a half step have reached the host
 };
 
 // Element-loop assembly from caller-supplied connectivity: the element loop of
@@ -795,6 +817,14 @@ class AssembledMultiGridCycle : public ILinearIterator {
     // are FP64 buffers of N entries with `lattice_halo()` zero entries on
     // each side (allocated by the caller).
     bool lattice_ready(const GPUSparseMatrix& A) const;
+    // The cycle for solvers of non-symmetric problems on lattice vectors:
+    // krylov_cycle() turns the defect written to the level buffer `defect`
+    // (any entries, the correction zeroed) into `correction`, both N entries
+    // in the precision of the levels.
+    bool krylov_ready(const GPUSparseMatrix& A) const;
+    Precision precision() const { return prec_; }
+    void krylov_buffers(void*& defect, void*& correction);
+    void krylov_cycle();
     int64_t lattice_size() const;
     int64_t lattice_halo() const;
     const int32_t* dof_of_lattice() const;

@@ -801,6 +801,33 @@ void GPUSparseMatrix::axpy(GPUVector& dest, double a1, const GPUVector& v1, doub
                                              w1.data(), dest.data(), 0, lanes_, context().stream)));
 }
 
+void GPUSparseMatrix::renumber_dictionary(const int32_t* map, DeviceBuffer<int32_t>& order,
+                                          DeviceBuffer<int32_t>& dict) const {
+    auto& c = context();
+    order.resize(slice_order_.size());
+    dict.resize(d_dict_.size());
+    UGX_LAUNCH(renumber(order.size(), slice_order_.get(), map, order.get(), c.stream));
+    UGX_LAUNCH(renumber(dict.size(), d_dict_.get(), map, dict.get(), c.stream));
+}
+
+int64_t GPUSparseMatrix::dictionary_partials() const { return 2 * dict_spmv_blocks(slice_order_.size() / 64); }
+
+template <typename T>
+void GPUSparseMatrix::dictionary_product(const DeviceBuffer<int32_t>& order, const DeviceBuffer<int32_t>& dict,
+                                         const T* x, double* y, const double* u, double* part, double* out) const {
+    auto& c = context();
+    const int64_t ns = slice_order_.size() / 64;
+    UGX_LAUNCH(dict_spmv_dots<T>(rows_, ns, d_width_.get(), d_dptr_.get(), dict.get(), d_vptr_.get(), d_iptr_.get(),
+                                 d_val_.get(), d_idx_.get(), order.get(), x, y, u, part, c.stream));
+    UGX_LAUNCH(sum_arrays(2, (int)dict_spmv_blocks(ns), part, out, c.stream));
+}
+template void GPUSparseMatrix::dictionary_product<float>(const DeviceBuffer<int32_t>&, const DeviceBuffer<int32_t>&,
+                                                         const float*, double*, const double*, double*,
+                                                         double*) const;
+template void GPUSparseMatrix::dictionary_product<double>(const DeviceBuffer<int32_t>&, const DeviceBuffer<int32_t>&,
+                                                          const double*, double*, const double*, double*,
+                                                          double*) const;
+
 void GPUSparseMatrix::apply_ignore_zero_rows(GPUVector& dest, double beta, const GPUVector& w) const {
     require_device("apply_ignore_zero_rows");
     if (dict_valid_)
@@ -1087,7 +1114,108 @@ bool CG::apply_return_defect(GPUVector& x, GPUVector& b) {
     return conv_->post();
 }
 
+BiCGStab::~BiCGStab() {
+    if (event_) (void)hipEventDestroy((hipEvent_t)event_);
+}
+
+template <typename T>
+bool BiCGStab::apply_lattice(GPUVector& x, GPUVector& b, AssembledMultiGridCycle& gmg) {
+    // the steps, checks and their order are those of apply_return_defect
+    auto& c = context();
+    const GPUSparseMatrix& A = op_->get_matrix();
+    const int64_t N = b.size();
+    op_->apply_sub(b, x);
+    for (auto* w : {&ws_x_, &ws_r_, &ws_r0_, &ws_p_, &ws_v_, &ws_s_, &ws_t_}) w->resize(N);
+    ws_partial_.resize(std::max<int64_t>(A.dictionary_partials(), 2 * kBicgMaxBlocks));
+    ws_sc_.resize(8);
+    if (!event_) {
+        hipEvent_t e;
+        UGX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        event_ = (void*)e;
+    }
+    double *xl = ws_x_.get(), *r = ws_r_.get(), *r0 = ws_r0_.get(), *p = ws_p_.get(), *v = ws_v_.get(),
+           *s = ws_s_.get(), *t = ws_t_.get(), *part = ws_partial_.get(), *sc = ws_sc_.get();
+    void *vd = nullptr, *vc = nullptr;
+    gmg.krylov_buffers(vd, vc);
+    T *cd = static_cast<T*>(vd), *cc = static_cast<T*>(vc);
+    UGX_LAUNCH((permute_to<double, double>(N, gmg.dof_of_lattice(), x.data(), xl, c.stream)));
+    UGX_LAUNCH((permute_to<double, double>(N, gmg.dof_of_lattice(), b.data(), r, c.stream)));
+    A.renumber_dictionary(gmg.lattice_of_dof(), ws_order_, ws_dict_);
+    // scalars on the device: 0 (v, r0), 1 (v, v), 2 (s, s), 3 (t, s), 4 (t, t), 5 (r, r), 6 (r0, r)
+    auto read = [&](int first, int n) {
+        UGX_HIP(hipMemcpyAsync(c.red_host, sc + first, sizeof(double) * n, hipMemcpyDeviceToHost, c.stream));
+    };
+    conv_->set_name(name());
+    double rr = dev_dot(N, r, r, false), r0r = rr;
+    conv_->start_defect(std::sqrt(rr));
+    double rho = 1, alpha = 1, omega = 1, norm_r0 = 0.0;
+    bool restart = true, ok = true;
+    const double* defect = r;
+    while (!conv_->iteration_ended()) {
+        if (num_restarts_ > 0 && conv_->step() % num_restarts_ == 0) restart = true;
+        const bool first = restart;
+        if (restart) {
+            alpha = 0.0;
+            omega = 1.0;
+            rho = 1.0;
+            norm_r0 = conv_->defect();
+            restart = false;
+            r0r = rr;   // r0 = r
+        }
+        const double rho_old = rho;
+        rho = r0r;
+        const double norm_r = conv_->defect();
+        if (std::fabs(rho) / (norm_r * norm_r0) <= min_ortho_) restart = true;
+        ok = rho_old != 0.0;
+        if (!ok) break;
+        const double beta = (rho / rho_old) * (alpha / omega);
+        UGX_LAUNCH(bicg_p<T>(N, first, beta, omega, r, p, v, r0, cd, cc, c.stream));
+        gmg.krylov_cycle();                                                            // q = B p
+        A.dictionary_product<T>(ws_order_, ws_dict_, cc, v, r0, part, sc + 0);         // v = A q
+        UGX_LAUNCH(bicg_s<T>(N, rho, sc + 0, r, v, cc, s, xl, part, sc + 2, cd, cc, c.stream));
+        read(0, 3);
+        UGX_HIP(hipEventRecord((hipEvent_t)event_, c.stream));
+        // the second half is queued before the host has looked at (s, s): where
+        // the iteration ends there, it has only written scratch
+        gmg.krylov_cycle();                                                            // q = B s
+        A.dictionary_product<T>(ws_order_, ws_dict_, cc, t, s, part, sc + 3);          // t = A q
+        UGX_HIP(hipEventSynchronize((hipEvent_t)event_));
+        alpha = c.red_host[0];
+        ok = alpha != 0.0;
+        if (!ok) break;
+        alpha = rho / alpha;
+        conv_->update_defect(std::sqrt(c.red_host[2]));
+        if (conv_->iteration_ended()) {
+            defect = s;
+            break;
+        }
+        UGX_LAUNCH(bicg_r<T>(N, sc + 3, s, t, cc, r0, r, xl, part, sc + 5, c.stream));
+        read(3, 4);
+        sync();
+        const double tt = c.red_host[1];
+        omega = c.red_host[0];
+        ok = tt != 0.0;
+        if (!ok) break;
+        omega = omega / tt;
+        rr = c.red_host[2];
+        r0r = c.red_host[3];
+        conv_->update_defect(std::sqrt(rr));
+        ok = omega != 0.0;
+        if (!ok) break;
+    }
+    UGX_LAUNCH((permute_scatter<double, double>(N, gmg.dof_of_lattice(), xl, x.data(), c.stream)));
+    UGX_LAUNCH((permute_scatter<double, double>(N, gmg.dof_of_lattice(), defect, b.data(), c.stream)));
+    sync();
+    return ok && conv_->post();
+}
+
 bool BiCGStab::apply_return_defect(GPUVector& x, GPUVector& b) {
+    if (auto* gmg = dynamic_cast<AssembledMultiGridCycle*>(precond_.get())) {
+        const GPUSparseMatrix& A = op_->get_matrix();
+        if (gmg->krylov_ready(A) && A.dictionary_ready() && b.size() == A.num_rows() && x.size() == A.num_rows())
+            return gmg->precision() == Precision::F32 ? apply_lattice<float>(x, b, *gmg)
+                                                      : apply_lattice<double>(x, b, *gmg);
+    }
     // bicgstab.h:112-385 (restart every num_restarts_ steps and when the
     // orthogonality of r to r0 drops to min_ortho_, bicgstab.h:157-215)
     op_->apply_sub(b, x);
@@ -1836,6 +1964,8 @@ struct AssembledMultiGridCycle::Impl {
     virtual void apply_lattice(double* c_lat, const double* d_lat, double* cd_out, double* partial,
                                const float* d_lat_f32) = 0;
     virtual bool uses_f32_defect() const = 0;
+    virtual void cycle_buffers(void*& defect, void*& correction) = 0;
+    virtual void run_cycle() = 0;
     virtual bool surface_axpy(double* y, double alpha, const double* v, double beta, const double* x, double* yx_out,
                               double* partial) = 0;
     virtual bool surface_direction_axpy(double* q, const double* p_old, const double* z, const double* beta,
@@ -1949,9 +2079,15 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         hipGraphExec_t exec;
     };
     std::vector<CycleGraph> cycle_graphs;
+    // the cycle between two level buffers (krylov_cycle) and its graph
+    T* cycle_in = nullptr;
+    hipGraphExec_t cycle_exec = nullptr;
     void clear_graphs() {
         for (auto& g : cycle_graphs) (void)hipGraphExecDestroy(g.exec);
         cycle_graphs.clear();
+        if (cycle_exec) (void)hipGraphExecDestroy(cycle_exec);
+        cycle_exec = nullptr;
+        cycle_in = nullptr;
     }
     ~GmgImpl() override { clear_graphs(); }
 
@@ -2229,11 +2365,9 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
             std::swap(f.sd, f.sd2);
         }
         if (tets) {
-            UGX_LAUNCH(vec_set<T>(cl.N, cl.sc, 0.0, c.stream));
-            UGX_LAUNCH(restrict_tet<T>(cl.W, f.W, cl.N, f.sd, disc->level(lev).pcode.get(), cl.dir, f.dir, cl.sd,
-                                       c.stream));
-        } else {
             // the restriction also clears the coarse correction
+            UGX_LAUNCH(restrict_tet<T>(cl.W, f.W, cl.N, f.sd, disc->level(lev).pcode.get(), cl.sd, cl.sc, c.stream));
+        } else {
             UGX_LAUNCH(restrict_defect<T>(f.dim, cl.W, f.W, cl.N, f.sd, cl.dir, f.dir, cl.sd, c.stream, cl.sc));
         }
     }
@@ -2323,7 +2457,7 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         // reference workflow (adjusted solution and rhs); otherwise the full
         // level storage is used
         double tail = 0.0;
-        if (G.N > G.n_inner) {
+        if (sym_ok && G.N > G.n_inner) {
             UGX_LAUNCH(dot<double>(G.N - G.n_inner, d.data() + G.n_inner, d.data() + G.n_inner, c.red_partial,
                                    c.red_out, false, c.stream));
             UGX_HIP(hipMemcpyAsync(c.red_host, c.red_out, sizeof(double), hipMemcpyDeviceToHost, c.stream));
@@ -2429,6 +2563,52 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         UGX_HIP(hipGraphLaunch(exec, c.stream));
     }
 
+    void cycle_buffers(void*& defect, void*& correction) override {
+        if (!cycle_in) cycle_in = L[top].sd;
+        defect = cycle_in;
+        correction = L[top].sc;
+    }
+
+    void launch_cycle() {
+        GmgLevel<T>& t = L[top];
+        if (t.sd != cycle_in) std::swap(t.sd, t.sd2);   // an odd number of smoothing steps leaves them swapped
+        sym = sym_ok;
+        try {
+            lmgc(top, cycle, true);
+        } catch (...) {
+            clear_cycle_state();
+            throw;
+        }
+    }
+
+    // no host decisions between the two buffers: one graph for every call
+    void run_cycle() override {
+        auto& c = context();
+        if (!graphs) {
+            launch_cycle();
+            return;
+        }
+        if (!cycle_exec) {
+            UGX_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
+            hipGraph_t graph = nullptr;
+            try {
+                launch_cycle();
+            } catch (...) {
+                (void)hipStreamEndCapture(c.stream, &graph);
+                if (graph) (void)hipGraphDestroy(graph);
+                throw;
+            }
+            UGX_HIP(hipStreamEndCapture(c.stream, &graph));
+            const hipError_t e = hipGraphInstantiate(&cycle_exec, graph, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(graph);
+            if (e != hipSuccess) {
+                cycle_exec = nullptr;
+                throw UGError(std::string("GMG: graph instantiation failed: ") + hipGetErrorString(e));
+            }
+        }
+        UGX_HIP(hipGraphLaunch(cycle_exec, c.stream));
+    }
+
     bool surface_axpy(double* y, double alpha, const double* v, double beta, const double* x, double* yx_out,
                       double* partial) override {
         GmgLevel<T>& t = L[top];
@@ -2512,6 +2692,18 @@ AssembledMultiGridCycle::~AssembledMultiGridCycle() { delete impl_; }
 bool AssembledMultiGridCycle::lattice_ready(const GPUSparseMatrix& A) const {
     return impl_ && !transposed_ && disc_->symmetric() && mat_ == &A && A.version() == mat_version_ &&
            A.origin() == disc_.get();
+}
+bool AssembledMultiGridCycle::krylov_ready(const GPUSparseMatrix& A) const {
+    return impl_ && !transposed_ && !disc_->symmetric() && mat_ == &A && A.version() == mat_version_ &&
+           A.origin() == disc_.get();
+}
+void AssembledMultiGridCycle::krylov_buffers(void*& defect, void*& correction) {
+    if (!impl_) throw UGError("GMG: not initialised");
+    impl_->cycle_buffers(defect, correction);
+}
+void AssembledMultiGridCycle::krylov_cycle() {
+    if (!impl_) throw UGError("GMG: not initialised");
+    impl_->run_cycle();
 }
 int64_t AssembledMultiGridCycle::lattice_size() const { return disc_->level(disc_->top_level()).N; }
 int64_t AssembledMultiGridCycle::lattice_halo() const { return impl_ ? impl_->halo() : 0; }

@@ -294,31 +294,71 @@ __global__ __launch_bounds__(64) void k_dict_values(int64_t nrows, const int32_t
 }
 
 // y = alpha*v1 + beta*A*x (mode 0), or y = beta*A*x on rows with entries
-// (mode 1); one wave per slice, four slices per workgroup
+// (mode 1); one wave per slice, four slices per workgroup.
+// Bound by HBM: 9 bytes per entry and the dictionaries. Two things keep the
+// stream busy: the first kPre entries of every row and the row numbers are
+// requested before the dictionary and x (a chain of three dependent loads and
+// a barrier that the values do not depend on), and consecutive slices run on
+// one XCD, so the x values that neighbouring lattice blocks share are fetched
+// by one L2 instead of eight. One MI355X: the operator of 97^3 tetrahedral rows
+// 41 us without the two, 37 us with them and the partials below; the 257^3 Q1
+// operator runs at the stream's rate either way (990 us).
+// DOTS (mode 0): also the workgroup's partial sums of (y, u) and (y, y), in
+// part[block] and part[blocks + block]. x may be FP32 (converted as it is
+// staged); dict and order may number the columns and rows differently from
+// the matrix's own numbering (order and x, y then share that numbering).
+template <typename XT, bool DOTS>
 __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslices, const int32_t* __restrict__ width,
                                                    const int32_t* __restrict__ dptr, const int32_t* __restrict__ dict,
                                                    const int64_t* __restrict__ vptr, const int64_t* __restrict__ iptr,
                                                    const double* __restrict__ sval, const uint32_t* __restrict__ sidx,
                                                    const int32_t* __restrict__ order, double alpha, const double* v1,
-                                                   double beta, const double* __restrict__ x, double* y, int mode,
-                                                   const int32_t* __restrict__ rowptr) {
+                                                   double beta, const XT* __restrict__ x, double* y, int mode,
+                                                   const int32_t* __restrict__ rowptr, int64_t per_xcd,
+                                                   const double* __restrict__ u, double* __restrict__ part) {
     __shared__ double xl[4][256];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t t = (int64_t)blockIdx.x * 4 + wave;
+    const int64_t lb = per_xcd ? (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
+    const int64_t t = lb * 4 + wave;
     double* xs = xl[wave];
-    int w = 0;
-    if (t < nslices) {
-        const int32_t d0 = dptr[t], u = dptr[t + 1] - d0;
-        for (int j = lane; j < u; j += 64) xs[j] = x[dict[d0 + j]];
-        if (lane == 0) xs[255] = 0.0;
-        w = width[t];
+    const bool live = t < nslices;
+    const int w = live ? width[t] : 0;
+    const dbl2* vp = reinterpret_cast<const dbl2*>(sval + (live ? vptr[t] : 0)) + lane;
+    const uint32_t* ip = sidx + (live ? iptr[t] : 0) + lane;
+    const int32_t r = live ? order[t * 64 + lane] : -1;
+    constexpr int kPre = 8;
+    uint32_t pw[kPre / 4];
+    dbl2 pv[kPre / 2];
+    const bool pre = w >= kPre;   // the same for every lane of the wave
+    if (pre) {
+#pragma unroll
+        for (int q = 0; q < kPre / 4; ++q) pw[q] = __builtin_nontemporal_load(ip + 64 * q);
+#pragma unroll
+        for (int q = 0; q < kPre / 2; ++q) pv[q] = __builtin_nontemporal_load(vp + 64 * q);
     }
+    if (live) {
+        const int32_t d0 = dptr[t], nd = dptr[t + 1] - d0;
+        for (int j = lane; j < nd; j += 64) xs[j] = (double)x[dict[d0 + j]];
+        if (lane == 0) xs[255] = 0.0;
+    }
+    const bool mine = r >= 0 && r < nrows;
+    double ur = 0.0;
+    if (DOTS) ur = mine ? u[r] : 0.0;
     __syncthreads();
-    if (t >= nslices) return;
-    const dbl2* vp = reinterpret_cast<const dbl2*>(sval + vptr[t]) + lane;
-    const uint32_t* ip = sidx + iptr[t] + lane;
+    if (!DOTS && !live) return;
     double s0 = 0.0, s1 = 0.0;
     int k = 0;
+    if (pre) {
+#pragma unroll
+        for (int q = 0; q < kPre / 4; ++q) {
+            const uint32_t word = pw[q];
+            s0 = fma(pv[2 * q].x, xs[word & 255u], s0);
+            s1 = fma(pv[2 * q].y, xs[(word >> 8) & 255u], s1);
+            s0 = fma(pv[2 * q + 1].x, xs[(word >> 16) & 255u], s0);
+            s1 = fma(pv[2 * q + 1].y, xs[word >> 24], s1);
+        }
+        k = kPre;
+    }
     for (; k + 4 <= w; k += 4) {
         const uint32_t word = __builtin_nontemporal_load(ip + 64 * (k >> 2));
         const dbl2 a = __builtin_nontemporal_load(vp + 64 * (k >> 1));
@@ -340,9 +380,28 @@ __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslice
             s0 = fma(b.x, xs[(word >> 16) & 255u], s0);
         }
     }
-    const int32_t r = order[t * 64 + lane];
-    if (r < 0 || r >= nrows) return;
     const double sum = s0 + s1;
+    if (DOTS) {
+        // mode 0 without v1: y = beta A x
+        double yr = mine ? 0.0 + beta * sum : 0.0, yu = yr * ur, yy = yr * yr;
+        if (mine) y[r] = yr;
+        for (int o = 32; o > 0; o >>= 1) {
+            yu += __shfl_down(yu, o, 64);
+            yy += __shfl_down(yy, o, 64);
+        }
+        __shared__ double sh[2][4];
+        if (lane == 0) {
+            sh[0][wave] = yu;
+            sh[1][wave] = yy;
+        }
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            const double* q = sh[threadIdx.x];
+            part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = (q[0] + q[1]) + (q[2] + q[3]);
+        }
+        return;
+    }
+    if (!mine) return;
     if (mode == 1) {
         if (rowptr[r + 1] > rowptr[r]) y[r] = beta * sum;
     } else {
@@ -428,10 +487,35 @@ int dict_spmv(int64_t nrows, int64_t nslices, const int32_t* width, const int32_
               const int32_t* order, double alpha, const double* v1, double beta, const double* x, double* y, int mode,
               const int32_t* rowptr, hipStream_t s) {
     if (nslices <= 0) return 0;
-    hipLaunchKernelGGL(k_dict_spmv, dim3(nblk(nslices, 4)), dim3(256), 0, s, nrows, nslices, width, dptr, dict, vptr,
-                       iptr, sval, sidx, order, alpha, v1, beta, x, y, mode, rowptr);
+    const int64_t nb = (nslices + 3) / 4, per = nb >= 64 ? (nb + 7) / 8 : 0;
+    hipLaunchKernelGGL((k_dict_spmv<double, false>), dim3((unsigned)dict_spmv_blocks(nslices)), dim3(256), 0, s, nrows,
+                       nslices, width, dptr, dict, vptr, iptr, sval, sidx, order, alpha, v1, beta, x, y, mode, rowptr,
+                       per, (const double*)nullptr, (double*)nullptr);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
+
+int64_t dict_spmv_blocks(int64_t nslices) {
+    const int64_t nb = (nslices + 3) / 4;
+    return nb >= 64 ? (nb + 7) / 8 * 8 : nb;
+}
+
+template <typename XT>
+int dict_spmv_dots(int64_t nrows, int64_t nslices, const int32_t* width, const int32_t* dptr, const int32_t* dict,
+                   const int64_t* vptr, const int64_t* iptr, const double* sval, const uint32_t* sidx,
+                   const int32_t* order, const XT* x, double* y, const double* u, double* part, hipStream_t s) {
+    if (nslices <= 0) return -1;
+    const int64_t nb = (nslices + 3) / 4, per = nb >= 64 ? (nb + 7) / 8 : 0;
+    hipLaunchKernelGGL((k_dict_spmv<XT, true>), dim3((unsigned)dict_spmv_blocks(nslices)), dim3(256), 0, s, nrows,
+                       nslices, width, dptr, dict, vptr, iptr, sval, sidx, order, 0.0, (const double*)nullptr, 1.0, x,
+                       y, 0, (const int32_t*)nullptr, per, u, part);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+template int dict_spmv_dots<float>(int64_t, int64_t, const int32_t*, const int32_t*, const int32_t*, const int64_t*,
+                                   const int64_t*, const double*, const uint32_t*, const int32_t*, const float*,
+                                   double*, const double*, double*, hipStream_t);
+template int dict_spmv_dots<double>(int64_t, int64_t, const int32_t*, const int32_t*, const int32_t*, const int64_t*,
+                                    const int64_t*, const double*, const uint32_t*, const int32_t*, const double*,
+                                    double*, const double*, double*, hipStream_t);
 
 int64_t lattice_block_slots(int dim, int W) {
     const int e = dim == 3 ? 4 : 8;

@@ -281,29 +281,37 @@ __global__ __launch_bounds__(256) void k_prolong_add_tet(int Wc, int Wf, int64_t
     sc[i] = sc[i] + t;
 }
 
+// The Dirichlet points are the lattice boundary: a coarse boundary point takes
+// the value of its fine copy, and the fine neighbours of the others lie inside
+// the lattice and off its boundary. All codes and values of a point are loaded
+// before the first is looked at (loads behind branches ran one after another:
+// 97^3 -> 49^3 19 us, 4.7 us so). zc: the coarse correction, set to zero.
 template <typename TV>
 __global__ __launch_bounds__(256) void k_restrict_tet(int Wc, int Wf, int64_t n_c, const TV* __restrict__ sdf,
-                                                      const uint8_t* __restrict__ pcode,
-                                                      const uint8_t* __restrict__ dir_c,
-                                                      const uint8_t* __restrict__ dir_f, TV* __restrict__ sdc) {
+                                                      const uint8_t* __restrict__ pcode, TV* __restrict__ sdc,
+                                                      TV* __restrict__ zc) {
     const int64_t c = blockIdx.x * (int64_t)256 + threadIdx.x;
     if (c >= n_c) return;
     const int x = (int)(c % Wc), y = (int)((c / Wc) % Wc), z = (int)(c / ((int64_t)Wc * Wc));
     const int64_t f0 = ((int64_t)(2 * z) * Wf + 2 * y) * Wf + 2 * x;
-    if (dir_c[c]) {
+    zc[c] = (TV)0;
+    if (x == 0 || y == 0 || z == 0 || x == Wc - 1 || y == Wc - 1 || z == Wc - 1) {
         sdc[c] = sdf[f0];
         return;
     }
-    double acc = (double)sdf[f0];
+    uint8_t code[27];
+    TV val[27];
+#pragma unroll
+    for (int d = 0; d < 27; ++d) {
+        const int64_t f = f0 + ((int64_t)(d / 9 - 1) * Wf + (d / 3) % 3 - 1) * Wf + d % 3 - 1;
+        code[d] = pcode[f];
+        val[d] = sdf[f];
+    }
+    double acc = (double)val[13];
+#pragma unroll
     for (int d = 0; d < 27; ++d) {
         if (d == 13) continue;
-        const int dx = d % 3 - 1, dy = (d / 3) % 3 - 1, dz = d / 9 - 1;
-        const int fx = 2 * x + dx, fy = 2 * y + dy, fz = 2 * z + dz;
-        if (fx < 0 || fy < 0 || fz < 0 || fx >= Wf || fy >= Wf || fz >= Wf) continue;
-        const int64_t f = ((int64_t)fz * Wf + fy) * Wf + fx;
-        const int code = d > 13 ? d - 13 : 13 - d;
-        if (pcode[f] != code || dir_f[f]) continue;
-        acc += 0.5 * (double)sdf[f];
+        if (code[d] == (d > 13 ? d - 13 : 13 - d)) acc += 0.5 * (double)val[d];
     }
     sdc[c] = (TV)acc;
 }
@@ -432,17 +440,14 @@ template int prolong_add_tet<float>(int, int, int64_t, const float*, const uint8
                                     hipStream_t);
 
 template <typename TV>
-int restrict_tet(int Wc, int Wf, int64_t n_c, const TV* sdf, const uint8_t* pcode, const uint8_t* dir_c,
-                 const uint8_t* dir_f, TV* sdc, hipStream_t s) {
+int restrict_tet(int Wc, int Wf, int64_t n_c, const TV* sdf, const uint8_t* pcode, TV* sdc, TV* zero_c, hipStream_t s) {
     if (n_c <= 0) return 0;
     hipLaunchKernelGGL(k_restrict_tet<TV>, dim3((unsigned)((n_c + 255) / 256)), dim3(256), 0, s, Wc, Wf, n_c, sdf,
-                       pcode, dir_c, dir_f, sdc);
+                       pcode, sdc, zero_c);
     UGX_TET_CHECK();
 }
-template int restrict_tet<double>(int, int, int64_t, const double*, const uint8_t*, const uint8_t*, const uint8_t*,
-                                  double*, hipStream_t);
-template int restrict_tet<float>(int, int, int64_t, const float*, const uint8_t*, const uint8_t*, const uint8_t*,
-                                 float*, hipStream_t);
+template int restrict_tet<double>(int, int, int64_t, const double*, const uint8_t*, double*, double*, hipStream_t);
+template int restrict_tet<float>(int, int, int64_t, const float*, const uint8_t*, float*, float*, hipStream_t);
 
 template <typename T>
 int dia_transpose_elim(int W, int64_t n, const uint8_t* dir, const T* A, T* AT, hipStream_t s) {

@@ -257,8 +257,7 @@ template <typename TV>
 int prolong_add_tet(int Wc, int Wf, int64_t n_f, const TV* scc, const uint8_t* pcode, const uint8_t* dir_f, TV* st,
                     TV* sc, hipStream_t s);
 template <typename TV>
-int restrict_tet(int Wc, int Wf, int64_t n_c, const TV* sdf, const uint8_t* pcode, const uint8_t* dir_c,
-                 const uint8_t* dir_f, TV* sdc, hipStream_t s);
+int restrict_tet(int Wc, int Wf, int64_t n_c, const TV* sdf, const uint8_t* pcode, TV* sdc, TV* zero_c, hipStream_t s);
 // Galerkin coarse operator R A_f P of the P1 lattice transfer (dim 3: 27
 // diagonals, dim 2: 9), tiled DIA storage, FP64; Wf = 2 Wc - 1
 int rap_dia(int dim, int Wf, int Wc, const uint8_t* dir_f, const uint8_t* dir_c, const double* Af, double* Ac,
@@ -421,6 +420,29 @@ int dict_spmv(int64_t nrows, int64_t nslices, const int32_t* width, const int32_
               const int64_t* vptr, const int64_t* iptr, const double* sval, const uint32_t* sidx,
               const int32_t* order, double alpha, const double* v1, double beta, const double* x, double* y, int mode,
               const int32_t* rowptr, hipStream_t s);
+// workgroups of a dictionary product (partial sums per array of dict_spmv_dots)
+int64_t dict_spmv_blocks(int64_t nslices);
+// y = A x with the partial sums of (y, u) and (y, y) in part (2 x blocks); x in
+// FP32 or FP64; rows and columns numbered as order and dict say
+template <typename XT>
+int dict_spmv_dots(int64_t nrows, int64_t nslices, const int32_t* width, const int32_t* dptr, const int32_t* dict,
+                   const int64_t* vptr, const int64_t* iptr, const double* sval, const uint32_t* sidx,
+                   const int32_t* order, const XT* x, double* y, const double* u, double* part, hipStream_t s);
+// ---- BiCGStab on lattice vectors (bicgstab_kernels.hip) ----
+constexpr int kBicgMaxBlocks = 8192;   // partial sums per array of the updates
+template <typename T>
+int bicg_p(int64_t n, bool first, double beta, double omega, const double* r, double* p, const double* v, double* r0,
+           T* sd, T* sc, hipStream_t s);
+template <typename T>
+int bicg_s(int64_t n, double rho, const double* vr0, const double* r, const double* v, const T* q, double* s,
+           double* x, double* part, double* ss_out, T* sd, T* sc, hipStream_t st);
+template <typename T>
+int bicg_r(int64_t n, const double* st_tt, const double* s, const double* t, const T* q, const double* r0, double* r,
+           double* x, double* part, double* rr_r0r_out, hipStream_t st);
+// out[m] = sum of the np partials of array m
+int sum_arrays(int count, int np, const double* part, double* out, hipStream_t s);
+// out[i] = map[in[i]], negative entries -1
+int renumber(int64_t n, const int32_t* in, const int32_t* map, int32_t* out, hipStream_t s);
 // the slots of a lattice's rows in blocks of 64 points (4x4x4 or 8x8)
 int64_t lattice_block_slots(int dim, int W);
 int lattice_block_order(int dim, int W, const int32_t* dof_of_lat, int32_t* order, hipStream_t s);
