@@ -27,6 +27,10 @@
 #include <utility>
 #include <vector>
 
+namespace ugamd {
+struct SellEpilogue;
+}
+
 namespace ug {
 namespace gpu {
 
@@ -250,6 +254,10 @@ class GPUSparseMatrix {
     template <typename T>
     void dictionary_product(const DeviceBuffer<int32_t>& order, const DeviceBuffer<int32_t>& dict, const T* x,
                             double* y, const double* u, double* part, double* out) const;
+    // a step of the multigrid cycle over matrices: the product A w with the row
+    // operations of SellEpilogue (sliced-ELL layout only)
+    bool sliced_ell_ready() const { return sell_valid_ && !dict_valid_ && !building_; }
+    void cycle_product(const double* w, const ugamd::SellEpilogue& e) const;
     bool has_row_order() const { return rows_ > 0 && row_order_.size() == rows_; }
     int lanes() const { return lanes_; }
     void set_lanes(int g) {
@@ -284,6 +292,7 @@ class GPUSparseMatrix {
     DeviceBuffer<int32_t> sell_width_, sell_col_, row_order_;
     DeviceBuffer<int64_t> sell_ptr_;
     DeviceBuffer<double> sell_val_;
+    int32_t sell_max_width_ = 0;
     // dictionary layout
     bool build_dictionary();
     bool dict_enabled_ = true, dict_valid_ = false;
@@ -377,6 +386,7 @@ class Jacobi : public ILinearIterator {
     bool init(std::shared_ptr<MatrixOperator> J) override;
     bool apply(GPUVector& c, const GPUVector& d) override;
     void set_damp(double w) { omega_ = w; }
+    const double* inverse_diagonal() const { return dinv_.get(); }   // damped, after init
 
    private:
     double omega_;
@@ -747,6 +757,14 @@ class MatrixMultiGrid : public ILinearIterator {
     int lu_n_ = 0;
     DeviceBuffer<double> lu_linvT_, lu_uinvT_;
     DeviceBuffer<int32_t> lu_perm_;
+    // The cycle in fused steps (every matrix in the sliced-ELL layout): one
+    // product per smoothing step and transfer, with the Jacobi and correction
+    // updates that follow it in the same kernel; st2_: the second step buffer
+    // (neighbours read one while rows write the other).
+    bool fused_ready();
+    void lmgc_fused(int lev, int type, const double* defect, double* correction);
+    std::vector<GPUVector> st2_;
+    std::vector<char> fresh_;   // the level's first smoothing step came with the restriction
 };
 
 enum class Precision { F64 = 0, F32 = 1 };

@@ -423,7 +423,11 @@ void GPUSparseMatrix::build_spmv_layout() {
     std::vector<int32_t> w(nsl);
     sell_width_.download(w.data(), nsl);
     std::vector<int64_t> ptr(nsl + 1, 0);
-    for (int64_t t = 0; t < nsl; ++t) ptr[t + 1] = ptr[t] + (int64_t)64 * w[t];
+    sell_max_width_ = 0;
+    for (int64_t t = 0; t < nsl; ++t) {
+        ptr[t + 1] = ptr[t] + (int64_t)64 * w[t];
+        sell_max_width_ = std::max(sell_max_width_, w[t]);
+    }
     sell_ptr_.resize(nsl + 1);
     sell_ptr_.upload(ptr.data(), nsl + 1);
     sell_col_.resize(ptr[nsl]);
@@ -792,13 +796,19 @@ void GPUSparseMatrix::axpy(GPUVector& dest, double a1, const GPUVector& v1, doub
                              d_vptr_.get(), d_iptr_.get(), d_val_.get(), d_idx_.get(), slice_order_.get(), a1,
                              v1.data(), b1, w1.data(), dest.data(), 0, rowptr_.get(), context().stream));
     else if (sell_valid_)
-        UGX_LAUNCH((sell_spmv<double, double>(rows_, sell_ptr_.get(), sell_width_.get(), sell_col_.get(),
+        UGX_LAUNCH((sell_spmv<double, double>(rows_, sell_ptr_.get(), sell_width_.get(), sell_max_width_, sell_col_.get(),
                                               sell_val_.get(), a1, v1.data(), b1, w1.data(), dest.data(), 0,
                                               rowptr_.get(), has_row_order() ? row_order_.get() : nullptr,
                                               context().stream)));
     else
         UGX_LAUNCH((spmv_csr<double, double>(rows_, rowptr_.get(), col_.get(), val_.get(), a1, v1.data(), b1,
                                              w1.data(), dest.data(), 0, lanes_, context().stream)));
+}
+
+void GPUSparseMatrix::cycle_product(const double* w, const SellEpilogue& e) const {
+    if (!sliced_ell_ready()) throw UGError("GPUSparseMatrix::cycle_product: needs the sliced-ELL layout");
+    UGX_LAUNCH(sell_cycle(rows_, sell_ptr_.get(), sell_width_.get(), sell_max_width_, sell_col_.get(), sell_val_.get(),
+                          w, rowptr_.get(), has_row_order() ? row_order_.get() : nullptr, e, context().stream));
 }
 
 void GPUSparseMatrix::renumber_dictionary(const int32_t* map, DeviceBuffer<int32_t>& order,
@@ -835,7 +845,7 @@ void GPUSparseMatrix::apply_ignore_zero_rows(GPUVector& dest, double beta, const
                              d_vptr_.get(), d_iptr_.get(), d_val_.get(), d_idx_.get(), slice_order_.get(), 0.0,
                              dest.data(), beta, w.data(), dest.data(), 1, rowptr_.get(), context().stream));
     else if (sell_valid_)
-        UGX_LAUNCH((sell_spmv<double, double>(rows_, sell_ptr_.get(), sell_width_.get(), sell_col_.get(),
+        UGX_LAUNCH((sell_spmv<double, double>(rows_, sell_ptr_.get(), sell_width_.get(), sell_max_width_, sell_col_.get(),
                                               sell_val_.get(), 0.0, dest.data(), beta, w.data(), dest.data(), 1,
                                               rowptr_.get(), has_row_order() ? row_order_.get() : nullptr,
                                               context().stream)));
@@ -1079,7 +1089,14 @@ bool CG::apply_return_defect(GPUVector& x, GPUVector& b) {
             return apply_lattice(x, r, *gmg, 0, &r);
         }
     }
-    GPUVector q(r.size()), z(x.size()), p(x.size());
+    // rho, lambda, alpha and beta stay on the device (cg_update, cg_direction);
+    // the host reads |r|^2 and the breakdown flag once per step
+    auto& c = context();
+    const int64_t n = r.size();
+    GPUVector q(n), z(n), p(n);
+    ws_sc_.resize(8);
+    ws_sc_.zero();
+    double* sc = ws_sc_.get();
     if (precond_) {
         if (!precond_->apply(z, r)) return false;
     } else {
@@ -1088,28 +1105,24 @@ bool CG::apply_return_defect(GPUVector& x, GPUVector& b) {
     conv_->set_name(name());
     conv_->start(r);
     p = z;
-    double rho_old = z.dotprod(r), rho;
+    UGX_LAUNCH(dot<double>(n, z.data(), r.data(), c.red_partial, sc + 0, false, c.stream));
     while (!conv_->iteration_ended()) {
         op_->apply(q, p);
-        double lambda = q.dotprod(p);
-        if (lambda == 0.0) {
-            if (p.size()) return false;
-            lambda = 1.0;
-        }
-        const double alpha = rho_old / lambda;
-        VecScaleAdd(x, 1.0, x, alpha, p);
-        VecScaleAdd(r, 1.0, r, -alpha, q);
-        conv_->update(r);
+        UGX_LAUNCH(dot<double>(n, q.data(), p.data(), c.red_partial, sc + 1, false, c.stream));
+        UGX_LAUNCH(cg_update(n, sc, p.data(), q.data(), x.data(), r.data(), c.red_partial, c.stream));
+        UGX_HIP(hipMemcpyAsync(c.red_host, sc + 5, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+        sync();
+        if (c.red_host[1] != 0.0 && n) return false;   // lambda == 0 (x, r unchanged)
+        conv_->update_defect(std::sqrt(c.red_host[0]));
         if (conv_->iteration_ended()) break;
         if (precond_) {
             if (!precond_->apply(z, r)) return false;
         } else {
             z = r;
         }
-        rho = z.dotprod(r);
-        const double beta = rho / rho_old;
-        VecScaleAdd(p, beta, p, 1.0, z);
-        rho_old = rho;
+        UGX_LAUNCH(dot<double>(n, z.data(), r.data(), c.red_partial, sc + 4, false, c.stream));
+        UGX_LAUNCH(cg_beta(sc, c.stream));
+        UGX_LAUNCH(cg_direction(n, sc, p.data(), z.data(), c.stream));
     }
     return conv_->post();
 }
@@ -2834,12 +2847,113 @@ bool MatrixMultiGrid::apply(GPUVector& c, const GPUVector& d) {
     if (top_ < 0 || (int)sc_.size() != top_ + 1) throw UGError("MatrixMultiGrid: not initialised");
     if (d.size() != sd_[top_].size() || c.size() != sd_[top_].size()) throw UGError("GMG::apply: size mismatch");
     // mg_solver_impl.hpp:175-275
+    if (&c != &d && top_ > base_ && fused_ready()) {
+        // the top level works on the caller's vectors; with presmoothing its
+        // first step reads d and starts the correction
+        fresh_.assign(top_ + 1, 0);
+        if (nu1_ == 0) {
+            sd_[top_] = d;
+            c.set(0.0);
+        }
+        lmgc_fused(top_, cycle_, nu1_ == 0 ? sd_[top_].data() : d.data(), c.data());
+        return true;
+    }
     sd_[top_] = d;
     c.set(0.0);
     sc_[top_].set(0.0);
     lmgc(top_, cycle_);
     c += sc_[top_];
     return true;
+}
+
+bool MatrixMultiGrid::fused_ready() {
+    for (int l = base_; l <= top_; ++l) {
+        if (l > base_ && !(Aop(l).sliced_ell_ready() && P_[l]->sliced_ell_ready() && R_[l]->sliced_ell_ready()))
+            return false;
+    }
+    if ((int)st2_.size() != top_ + 1) {
+        st2_.assign(top_ + 1, GPUVector());
+        for (int l = base_ + 1; l <= top_; ++l) st2_[l].resize(st_[l].size());
+    }
+    return true;
+}
+
+// lmgc in fused steps: the defect is read from `defect` (the level's sd, or the
+// caller's vector on the top level) and kept in sd from the first update on
+void MatrixMultiGrid::lmgc_fused(int lev, int type, const double* defect, double* sc) {
+    auto& c = context();
+    double *sd = sd_[lev].data(), *st = st_[lev].data(), *st2 = st2_[lev].data();
+    const int64_t n = sd_[lev].size();
+    const GPUSparseMatrix& A = Aop(lev);
+    const double* dinv = smoother_[lev]->inverse_diagonal();
+    // presmoothing (mg_solver_impl.hpp:1686-1730): st = D sd, sd -= A st, sc += st
+    for (int nu = 0; nu < nu1_; ++nu) {
+        if (nu == 0) {
+            // the restriction has left st = D sd and sc = st (fresh_), a
+            // second visit of the level (W, F) continues its correction
+            if (!fresh_[lev]) {
+                UGX_LAUNCH((diag_mult<double, double>(n, st, dinv, defect, c.stream)));
+                if (lev == top_) UGX_LAUNCH((diag_mult<double, double>(n, sc, dinv, defect, c.stream)));
+                else UGX_LAUNCH(vec_scale_add<double>(n, sc, 1.0, sc, 1.0, st, 0.0, nullptr, c.stream));
+            }
+            fresh_[lev] = 0;
+        }
+        SellEpilogue e;
+        e.sub = nu == 0 ? defect : sd;
+        e.out = sd;
+        if (nu + 1 < nu1_) {
+            e.dinv = dinv;
+            e.st = st2;
+            e.sc = sc;
+        }
+        A.cycle_product(st, e);
+        std::swap(st, st2);
+    }
+    // restriction (StdTransfer::do_restrict) and the coarse level's first step
+    {
+        SellEpilogue e;
+        e.out = sd_[lev - 1].data();
+        e.keep_empty = 1;
+        if (lev - 1 > base_) {
+            if (nu1_ > 0) {
+                e.dinv = smoother_[lev - 1]->inverse_diagonal();
+                e.st = st_[lev - 1].data();
+                e.sc = sc_[lev - 1].data();
+                e.sc_set = 1;
+                fresh_[lev - 1] = 1;
+            } else {
+                sc_[lev - 1].set(0.0);
+            }
+        }
+        R_[lev]->cycle_product(sd, e);
+    }
+    if (lev - 1 == base_) {
+        base_solve(lev - 1);
+    } else if (type == _F_) {
+        lmgc_fused(lev - 1, _F_, sd_[lev - 1].data(), sc_[lev - 1].data());
+        lmgc_fused(lev - 1, _V_, sd_[lev - 1].data(), sc_[lev - 1].data());
+    } else {
+        for (int i = 0; i < type; ++i) lmgc_fused(lev - 1, type, sd_[lev - 1].data(), sc_[lev - 1].data());
+    }
+    // prolongation (StdTransfer::prolongate): st = P sc_{l-1}, sc += st
+    {
+        SellEpilogue e;
+        e.out = st;
+        e.sc = sc;
+        P_[lev]->cycle_product(sc_[lev - 1].data(), e);
+    }
+    // postsmoothing: sd -= A st, st = D sd, sc += st. The top level's defect
+    // after its last step is not formed: apply() returns the correction alone
+    for (int nu = 0; nu < nu2_; ++nu) {
+        SellEpilogue e;
+        e.sub = sd;
+        e.out = sd;
+        e.dinv = dinv;
+        e.st = st2;
+        e.sc = sc;
+        A.cycle_product(st, e);
+        std::swap(st, st2);
+    }
 }
 
 void MatrixMultiGrid::lmgc(int lev, int type) {

@@ -259,54 +259,135 @@ __global__ __launch_bounds__(64) void k_sell_fill(int64_t nrows, int64_t ncols, 
     }
 }
 
+// The row sums of a sliced-ELL matrix and what a product does with them.
+// Each of a slice's 64 rows belongs to one lane; WAVES wavefronts share a
+// slice, each summing every WAVES-th entry, combined through LDS in a fixed
+// order. WAVES 1 (four slices a workgroup) streams the matrices of many short
+// rows: 400,003 rows of about 16 entries, 57 us, bound by the gathers. Where rows
+// are wide and few (Q2 operators and transfers: up to 125 entries, 1 - 560
+// slices), one lane's chain of loads and gathers is the time: 20 - 30 us
+// whatever the size with one wave, 9.8 - 13.7 us with four (one MI355X, 729 -
+// 35,937 rows); with sixteen the chain is one round of eight entries and the
+// solve with these matrices takes 2.57 ms instead of 2.71. sell_waves() draws the
+// line.
+constexpr int sell_block(int waves) { return waves == 1 ? 256 : 64 * waves; }
+
+template <typename TM, typename TV, int WAVES>
+__device__ __forceinline__ bool sell_row_sum(int64_t nrows, const int64_t* __restrict__ slice_ptr,
+                                             const int32_t* __restrict__ width, const int32_t* __restrict__ scol,
+                                             const TM* __restrict__ sval, const TV* __restrict__ w,
+                                             const int32_t* __restrict__ order, int64_t nblocks, int64_t& r,
+                                             double& sum) {
+    const int64_t lb = xcd_block(nblocks);
+    if (lb >= nblocks) return false;   // the whole workgroup
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t t = WAVES == 1 ? lb * 4 + wave : lb;
+    const int64_t nslices = (nrows + 63) / 64;
+    if (WAVES == 1 && t >= nslices) return false;
+    const int64_t p = t * 64 + lane;
+    const int32_t wd = width[t];
+    const int32_t* cp = scol + slice_ptr[t] + lane;
+    const TM* vp = sval + slice_ptr[t] + lane;
+    double s0 = 0.0, s1 = 0.0;
+    if (WAVES == 1) {
+        int32_t k = 0;
+        for (; k + 4 <= wd; k += 4) {
+            int32_t c[4];
+            double a[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) c[u] = __builtin_nontemporal_load(cp + 64 * (k + u));
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[u] = (double)__builtin_nontemporal_load(vp + 64 * (k + u));
+#pragma unroll
+            for (int u = 0; u < 4; u += 2) {
+                s0 = fma(a[u], (double)w[c[u]], s0);
+                s1 = fma(a[u + 1], (double)w[c[u + 1]], s1);
+            }
+        }
+        for (; k < wd; ++k) {
+            const int32_t c0 = __builtin_nontemporal_load(cp + 64 * k);
+            const double a0 = (double)__builtin_nontemporal_load(vp + 64 * k);
+            s0 = fma(a0, (double)w[c0], s0);
+        }
+    } else {
+        // entries wave, wave + WAVES, ...: which sum an entry goes to depends on
+        // its place in the row alone, not on the width of the slice. The last
+        // round loads the slice's last entry for the ones it lacks.
+        for (int32_t k0 = wave; k0 < wd; k0 += 8 * WAVES) {
+            int32_t c[8];
+            double a[8], x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int32_t k = k0 + u * WAVES < wd ? k0 + u * WAVES : wd - 1;
+                c[u] = __builtin_nontemporal_load(cp + 64 * k);
+                a[u] = (double)__builtin_nontemporal_load(vp + 64 * k);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = (double)w[c[u]];
+#pragma unroll
+            for (int u = 0; u < 8; u += 2) {
+                const double t0 = fma(a[u], x[u], s0), t1 = fma(a[u + 1], x[u + 1], s1);
+                s0 = k0 + u * WAVES < wd ? t0 : s0;
+                s1 = k0 + (u + 1) * WAVES < wd ? t1 : s1;
+            }
+        }
+    }
+    sum = s0 + s1;
+    if (WAVES > 1) {
+        __shared__ double sh[WAVES][64];
+        sh[wave][lane] = sum;
+        __syncthreads();
+        if (wave != 0) return false;
+        sum = sh[0][lane];
+#pragma unroll
+        for (int u = 1; u < WAVES; ++u) sum += sh[u][lane];
+    }
+    if (p >= nrows) return false;
+    r = sell_row(order, p);
+    return true;
+}
+
 // dest = alpha*v1 + beta*A*w (mode 0) or dest = beta*A*w on rows with entries
 // (mode 1, needs rowptr)
-template <typename TM, typename TV>
-__global__ __launch_bounds__(256) void k_sell_spmv(int64_t nrows, const int64_t* __restrict__ slice_ptr,
+template <typename TM, typename TV, int WAVES>
+__global__ __launch_bounds__(sell_block(WAVES)) void k_sell_spmv(int64_t nrows, const int64_t* __restrict__ slice_ptr,
                                                    const int32_t* __restrict__ width, const int32_t* __restrict__ scol,
                                                    const TM* __restrict__ sval, double alpha, const TV* v1, double beta,
                                                    const TV* __restrict__ w, TV* dest, int mode,
                                                    const int32_t* __restrict__ rowptr,
                                                    const int32_t* __restrict__ order, int64_t nblocks) {
-    const int64_t lb = xcd_block(nblocks);
-    if (lb >= nblocks) return;
-    const int64_t p = lb * 256 + threadIdx.x;
-    const int64_t t = p >> 6;
-    if (t >= (nrows + 63) / 64) return;
-    const int lane = (int)(p & 63);
-    const int32_t wd = width[t];
-    const int32_t* cp = scol + slice_ptr[t] + lane;
-    const TM* vp = sval + slice_ptr[t] + lane;
-    double s0 = 0.0, s1 = 0.0;
-    int32_t k = 0;
-    for (; k + 4 <= wd; k += 4) {
-        const int32_t c0 = __builtin_nontemporal_load(cp + 64 * k);
-        const int32_t c1 = __builtin_nontemporal_load(cp + 64 * (k + 1));
-        const int32_t c2 = __builtin_nontemporal_load(cp + 64 * (k + 2));
-        const int32_t c3 = __builtin_nontemporal_load(cp + 64 * (k + 3));
-        const double a0 = (double)__builtin_nontemporal_load(vp + 64 * k);
-        const double a1 = (double)__builtin_nontemporal_load(vp + 64 * (k + 1));
-        const double a2 = (double)__builtin_nontemporal_load(vp + 64 * (k + 2));
-        const double a3 = (double)__builtin_nontemporal_load(vp + 64 * (k + 3));
-        s0 = fma(a0, (double)w[c0], s0);
-        s1 = fma(a1, (double)w[c1], s1);
-        s0 = fma(a2, (double)w[c2], s0);
-        s1 = fma(a3, (double)w[c3], s1);
-    }
-    for (; k < wd; ++k) {
-        const int32_t c0 = __builtin_nontemporal_load(cp + 64 * k);
-        const double a0 = (double)__builtin_nontemporal_load(vp + 64 * k);
-        s0 = fma(a0, (double)w[c0], s0);
-    }
-    if (p >= nrows) return;
-    const int64_t r = sell_row(order, p);
-    const double sum = s0 + s1;
+    int64_t r;
+    double sum;
+    if (!sell_row_sum<TM, TV, WAVES>(nrows, slice_ptr, width, scol, sval, w, order, nblocks, r, sum)) return;
     if (mode == 1) {
         if (rowptr[r + 1] > rowptr[r]) dest[r] = (TV)(beta * sum);
     } else {
         const double base = (alpha == 0.0) ? 0.0 : alpha * (double)v1[r];
         dest[r] = (TV)(base + beta * sum);
     }
+}
+
+// a product of the multigrid cycle over matrices with the row operations that
+// follow it (SellEpilogue)
+template <int WAVES>
+__global__ __launch_bounds__(sell_block(WAVES)) void k_sell_cycle(int64_t nrows, const int64_t* __restrict__ slice_ptr,
+                                                    const int32_t* __restrict__ width, const int32_t* __restrict__ scol,
+                                                    const double* __restrict__ sval, const double* __restrict__ w,
+                                                    const int32_t* __restrict__ rowptr,
+                                                    const int32_t* __restrict__ order, int64_t nblocks,
+                                                    SellEpilogue e) {
+    int64_t r;
+    double v;
+    if (!sell_row_sum<double, double, WAVES>(nrows, slice_ptr, width, scol, sval, w, order, nblocks, r, v)) return;
+    const double d = e.dinv ? e.dinv[r] : 0.0, c = e.sc && !e.sc_set ? e.sc[r] : 0.0;   // in flight together
+    if (e.sub) v = 1.0 * e.sub[r] + -1.0 * v;
+    else if (e.keep_empty && rowptr[r + 1] == rowptr[r]) v = e.out[r];
+    if (e.out) e.out[r] = v;
+    if (e.dinv) {
+        v = d * v;
+        e.st[r] = v;
+    }
+    if (e.sc) e.sc[r] = e.sc_set ? v : 1.0 * c + 1.0 * v;
 }
 
 // ---------------------------------------------------------------------------
@@ -3088,19 +3169,58 @@ int sell_fill(int64_t nrows, int64_t ncols, const int32_t* rowptr, const int32_t
 template int sell_fill<double>(int64_t, int64_t, const int32_t*, const int32_t*, const double*, const int32_t*,
                                const int64_t*, const int32_t*, int32_t*, double*, hipStream_t, bool);
 
+// Several waves a slice where the slices do not fill the chip by themselves
+// (fewer than 16 waves a CU), so that a wave has at most about eight entries:
+// one wave 23.5 us on 35,937 rows of up to 125 entries, four 13.7, sixteen less
+// again; 7.5 - 9.2 us with one wave on rows of up to 27 entries.
+static int sell_waves(int64_t nslices, int max_width) {
+    if (nslices >= (int64_t)device_cus() * 16 || max_width <= 8) return 1;
+    return max_width > 32 ? 16 : 4;
+}
+
+template <typename TM, typename TV, int WAVES>
+static void launch_sell_spmv(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, const int32_t* scol,
+                             const TM* sval, double alpha, const TV* v1, double beta, const TV* w, TV* dest, int mode,
+                             const int32_t* rowptr, const int32_t* order, hipStream_t s) {
+    const int64_t nsl = (nrows + 63) / 64, nb = WAVES == 1 ? (nsl + 3) / 4 : nsl;
+    hipLaunchKernelGGL((k_sell_spmv<TM, TV, WAVES>), dim3(remapped_grid(nb)), dim3(sell_block(WAVES)), 0, s, nrows,
+                       slice_ptr, width, scol, sval, alpha, v1, beta, w, dest, mode, rowptr, order, nb);
+}
+
 template <typename TM, typename TV>
-int sell_spmv(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, const int32_t* scol, const TM* sval,
-              double alpha, const TV* v1, double beta, const TV* w, TV* dest, int mode, const int32_t* rowptr,
-              const int32_t* order, hipStream_t s) {
+int sell_spmv(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, int max_width, const int32_t* scol,
+              const TM* sval, double alpha, const TV* v1, double beta, const TV* w, TV* dest, int mode,
+              const int32_t* rowptr, const int32_t* order, hipStream_t s) {
     if (nrows <= 0) return 0;
-    const int64_t nb = (((nrows + 63) / 64) * 64 + 255) / 256;
-    hipLaunchKernelGGL((k_sell_spmv<TM, TV>), dim3(remapped_grid(nb)), dim3(256), 0, s, nrows, slice_ptr, width,
-                       scol, sval, alpha, v1, beta, w, dest, mode, rowptr, order, nb);
+    const int waves = sell_waves((nrows + 63) / 64, max_width);
+    auto* f = waves == 16  ? &launch_sell_spmv<TM, TV, 16>
+              : waves == 4 ? &launch_sell_spmv<TM, TV, 4>
+                           : &launch_sell_spmv<TM, TV, 1>;
+    f(nrows, slice_ptr, width, scol, sval, alpha, v1, beta, w, dest, mode, rowptr, order, s);
     UGX_CHECK_LAUNCH();
 }
-template int sell_spmv<double, double>(int64_t, const int64_t*, const int32_t*, const int32_t*, const double*, double,
-                                       const double*, double, const double*, double*, int, const int32_t*,
+template int sell_spmv<double, double>(int64_t, const int64_t*, const int32_t*, int, const int32_t*, const double*,
+                                       double, const double*, double, const double*, double*, int, const int32_t*,
                                        const int32_t*, hipStream_t);
+
+template <int WAVES>
+static void launch_sell_cycle(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, const int32_t* scol,
+                              const double* sval, const double* w, const int32_t* rowptr, const int32_t* order,
+                              const SellEpilogue& e, hipStream_t s) {
+    const int64_t nsl = (nrows + 63) / 64, nb = WAVES == 1 ? (nsl + 3) / 4 : nsl;
+    hipLaunchKernelGGL(k_sell_cycle<WAVES>, dim3(remapped_grid(nb)), dim3(sell_block(WAVES)), 0, s, nrows, slice_ptr,
+                       width, scol, sval, w, rowptr, order, nb, e);
+}
+
+int sell_cycle(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, int max_width, const int32_t* scol,
+               const double* sval, const double* w, const int32_t* rowptr, const int32_t* order,
+               const SellEpilogue& e, hipStream_t s) {
+    if (nrows <= 0) return 0;
+    const int waves = sell_waves((nrows + 63) / 64, max_width);
+    auto* f = waves == 16 ? &launch_sell_cycle<16> : waves == 4 ? &launch_sell_cycle<4> : &launch_sell_cycle<1>;
+    f(nrows, slice_ptr, width, scol, sval, w, rowptr, order, e, s);
+    UGX_CHECK_LAUNCH();
+}
 
 int adjoint_grad_q1_hex(int n, double h, const double* theta, const int32_t* dof_of_lat, int64_t n_inner,
                         const double* u, const double* lambda, double* grad, hipStream_t s) {

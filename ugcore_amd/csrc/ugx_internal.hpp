@@ -18,10 +18,27 @@ template <typename TM>
 int sell_fill(int64_t nrows, int64_t ncols, const int32_t* rowptr, const int32_t* col, const TM* val,
               const int32_t* order, const int64_t* slice_ptr, const int32_t* width, int32_t* scol, TM* sval,
               hipStream_t s, bool vals_only = false);
+// max_width: the widest slice
 template <typename TM, typename TV>
-int sell_spmv(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, const int32_t* scol, const TM* sval,
-              double alpha, const TV* v1, double beta, const TV* w, TV* dest, int mode, const int32_t* rowptr,
-              const int32_t* order, hipStream_t s);
+int sell_spmv(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, int max_width, const int32_t* scol,
+              const TM* sval, double alpha, const TV* v1, double beta, const TV* w, TV* dest, int mode,
+              const int32_t* rowptr, const int32_t* order, hipStream_t s);
+// what a step of the multigrid cycle over matrices does with a product A w:
+//   v = sub - A w (where sub is given), A w, or out on rows without entries
+//   (keep_empty)
+//   out = v (where given);  with dinv: v = dinv .* v, st = v
+//   sc = v (sc_set) or sc += v (where given)
+struct SellEpilogue {
+    const double* sub = nullptr;
+    double* out = nullptr;
+    const double* dinv = nullptr;
+    double* st = nullptr;
+    double* sc = nullptr;
+    int keep_empty = 0, sc_set = 0;
+};
+int sell_cycle(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, int max_width, const int32_t* scol,
+               const double* sval, const double* w, const int32_t* rowptr, const int32_t* order,
+               const SellEpilogue& e, hipStream_t s);
 
 template <typename T>
 int vec_set(int64_t n, T* x, double v, hipStream_t s);
