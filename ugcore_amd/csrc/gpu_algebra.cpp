@@ -2346,7 +2346,7 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         first_defect_f32 = nullptr;
         for (auto& l : L) l.acc_deferred = false;
     }
-    bool first_step_fused() const { return mf && nu1 > 0 && top > base && q1mf_first_fits(L[top].W, sizeof(T)); }
+    bool first_step_fused() const { return mf && nu1 > 0 && top > base && q1mf_fused_fits(L[top].W); }
 
     void base_solve(int lev) {
         auto& c = context();
@@ -2407,7 +2407,7 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         // step, the deferred correction update, its conversion and (z, r) in
         // one pass (run_lattice then has nothing left to do)
         const bool fuse_last = fuse_smoothing && defer_top_final && lev == top && sym && mf && nu2 >= 2 &&
-                               q1mf_last_fits(f.W, sizeof(T));
+                               q1mf_fused_fits(f.W);
         for (int nu = 0; nu < nu2; ++nu) {
             if (fuse_last && nu == nu2 - 2) {
                 if (last_out) {

@@ -1136,8 +1136,9 @@ __global__ __launch_bounds__(256) void k_dias27_staged_jacobi_step(int64_t n, Di
 }
 
 // ---------------------------------------------------------------------------
-// Matrix-free Q1 operator of a uniformly refined cube with a coefficient that
-// is constant per element (the top level of the hexahedral hierarchy):
+// The matrix-free Q1 operator (q1mf_kernels.hip) plane by plane, for the
+// widths that file has no schedule for (513): the operator of a uniformly
+// refined cube with a coefficient that is constant per element,
 // A = sum_e c_e K_ref with c_e = h k_e and the unit-cube Q1 stiffness K_ref
 // (diagonal 1/3, face diagonals -1/12, body diagonal -1/12, couplings along
 // element edges 0), so for an interior row
@@ -1254,66 +1255,6 @@ __device__ __forceinline__ void q1mf_block(const MfMap& m, const T* __restrict__
     }
 }
 
-// z-marching variant: a block owns TY lines of a chunk of ZC planes and walks
-// it plane by plane. The staged values of the planes k-1, k, k+1 live in an
-// LDS ring of mf_slots() planes, the block's cells in a second ring of one
-// plane fewer; the loads of plane k+2 are issued into registers before plane
-// k is computed and stored after it (into the slot of plane k-1, behind a
-// second barrier with the 3-plane ring), so every plane is read once per
-// block and its load latency overlaps the arithmetic.
-struct MfZMap {
-    int32_t W, TY, nchunks;
-    int32_t glo[8], gsz[8];
-};
-// tile shape of the z-marching kernels: lines per block and planes per block
-// (FP32 / FP64), staged entries and rows per thread and plane. Measured on one
-// MI355X at 257^3: the small per-thread arrays keep the register count low
-// enough for more resident waves, which matters more than the y halo of the
-// narrow bands (2 lines: FP32 Jacobi step 0.159 -> 0.140 ms, FP64 operator
-// 0.235 -> 0.191 ms against 4-line bands with 7 staged entries and 5 rows).
-// The number of plane chunks per band is chosen at launch so that the whole
-// grid is resident at once (make_mf_zmap asks the runtime how many blocks of
-// the kernel fit on a CU): at 257^3 with 16-plane chunks the FP32 grid needed
-// about 1.5 rounds, and one round measured 0.134 -> 0.118 ms.
-#ifndef UGX_MF_TY32
-#define UGX_MF_TY32 2
-#endif
-#ifndef UGX_MF_TY64
-#define UGX_MF_TY64 2
-#endif
-#ifndef UGX_MF_PF
-#define UGX_MF_PF 5
-#endif
-constexpr int kMfPrefetch = UGX_MF_PF;   // staged entries per thread and plane (P <= kMfPrefetch * 256)
-
-#ifndef UGX_MF_WAVES32
-#define UGX_MF_WAVES32 7
-#endif
-// planes in the staged LDS ring (FP32 / FP64): 4 = three in use and one being
-// filled; 3 = the filled plane overwrites the oldest one after a second
-// barrier per plane, which leaves room for more workgroups per CU. The cell
-// ring holds one plane fewer. Measured at 257^3 with one-round grids: 3 slots
-// let 7 FP32 workgroups (18.6 KB each, <= 72 VGPRs) and 4 FP64 workgroups
-// share a CU instead of 6 and 3: Jacobi step 0.114 -> 0.107 ms, FP64 operator
-// 0.185 -> 0.167 ms (8 FP32 workgroups need <= 64 VGPRs and spill: 0.124 ms).
-#ifndef UGX_MF_SLOTS32
-#define UGX_MF_SLOTS32 3
-#endif
-#ifndef UGX_MF_SLOTS64
-#define UGX_MF_SLOTS64 3
-#endif
-__host__ __device__ constexpr int mf_slots(size_t elem) { return elem == 4 ? UGX_MF_SLOTS32 : UGX_MF_SLOTS64; }
-// at most this many z-marching workgroups per CU are planned for: the FP32
-// d -= A x kernel fits 8 (61 VGPRs) but measured 114.7 us with 8 and 91.9 us
-// with 7 at 257^3; the other kernels fit 7 (FP32) or 4 (FP64) anyway
-#ifndef UGX_MF_MAXRES
-#define UGX_MF_MAXRES 7
-#endif
-#ifndef UGX_MF_ROWS
-#define UGX_MF_ROWS 3
-#endif
-constexpr int kMfRows = UGX_MF_ROWS;   // rows per thread and plane (R + 63 <= kMfRows * 256)
-
 // the coarse correction the prolongation reads: sc, or (with dinv) the value
 // the coarse level's deferred last post-smoothing update sc + dinv .* sd would
 // store, with the arithmetic of k_jacobi_accumulate
@@ -1321,267 +1262,6 @@ template <typename TV>
 __device__ __forceinline__ TV coarse_fold(TV sc, TV dinv, TV sd) {
     return (TV)((double)sc + (double)dinv * (double)sd);
 }
-// the Q1 operator at an interior lattice row from staged planes: sm, s0, sp
-// hold the operand on planes k-1, k, k+1 (the row at offset cc0, its
-// neighbours at cc0 +- 1, +- W), cm and c0 the per-element coefficients
-// h k_e of the cell planes below and above it (the row's lower-left cell at
-// offset cl0, lines CX apart). (A x)_i = (1/3) x_i sum_e c_e - (1/12) sum of
-// the 20 diagonal neighbours, each weighted by the coefficients of the cells
-// it shares with the row (one for a body diagonal, two for a face diagonal);
-// the 6 axis neighbours have weight 0 in the Q1 stiffness of a cube.
-template <typename T>
-__device__ __forceinline__ T q1mf_row(const T* sm, const T* s0, const T* sp, const T* cm, const T* c0, int cc0,
-                                      int cl0, int W, int CX, T xi) {
-    auto X = [&](int dx, int dy, int dz) {
-        const T* pl = dz < 0 ? sm : (dz > 0 ? sp : s0);
-        return pl[cc0 + dy * W + dx];
-    };
-    T ce[2][2][2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-            for (int aa = 0; aa < 2; ++aa) ce[c][bb][aa] = (c ? c0 : cm)[cl0 + bb * CX + aa];
-    T csum = (T)0, off = (T)0;
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-            for (int aa = 0; aa < 2; ++aa) {
-                csum += ce[c][bb][aa];
-                off = fma(ce[c][bb][aa], X(2 * aa - 1, 2 * bb - 1, 2 * c - 1), off);
-            }
-#pragma unroll
-    for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-        for (int aa = 0; aa < 2; ++aa) off = fma(ce[0][bb][aa] + ce[1][bb][aa], X(2 * aa - 1, 2 * bb - 1, 0), off);
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int aa = 0; aa < 2; ++aa) off = fma(ce[c][0][aa] + ce[c][1][aa], X(2 * aa - 1, 0, 2 * c - 1), off);
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb) off = fma(ce[c][bb][0] + ce[c][bb][1], X(0, 2 * bb - 1, 2 * c - 1), off);
-    return csum * xi * (T)(1.0 / 3.0) - off * (T)(1.0 / 12.0);
-}
-
-// The rows' own inputs and outputs (read and written once per launch) use
-// nontemporal loads and stores, which leave the L2 to the staged planes that
-// neighbouring bands share (measured at 257^3: FP32-preconditioned solve
-// 10.34 against 10.40 ms, FP64 15.00 against 15.08 ms).
-// MODE 0: fused Jacobi step (staged st = dinv.*sd; sd_out = sd - A st; sc += st)
-// MODE 1: d_out = d_in - A x;  MODE 2: y = alpha v + beta A x
-// MODE 3: the first Jacobi step of a cycle from the FP64 defect d64 and a zero
-//         correction: sd = (T)d64, st = dinv.*sd; sd_out = sd - A st; sc = st
-//         (the conversion rounds as k_convert does, so this equals k_convert,
-//         zeroing sc and MODE 0)
-// MODE 4: the same from a defect already in T (b_in = sd): MODE 0 without
-//         reading sc
-// MODE 5: the CG direction update fused with the operator: staged
-//         p_new = fma(beta, p_old, z) (a_in = p_old, b_in = z, beta = *d64,
-//         the arithmetic of k_cg_direction), out1 = p_new for the block's rows,
-//         y = A p_new and the (y, p_new) partials as MODE 2 with alpha 0
-// MODE 7: the last post-smoothing step of a cycle fused with the correction
-//         update that ends it, its conversion and the (z, r) partials: MODE 0
-//         (a_in = dinv, b_in = sd_in, c_in = sc) without storing sd_out or
-//         sc, then z = (double)(sc_new + dinv .* sd_out) with the arithmetic
-//         of k_jacobi_convert_dot (z64 = z, d64 = r)
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? UGX_MF_WAVES32 : 1)))
-void k_q1mf_z(MfZMap m, const T* __restrict__ cell, const T* __restrict__ a_in,
-                                                const T* __restrict__ b_in, const T* c_in, T* out0, T* out1,
-                                                double alpha, double beta, double* dot_partial,
-                                                const double* __restrict__ d64, double* __restrict__ z64) {
-    // c_in and out0 may alias (d_out = d_in); every row is read and then
-    // written by the same thread. MODE 2 with dot_partial: per-block partial
-    // sums of y_i * x_i (fixed order) in dot_partial[blockIdx.x]
-    double dot_acc = 0.0;
-    __shared__ double dot_sh[4];
-    auto finish_dot = [&]() {
-        if ((MODE != 2 && MODE != 5 && MODE != 7) || !dot_partial) return;
-        double v = dot_acc;
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-        if ((threadIdx.x & 63) == 0) dot_sh[threadIdx.x >> 6] = v;
-        __syncthreads();
-        if (threadIdx.x == 0) dot_partial[blockIdx.x] = (dot_sh[0] + dot_sh[1]) + (dot_sh[2] + dot_sh[3]);
-    };
-    // MODE 0: a_in = dinv, b_in = sd_in, out0 = sd_out, out1 = sc
-    // MODE 1: a_in = x, c_in = d_in, out0 = d_out
-    // MODE 2: a_in = x, c_in = v, out0 = y
-    const int xc = blockIdx.x & 7, q = blockIdx.x >> 3, g = m.gsz[xc];
-    const int chunk = g == 0 ? 0 : q / g;
-    if (g == 0 || chunk >= m.nchunks) {
-        finish_dot();   // idle block: partial 0
-        return;
-    }
-    const int band = m.glo[xc] + (q - chunk * g);
-    const int W = m.W, n = W - 1, TY = m.TY;
-    const int j0 = band * TY, j1 = j0 + TY < W ? j0 + TY : W, R = (j1 - j0) * W;
-    // the W planes split evenly over the chunks (about ZC each)
-    const int k0 = (int)((int64_t)chunk * W / m.nchunks), k1 = (int)((int64_t)(chunk + 1) * W / m.nchunks);
-    const int P = R + 2 * W + 2;
-    const int CX = n + 2, CL = (TY + 1) * CX;
-    const int64_t W2 = (int64_t)W * W;
-    T* ring = lds_base<T>();
-    constexpr int SL = mf_slots(sizeof(T)), CS = SL - 1;
-    T* cring = ring + SL * P;
-    const int tid = threadIdx.x, step = blockDim.x;
-    auto plane_first = [&](int p) { return (int64_t)p * W2 + (int64_t)(j0 - 1) * W - 1; };
-    auto cell_value = [&](int cz, int t) -> T {
-        const int line = t / CX, cx = t - line * CX;
-        const int cy = j0 - 1 + line;
-        if (cz < 0 || cz >= n || cy < 0 || cy >= n || cx < 1 || cx > n) return (T)0;
-        return cell[((int64_t)cz * n + cy) * n + cx - 1];
-    };
-    const T bcg = MODE == 5 ? (T)*d64 : (T)0;   // the CG's beta (MODE 5)
-    auto staged = [&](int64_t j) -> T {
-        return (MODE == 0 || MODE == 4 || MODE == 7) ? a_in[j] * b_in[j]
-               : MODE == 3             ? a_in[j] * (T)d64[j]
-               : MODE == 5             ? (T)fma((double)bcg, (double)a_in[j], (double)b_in[j])
-                                       : a_in[j];
-    };
-    // the cell each prefetch slot stages sits at the same place of every cell
-    // plane: its offset inside the plane, or -1 outside the lattice / the tile
-    int coff[kMfPrefetch];
-#pragma unroll
-    for (int u = 0; u < kMfPrefetch; ++u) {
-        const int t = tid + u * step;
-        coff[u] = -1;
-        if (t < CL) {
-            const int line = t / CX, cx = t - line * CX, cy = j0 - 1 + line;
-            if (cy >= 0 && cy < n && cx >= 1 && cx <= n) coff[u] = cy * n + cx - 1;
-        }
-    }
-    for (int p = k0 - 1; p <= k0 + 1; ++p) {
-        T* dst = ring + ((p + SL) % SL) * P;
-        const int64_t f0 = plane_first(p);
-        for (int t = tid; t < P; t += step) dst[t] = staged(f0 + t);
-    }
-    for (int cz = k0 - 1; cz <= k0; ++cz) {
-        T* dst = cring + ((cz + CS) % CS) * CL;
-        for (int t = tid; t < CL; t += step) dst[t] = cell_value(cz, t);
-    }
-    __syncthreads();
-    for (int k = k0; k < k1; ++k) {
-        const int64_t base = (int64_t)k * W2 + (int64_t)j0 * W;
-        const int a0 = (int)(base & 63);
-        // 1. issue every global load of this step: plane k+2 (raw), cell plane
-        //    k+1, and the row inputs of plane k
-        T pa[kMfPrefetch], pb[kMfPrefetch], cv[kMfPrefetch];
-        const int64_t f2 = plane_first(k + 2);
-        const bool more = (k + 1 < k1);
-#pragma unroll
-        for (int u = 0; u < kMfPrefetch; ++u) {
-            const int t = tid + u * step;
-            const bool ok = more && t < P;
-            pa[u] = ok ? a_in[f2 + t] : (T)0;
-            if (MODE == 0 || MODE == 4 || MODE == 5 || MODE == 7) pb[u] = ok ? b_in[f2 + t] : (T)0;
-            if (MODE == 3) pb[u] = ok ? (T)d64[f2 + t] : (T)0;
-            cv[u] = (more && coff[u] >= 0 && k + 1 < n) ? cell[(int64_t)(k + 1) * n * n + coff[u]] : (T)0;
-        }
-        T ra[kMfRows], rb[kMfRows];
-        // MODE 7: dinv and r of the rows; FP64 reads them with the other row
-        // inputs, FP32 at the output (its registers are kept for the plane
-        // loop: 7 resident waves instead of 5, measured 148 against 179 us
-        // per step at 257^3; FP64 the other way round, 222 against 253 us)
-        constexpr bool EAGER7 = MODE == 7 && sizeof(T) == 8;
-        T rd[EAGER7 ? kMfRows : 1];
-        double rr[EAGER7 ? kMfRows : 1];
-#pragma unroll
-        for (int u = 0; u < kMfRows; ++u) {
-            const int r = tid + u * step - a0;
-            const bool ok = r >= 0 && r < R;
-            if (MODE == 0) {
-                ra[u] = ok ? ldnt(b_in + base + r) : (T)0;   // sd_in
-                rb[u] = ok ? ldnt(out1 + base + r) : (T)0;   // sc
-            } else if (MODE == 3) {
-                ra[u] = ok ? (T)ldnt(d64 + base + r) : (T)0;   // sd_in
-            } else if (MODE == 4) {
-                ra[u] = ok ? ldnt(b_in + base + r) : (T)0;     // sd_in
-            } else if (MODE == 7) {
-                ra[u] = ok ? ldnt(b_in + base + r) : (T)0;   // sd_in
-                rb[u] = ok ? ldnt(c_in + base + r) : (T)0;   // sc
-                if constexpr (EAGER7) {
-                    rd[u] = ok ? a_in[base + r] : (T)0;                     // dinv
-                    rr[u] = (ok && dot_partial) ? d64[base + r] : 0.0;      // r
-                }
-            } else if (MODE == 1) {
-                ra[u] = ok ? ldnt(c_in + base + r) : (T)0;   // d_in
-            } else {
-                ra[u] = (ok && alpha != 0.0) ? ldnt(c_in + base + r) : (T)0;   // v
-            }
-        }
-        // 2. the operator on this thread's rows of plane k
-        const T* sm = ring + ((k - 1 + SL) % SL) * P;
-        const T* s0 = ring + (k % SL) * P;
-        const T* sp = ring + ((k + 1) % SL) * P;
-        const T* cm = cring + ((k - 1 + CS) % CS) * CL;
-        const T* c0 = cring + (k % CS) * CL;
-        const bool plane_bnd = (k == 0 || k == W - 1);
-#pragma unroll
-        for (int u = 0; u < kMfRows; ++u) {
-            const int r = tid + u * step - a0;
-            if (r < 0 || r >= R) continue;
-            // line jl < TY of the band and column x of row r
-            int jl = 0, x = r;
-            while (x >= W) {
-                x -= W;
-                ++jl;
-            }
-            const int y = j0 + jl;
-            const int cc0 = r + W + 1;
-            const T xi = s0[cc0];
-            const T sv = (plane_bnd || x == 0 || x == W - 1 || y == 0 || y == W - 1)
-                             ? xi
-                             : q1mf_row(sm, s0, sp, cm, c0, cc0, jl * CX + x, W, CX, xi);
-            // 3. outputs
-            const int64_t i = base + r;
-            if (MODE == 0) {
-                stnt(ra[u] - sv, out0 + i);
-                stnt(rb[u] + xi, out1 + i);
-            } else if (MODE == 3 || MODE == 4) {
-                stnt(ra[u] - sv, out0 + i);
-                stnt(xi, out1 + i);
-            } else if (MODE == 1) {
-                stnt(ra[u] - sv, out0 + i);
-            } else if (MODE == 7) {
-                const T sd_out = ra[u] - sv, sc_new = rb[u] + xi;
-                const T dv = EAGER7 ? rd[EAGER7 ? u : 0] : a_in[i];
-                const double zi = (double)(T)((double)sc_new + (double)dv * (double)sd_out);
-                stnt(zi, z64 + i);
-                if (dot_partial) dot_acc += zi * (EAGER7 ? rr[EAGER7 ? u : 0] : d64[i]);
-            } else {
-                const T yv = (T)((alpha == 0.0 ? 0.0 : alpha * (double)ra[u]) + beta * (double)sv);
-                stnt(yv, out0 + i);
-                if (MODE == 5) stnt(xi, out1 + i);   // p_new
-                dot_acc += (double)yv * (double)xi;
-            }
-        }
-        // 4. the prefetched plane k+2 and cell plane k+1 into the rings (with
-        //    the short ring they replace planes k-1 and cell plane k-1, which
-        //    every thread must have finished reading)
-        if (SL == 3) __syncthreads();
-        if (more) {
-            T* dst = ring + ((k + 2) % SL) * P;
-            T* cdst = cring + ((k + 1) % CS) * CL;
-#pragma unroll
-            for (int u = 0; u < kMfPrefetch; ++u) {
-                const int t = tid + u * step;
-                if (t < P)
-                    dst[t] = (MODE == 0 || MODE == 3 || MODE == 4 || MODE == 7) ? pa[u] * pb[u]
-                             : MODE == 5 ? (T)fma((double)bcg, (double)pa[u], (double)pb[u])
-                                         : pa[u];
-                if (t < CL) cdst[t] = cv[u];
-            }
-        }
-        __syncthreads();
-    }
-    finish_dot();
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void k_q1mf_jacobi_step(MfMap m, const T* __restrict__ cell,
                                                           const T* __restrict__ dinv, const T* __restrict__ sd_in,
@@ -2593,7 +2273,7 @@ static int64_t make_staged_map(int64_t n, int nd, const int32_t* off, size_t ele
 
 // workgroups of `kernel` (256 threads, `lds` bytes of LDS) resident on one CU,
 // and the device's CU count; both asked once and kept
-static int mf_resident_blocks(const void* kernel, size_t lds) {
+int resident_blocks(const void* kernel, size_t lds) {
     static std::mutex mu;
     static std::vector<std::pair<std::pair<const void*, size_t>, int>> cache;
     std::lock_guard<std::mutex> lock(mu);
@@ -2604,7 +2284,7 @@ static int mf_resident_blocks(const void* kernel, size_t lds) {
     cache.push_back({{kernel, lds}, nb});
     return nb;
 }
-static int device_cus() {
+int device_cus() {
     static int cus = 0;
     if (cus == 0) {
         int dev = 0, n = 0;
@@ -2613,35 +2293,6 @@ static int device_cus() {
         cus = n;
     }
     return cus;
-}
-
-// z-marching plan: bands of TY lines grouped per XCD (blockIdx % 8), and as
-// many plane chunks per band as make the grid resident at once (each XCD's
-// group of bands times the chunks fills at most its CUs' workgroup slots;
-// chunks of at least 4 planes); returns the grid (0 when the prefetch
-// registers cannot hold a plane)
-static int64_t make_mf_zmap(int W, size_t elem, const void* kernel, MfZMap& m, size_t& lds) {
-    m = MfZMap{};
-    m.W = W;
-    m.TY = elem == 8 ? UGX_MF_TY64 : UGX_MF_TY32;
-    const int64_t P = (int64_t)m.TY * W + 2 * W + 2, CL = (int64_t)(m.TY + 1) * (W + 1);
-    if (P > (int64_t)kMfPrefetch * 256 || CL > (int64_t)kMfPrefetch * 256 || W < 8) return 0;
-    if ((int64_t)m.TY * W + 63 > (int64_t)kMfRows * 256) return 0;
-    const int64_t nb = (W + m.TY - 1) / m.TY;
-    int32_t maxg = 0;
-    for (int c = 0; c < 8; ++c) {
-        const int64_t b0 = c * nb / 8, b1 = (c + 1) * nb / 8;
-        m.glo[c] = (int32_t)b0;
-        m.gsz[c] = (int32_t)(b1 - b0);
-        maxg = m.gsz[c] > maxg ? m.gsz[c] : maxg;
-    }
-    lds = (size_t)(mf_slots(elem) * P + (mf_slots(elem) - 1) * CL) * elem;
-    if (lds > 64 * 1024) return 0;
-    const int64_t slots = (int64_t)(device_cus() / 8) * std::min(UGX_MF_MAXRES, mf_resident_blocks(kernel, lds));
-    int64_t nch = maxg > 0 ? slots / maxg : 1;
-    nch = std::min<int64_t>(std::max<int64_t>(nch, 1), std::max(1, W / 4));
-    m.nchunks = (int32_t)nch;
-    return 8 * (int64_t)maxg * m.nchunks;
 }
 
 // matrix-free launch plan: bands of 4 lines grouped per XCD (any W >= 3)
@@ -2748,14 +2399,7 @@ template int dias_jacobi_step<double, double>(int64_t, int, const int32_t*, cons
 template int dias_jacobi_step<float, float>(int64_t, int, const int32_t*, const float*, const float*, const float*, float*, float*, hipStream_t);
 
 template <typename T>
-int q1mf_jacobi_step(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s) {
-    MfZMap zm;
-    size_t zlds;
-    if (const int64_t zgrid = make_mf_zmap(W, sizeof(T), reinterpret_cast<const void*>(&k_q1mf_z<T, 0>), zm, zlds)) {
-        hipLaunchKernelGGL((k_q1mf_z<T, 0>), dim3(zgrid), dim3(256), zlds, s, zm, cell, dinv, sd_in, (const T*)nullptr,
-                           sd_out, sc, 0.0, 0.0, (double*)nullptr, (const double*)nullptr, (double*)nullptr);
-        UGX_CHECK_LAUNCH();
-    }
+int q1mf_planes_jacobi_step(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s) {
     MfMap m;
     size_t lds;
     const int64_t grid = make_mf_map(W, sizeof(T), m, lds);
@@ -2763,50 +2407,12 @@ int q1mf_jacobi_step(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_
     hipLaunchKernelGGL(k_q1mf_jacobi_step<T>, dim3(grid), dim3(256), lds, s, m, cell, dinv, sd_in, sd_out, sc);
     UGX_CHECK_LAUNCH();
 }
-template int q1mf_jacobi_step<float>(int, const float*, const float*, const float*, float*, float*, hipStream_t);
-template int q1mf_jacobi_step<double>(int, const double*, const double*, const double*, double*, double*, hipStream_t);
+template int q1mf_planes_jacobi_step<float>(int, const float*, const float*, const float*, float*, float*, hipStream_t);
+template int q1mf_planes_jacobi_step<double>(int, const double*, const double*, const double*, double*, double*,
+                                             hipStream_t);
 
 template <typename T>
-int q1mf_jacobi_first(int W, const T* cell, const T* dinv, const double* d64, T* sd_out, T* sc, hipStream_t s) {
-    MfZMap zm;
-    size_t zlds;
-    const int64_t zgrid = make_mf_zmap(W, sizeof(T), reinterpret_cast<const void*>(&k_q1mf_z<T, 3>), zm, zlds);
-    if (!zgrid) return -1;
-    hipLaunchKernelGGL((k_q1mf_z<T, 3>), dim3(zgrid), dim3(256), zlds, s, zm, cell, dinv, (const T*)nullptr,
-                       (const T*)nullptr, sd_out, sc, 0.0, 0.0, (double*)nullptr, d64, (double*)nullptr);
-    UGX_CHECK_LAUNCH();
-}
-bool q1mf_first_fits(int W, size_t elem) {
-    MfZMap zm;
-    size_t lds;
-    const void* k = elem == 4 ? reinterpret_cast<const void*>(&k_q1mf_z<float, 3>)
-                              : reinterpret_cast<const void*>(&k_q1mf_z<double, 3>);
-    return make_mf_zmap(W, elem, k, zm, lds) != 0;
-}
-template <typename T>
-int q1mf_jacobi_first_t(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s) {
-    MfZMap zm;
-    size_t zlds;
-    const int64_t zgrid = make_mf_zmap(W, sizeof(T), reinterpret_cast<const void*>(&k_q1mf_z<T, 4>), zm, zlds);
-    if (!zgrid) return -1;
-    hipLaunchKernelGGL((k_q1mf_z<T, 4>), dim3(zgrid), dim3(256), zlds, s, zm, cell, dinv, sd_in, (const T*)nullptr,
-                       sd_out, sc, 0.0, 0.0, (double*)nullptr, (const double*)nullptr, (double*)nullptr);
-    UGX_CHECK_LAUNCH();
-}
-template int q1mf_jacobi_first_t<float>(int, const float*, const float*, const float*, float*, float*, hipStream_t);
-template int q1mf_jacobi_first<float>(int, const float*, const float*, const double*, float*, float*, hipStream_t);
-template int q1mf_jacobi_first<double>(int, const double*, const double*, const double*, double*, double*,
-                                       hipStream_t);
-
-template <typename T>
-int q1mf_apply_sub(int W, const T* cell, const T* x, const T* d_in, T* d_out, hipStream_t s) {
-    MfZMap zm;
-    size_t zlds;
-    if (const int64_t zgrid = make_mf_zmap(W, sizeof(T), reinterpret_cast<const void*>(&k_q1mf_z<T, 1>), zm, zlds)) {
-        hipLaunchKernelGGL((k_q1mf_z<T, 1>), dim3(zgrid), dim3(256), zlds, s, zm, cell, x, (const T*)nullptr, d_in,
-                           d_out, (T*)nullptr, 0.0, 0.0, (double*)nullptr, (const double*)nullptr, (double*)nullptr);
-        UGX_CHECK_LAUNCH();
-    }
+int q1mf_planes_apply_sub(int W, const T* cell, const T* x, const T* d_in, T* d_out, hipStream_t s) {
     MfMap m;
     size_t lds;
     const int64_t grid = make_mf_map(W, sizeof(T), m, lds);
@@ -2814,53 +2420,11 @@ int q1mf_apply_sub(int W, const T* cell, const T* x, const T* d_in, T* d_out, hi
     hipLaunchKernelGGL(k_q1mf_apply_sub<T>, dim3(grid), dim3(256), lds, s, m, cell, x, d_in, d_out);
     UGX_CHECK_LAUNCH();
 }
-template int q1mf_apply_sub<float>(int, const float*, const float*, const float*, float*, hipStream_t);
-template int q1mf_apply_sub<double>(int, const double*, const double*, const double*, double*, hipStream_t);
-
-// the last post-smoothing step of a cycle fused with the correction update
-// that ends it: z = (double)(sc_new + dinv .* sd_out) for sd_out = sd_in - A st,
-// sc_new = sc + st, st = dinv .* sd_in (the arithmetic of q1mf_jacobi_step
-// followed by jacobi_convert_dot; sd_out and sc_new are not stored). With
-// dot_partial, the per-block partials of (z, r) (n_partial in: capacity, out:
-// number written). -1 when the lattice does not fit the z-marching plan
-template <typename T>
-int q1mf_jacobi_last(int W, const T* cell, const T* dinv, const T* sd_in, const T* sc, double* z, const double* r,
-                     hipStream_t s, double* dot_partial, int* n_partial) {
-    MfZMap zm;
-    size_t zlds;
-    const int64_t zgrid = make_mf_zmap(W, sizeof(T), reinterpret_cast<const void*>(&k_q1mf_z<T, 7>), zm, zlds);
-    if (!zgrid) return -1;
-    if (dot_partial && (!n_partial || zgrid > *n_partial)) return -1;
-    hipLaunchKernelGGL((k_q1mf_z<T, 7>), dim3(zgrid), dim3(256), zlds, s, zm, cell, dinv, sd_in, sc, (T*)nullptr,
-                       (T*)nullptr, 0.0, 0.0, dot_partial, r, z);
-    if (n_partial) *n_partial = (int)zgrid;
-    UGX_CHECK_LAUNCH();
-}
-bool q1mf_last_fits(int W, size_t elem) {
-    MfZMap zm;
-    size_t lds;
-    const void* k = elem == 4 ? reinterpret_cast<const void*>(&k_q1mf_z<float, 7>)
-                              : reinterpret_cast<const void*>(&k_q1mf_z<double, 7>);
-    return make_mf_zmap(W, elem, k, zm, lds) != 0;
-}
-template int q1mf_jacobi_last<float>(int, const float*, const float*, const float*, const float*, double*,
-                                     const double*, hipStream_t, double*, int*);
-template int q1mf_jacobi_last<double>(int, const double*, const double*, const double*, const double*, double*,
-                                      const double*, hipStream_t, double*, int*);
+template int q1mf_planes_apply_sub<float>(int, const float*, const float*, const float*, float*, hipStream_t);
+template int q1mf_planes_apply_sub<double>(int, const double*, const double*, const double*, double*, hipStream_t);
 
 template <typename T>
-int q1mf_axpy(int W, const T* cell, double alpha, const T* v, double beta, const T* x, T* y, hipStream_t s,
-              double* dot_partial, int* n_partial) {
-    MfZMap zm;
-    size_t zlds;
-    if (const int64_t zgrid = make_mf_zmap(W, sizeof(T), reinterpret_cast<const void*>(&k_q1mf_z<T, 2>), zm, zlds)) {
-        if (dot_partial && n_partial && zgrid > *n_partial) return -1;
-        hipLaunchKernelGGL((k_q1mf_z<T, 2>), dim3(zgrid), dim3(256), zlds, s, zm, cell, x, (const T*)nullptr, v, y,
-                           (T*)nullptr, alpha, beta, dot_partial, (const double*)nullptr, (double*)nullptr);
-        if (n_partial) *n_partial = (int)zgrid;
-        UGX_CHECK_LAUNCH();
-    }
-    if (dot_partial) return -1;   // the fused dot needs the z-marching kernel
+int q1mf_planes_axpy(int W, const T* cell, double alpha, const T* v, double beta, const T* x, T* y, hipStream_t s) {
     MfMap m;
     size_t lds;
     const int64_t grid = make_mf_map(W, sizeof(T), m, lds);
@@ -2868,46 +2432,8 @@ int q1mf_axpy(int W, const T* cell, double alpha, const T* v, double beta, const
     hipLaunchKernelGGL(k_q1mf_axpy<T>, dim3(grid), dim3(256), lds, s, m, cell, alpha, v, beta, x, y);
     UGX_CHECK_LAUNCH();
 }
-template int q1mf_axpy<double>(int, const double*, double, const double*, double, const double*, double*, hipStream_t,
-                               double*, int*);
-
-// p_new = fma(beta, p_old, z) (beta = *beta_dev), y = A p_new and the (y, p_new)
-// partials in one pass; p_new must not alias p_old (other workgroups still
-// stage p_old around their bands)
-template <typename T>
-int q1mf_direction_axpy(int W, const T* cell, const T* p_old, const T* z, const double* beta_dev, T* p_new, T* y,
-                        hipStream_t s, double* dot_partial, int* n_partial) {
-    if (p_new == p_old) return -1;
-    MfZMap zm;
-    size_t zlds;
-    const int64_t zgrid = make_mf_zmap(W, sizeof(T), reinterpret_cast<const void*>(&k_q1mf_z<T, 5>), zm, zlds);
-    if (!zgrid || !dot_partial || !n_partial || zgrid > *n_partial) return -1;
-    hipLaunchKernelGGL((k_q1mf_z<T, 5>), dim3(zgrid), dim3(256), zlds, s, zm, cell, p_old, z, (const T*)nullptr, y,
-                       p_new, 0.0, 1.0, dot_partial, beta_dev, (double*)nullptr);
-    *n_partial = (int)zgrid;
-    UGX_CHECK_LAUNCH();
-}
-template int q1mf_direction_axpy<double>(int, const double*, const double*, const double*, const double*, double*,
-                                         double*, hipStream_t, double*, int*);
-
-// asks the runtime for the residency of every z-marching kernel at lattice
-// width W, so that no query happens inside a captured cycle
-int q1mf_prepare(int W) {
-    MfZMap zm;
-    size_t lds;
-    make_mf_zmap(W, 4, reinterpret_cast<const void*>(&k_q1mf_z<float, 0>), zm, lds);
-    make_mf_zmap(W, 4, reinterpret_cast<const void*>(&k_q1mf_z<float, 1>), zm, lds);
-    make_mf_zmap(W, 4, reinterpret_cast<const void*>(&k_q1mf_z<float, 3>), zm, lds);
-    make_mf_zmap(W, 4, reinterpret_cast<const void*>(&k_q1mf_z<float, 4>), zm, lds);
-    make_mf_zmap(W, 4, reinterpret_cast<const void*>(&k_q1mf_z<float, 7>), zm, lds);
-    make_mf_zmap(W, 8, reinterpret_cast<const void*>(&k_q1mf_z<double, 7>), zm, lds);
-    make_mf_zmap(W, 8, reinterpret_cast<const void*>(&k_q1mf_z<double, 3>), zm, lds);
-    make_mf_zmap(W, 8, reinterpret_cast<const void*>(&k_q1mf_z<double, 0>), zm, lds);
-    make_mf_zmap(W, 8, reinterpret_cast<const void*>(&k_q1mf_z<double, 1>), zm, lds);
-    make_mf_zmap(W, 8, reinterpret_cast<const void*>(&k_q1mf_z<double, 2>), zm, lds);
-    make_mf_zmap(W, 8, reinterpret_cast<const void*>(&k_q1mf_z<double, 5>), zm, lds);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
-}
+template int q1mf_planes_axpy<double>(int, const double*, double, const double*, double, const double*, double*,
+                                      hipStream_t);
 
 template <typename T>
 int q1mf_coeff(int64_t ne, double h, const double* theta, T* c, hipStream_t s) {
@@ -3019,6 +2545,10 @@ template int prolong_add<double>(int, int, int, int64_t, const double*, const ui
 template int prolong_add<float>(int, int, int, int64_t, const float*, const uint8_t*, float*, float*, hipStream_t,
                                 const float*, const float*);
 
+// at most this many workgroups per CU are planned for (8 or 10, more and
+// shorter chunks, measured 37.3 against 31.6 us at 257^3 -> 129^3)
+constexpr int kRzResident = 7;
+
 // plan of k_restrict3_z: 2-line bands (1-line when a staged plane would not
 // fit the slots) grouped per XCD, chunks so that the grid is one round;
 // returns the grid, 0 when the plan does not apply
@@ -3042,7 +2572,7 @@ static int64_t make_rz_map(int Wc, int Wf, RzMap& m, size_t& lds) {
     }
     if (maxg == 0) return 0;
     const int64_t slots = (int64_t)(device_cus() / 8) *
-                          std::min(UGX_MF_MAXRES, mf_resident_blocks(reinterpret_cast<const void*>(&k_restrict3_z<TV>), lds));
+                          std::min(kRzResident, resident_blocks(reinterpret_cast<const void*>(&k_restrict3_z<TV>), lds));
     int64_t nch = slots / maxg;
     nch = std::min<int64_t>(std::max<int64_t>(nch, 1), std::max(1, Wc / 2));
     m.nchunks = (int32_t)nch;

@@ -85,13 +85,26 @@ int dia_axpy(int64_t n, int nd, const int32_t* off, const TM* A, double alpha, c
 template <typename TM, typename TV>
 int dia_jacobi_step(int64_t n, int nd, const int32_t* off, const TM* A, const TV* dinv, const TV* sd_in, TV* sd_out,
                     TV* sc, hipStream_t s);
+// workgroups of `kernel` (256 threads, `lds` bytes of dynamic LDS) resident on
+// one CU, and the device's CU count; both asked once and kept
+int resident_blocks(const void* kernel, size_t lds);
+int device_cus();
 // residency queries of the matrix-free kernels at lattice width W, made
 // before any cycle is captured into a graph
 int q1mf_prepare(int W);
+// whether q1mf_kernels.hip has a schedule for this lattice width: then every
+// function below applies, otherwise only q1mf_jacobi_step, q1mf_apply_sub and
+// q1mf_axpy without partial sums (the plane-by-plane kernels)
+bool q1mf_fused_fits(int W);
+template <typename T>
+int q1mf_planes_jacobi_step(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s);
+template <typename T>
+int q1mf_planes_apply_sub(int W, const T* cell, const T* x, const T* d_in, T* d_out, hipStream_t s);
+template <typename T>
+int q1mf_planes_axpy(int W, const T* cell, double alpha, const T* v, double beta, const T* x, T* y, hipStream_t s);
 // the first Jacobi step of a cycle from the FP64 defect d64 and a zero
 // correction (sd_out = (T)d64 - A st, sc = st, st = dinv .* (T)d64), when
-// q1mf_first_fits(W, sizeof(T)) (the z-marching plan applies)
-bool q1mf_first_fits(int W, size_t elem);
+// q1mf_fused_fits(W)
 template <typename T>
 int q1mf_jacobi_first(int W, const T* cell, const T* dinv, const double* d64, T* sd_out, T* sc, hipStream_t s);
 // the CG direction update fused with the operator: p_new = fma(*beta_dev,
@@ -139,12 +152,10 @@ int q1mf_apply_sub(int W, const T* cell, const T* x, const T* d_in, T* d_out, hi
 // its conversion: z = (double)(sc + st + dinv .* (sd_in - A st)), st =
 // dinv .* sd_in (q1mf_jacobi_step then jacobi_convert_dot, without storing the
 // step's outputs); with dot_partial also the (z, r) partials (n_partial in:
-// capacity, out: number written). q1mf_last_fits(W, sizeof(T)) tells whether
-// the plan applies.
+// capacity, out: number written); q1mf_fused_fits(W)
 template <typename T>
 int q1mf_jacobi_last(int W, const T* cell, const T* dinv, const T* sd_in, const T* sc, double* z, const double* r,
                      hipStream_t s, double* dot_partial, int* n_partial);
-bool q1mf_last_fits(int W, size_t elem);
 // dot_partial (optional): per-block partial sums of y.x (n_partial in: capacity,
 // out: number written); needs the z-marching kernel
 template <typename T>
