@@ -616,6 +616,9 @@ class DomainDiscretization {
     // assemble a level operator in lattice numbering as DIA values (27 or 9
     // diagonals of length N, FP64), Dirichlet rows set
     void assemble_level_dia(int lev, DeviceBuffer<double>& dia, int& nd, std::vector<int32_t>& offsets);
+    // kind 0: the level operator in the forms the multigrid keeps (q1_level)
+    template <typename T>
+    void assemble_level_q1(int lev, double omega, T* full, T* up, T* dinv, double* up64, int* bad);
     // coordinates of the level's DoFs in DoF order (2 or 3 per DoF), as the
     // grid function's approximation space would give them to
     // SaveMatrixForConnectionViewer (grid_function_util.h)

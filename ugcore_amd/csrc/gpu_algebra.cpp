@@ -1964,6 +1964,14 @@ void DomainDiscretization::assemble_level_dia(int lev, DeviceBuffer<double>& dia
     UGX_LAUNCH(dirichlet_dia<double>(L.N, nd, nd / 2, L.dir.get(), dia.get(), c.stream));
 }
 
+template <typename T>
+void DomainDiscretization::assemble_level_q1(int lev, double omega, T* full, T* up, T* dinv, double* up64, int* bad) {
+    if (kind_ != 0) throw UGError("assemble_level_q1: hexahedra only");
+    LevelGrid& L = *levels_[lev];
+    UGX_LAUNCH(q1_level<T>(L.n, 1 << refs_, 1.0 / L.n, q1_tables_device(), exp_theta_device(), omega, full, up, dinv,
+                           up64, bad, context().stream));
+}
+
 // ---------------------------------------------------------------------------
 // AssembledMultiGridCycle
 // ---------------------------------------------------------------------------
@@ -2132,10 +2140,28 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                           "hierarchy)");
     }
 
-    void alloc_vec(DeviceBuffer<T>& buf, T*& p, int64_t N, int64_t H) {
-        buf.resize(N + 2 * H);
-        buf.zero();
-        p = buf.get() + H;
+    // the vectors of a level, their halos zero; every kernel writes its part of
+    // [0, N) before another reads it
+    void alloc_vectors(GmgLevel<T>& l) {
+        struct {
+            DeviceBuffer<T>* b;
+            T** p;
+        } v[5] = {{&l.b_dinv, &l.dinv}, {&l.b_sc, &l.sc}, {&l.b_sd, &l.sd}, {&l.b_sd2, &l.sd2}, {&l.b_st, &l.st}};
+        T* base[5];
+        for (int k = 0; k < 5; ++k) {
+            v[k].b->resize(l.N + 2 * l.H);
+            base[k] = v[k].b->get();
+            *v[k].p = base[k] + l.H;
+        }
+        UGX_LAUNCH(zero_halos<T>(l.N, l.H, base, context().stream));
+    }
+
+    void check_diagonal(int lev) {
+        auto& c = context();
+        int bad = 0;
+        UGX_HIP(hipMemcpyAsync(&bad, c.flag, sizeof(int), hipMemcpyDeviceToHost, c.stream));
+        sync();
+        if (bad && lev > base) throw UGError("GMG: Jacobi found a zero diagonal");
     }
 
     void init() override {
@@ -2190,6 +2216,24 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
             l.dir = G.dir.get();
             const int64_t W = G.W;
             l.H = G.dim == 3 ? ((W * W + W + 1 + 63) / 64) * 64 : ((W + 1 + 63) / 64) * 64;
+            alloc_vectors(l);
+            if (disc->kind() == 0 && !rap && !transposed && lev > base) {
+                // every form of the level's operator from one pass; the FP64
+                // copy of the top level's is the lattice CG's operator where
+                // that is not applied matrix-free
+                disc->level_dia_layout(lev, l.nd, l.off);
+                l.A.resize(dia_tiled_size(l.N, 14));
+                l.Afull.resize(dia_tiled_size(l.N, 27));
+                double* up64 = nullptr;
+                if (lev == top && !mf) {
+                    surf.resize(dia_tiled_size(l.N, 14));
+                    up64 = surf.get();
+                }
+                UGX_HIP(hipMemsetAsync(c.flag, 0, sizeof(int), c.stream));
+                disc->template assemble_level_q1<T>(lev, omega, l.Afull.get(), l.A.get(), l.dinv, up64, c.flag);
+                check_diagonal(lev);
+                continue;
+            }
             DeviceBuffer<double> A64;
             if (rap) {
                 A64 = std::move(galerkin[lev]);
@@ -2204,11 +2248,6 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                 UGX_LAUNCH(dia_transpose_elim<double>(l.W, l.N, l.dir, A64.get(), AT.get(), c.stream));
                 A64 = std::move(AT);
             }
-            alloc_vec(l.b_dinv, l.dinv, l.N, l.H);
-            alloc_vec(l.b_sc, l.sc, l.N, l.H);
-            alloc_vec(l.b_sd, l.sd, l.N, l.H);
-            alloc_vec(l.b_sd2, l.sd2, l.N, l.H);
-            alloc_vec(l.b_st, l.st, l.N, l.H);
             // Jacobi: diagInv = 1/(a_ii * (1/omega)) from the FP64 centre diagonal
             DeviceBuffer<double> dinv64(l.N);
             UGX_HIP(hipMemsetAsync(c.flag, 0, sizeof(int), c.stream));
@@ -2249,17 +2288,14 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                     UGX_LAUNCH((convert<double, T>(A64.size(), A64.get(), l.Afull.get(), c.stream)));
                     UGX_LAUNCH((convert<double, T>(l.N, dinv64.get(), l.dinv, c.stream)));
                 }
-                sync();
-                int bad = 0;
-                UGX_HIP(hipMemcpy(&bad, c.flag, sizeof(int), hipMemcpyDeviceToHost));
-                if (bad && lev > base) throw UGError("GMG: Jacobi found a zero diagonal");
+                check_diagonal(lev);
                 continue;
             }
             // symmetric Dirichlet-eliminated storage of the level operator
             const int nu = l.nd / 2 + 1;
             DeviceBuffer<double> U64(dia_tiled_size(l.N, nu));
             UGX_LAUNCH(dia_symmetrize<double>(l.N, l.nd, l.off.data(), l.dir, A64.get(), U64.get(), c.stream));
-            if (lev == top) {
+            if (lev == top && !mf) {
                 // the surface operator in lattice order (FP64, symmetric
                 // storage) for the CG fast path
                 surf.resize(U64.size());
@@ -2277,10 +2313,7 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                 UGX_LAUNCH((convert<double, T>(A64.size(), A64.get(), l.Afull.get(), c.stream)));
                 UGX_LAUNCH((convert<double, T>(l.N, dinv64.get(), l.dinv, c.stream)));
             }
-            sync();
-            int bad = 0;
-            UGX_HIP(hipMemcpy(&bad, c.flag, sizeof(int), hipMemcpyDeviceToHost));
-            if (bad && lev > base) throw UGError("GMG: Jacobi found a zero diagonal");
+            check_diagonal(lev);
         }
         plan_coarse_cycle();
     }

@@ -2063,6 +2063,15 @@ __global__ void k_dirichlet_dia(int64_t n, int nd, int centre, const uint8_t* di
     }
 }
 
+// the zero halos of up to five level vectors (n entries between h and h zeros)
+template <typename T>
+__global__ __launch_bounds__(256) void k_zero_halos(int64_t n, int64_t h, T* a, T* b, T* c, T* d, T* e) {
+    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (i >= 2 * h) return;
+    const int64_t j = i < h ? i : n + i;
+    a[j] = b[j] = c[j] = d[j] = e[j] = (T)0;
+}
+
 // convert DIA values between precisions
 template <typename TA, typename TB>
 __global__ __launch_bounds__(256) void k_convert(int64_t n, const TA* a, TB* b) {
@@ -2673,6 +2682,16 @@ int convert(int64_t n, const TA* a, TB* b, hipStream_t s) {
 template int convert<double, float>(int64_t, const double*, float*, hipStream_t);
 template int convert<float, double>(int64_t, const float*, double*, hipStream_t);
 template int convert<double, double>(int64_t, const double*, double*, hipStream_t);
+
+template <typename T>
+int zero_halos(int64_t n, int64_t h, T* const (&v)[5], hipStream_t s) {
+    if (h <= 0) return 0;
+    hipLaunchKernelGGL(k_zero_halos<T>, dim3((unsigned)((2 * h + 255) / 256)), dim3(256), 0, s, n, h, v[0], v[1], v[2], v[3],
+                       v[4]);
+    UGX_CHECK_LAUNCH();
+}
+template int zero_halos<float>(int64_t, int64_t, float* const (&)[5], hipStream_t);
+template int zero_halos<double>(int64_t, int64_t, double* const (&)[5], hipStream_t);
 
 int boundary_flags(int dim, int W, int64_t n, uint8_t* dir, hipStream_t s) {
     hipLaunchKernelGGL(k_boundary_flags, dim3(vec_grid(n)), dim3(256), 0, s, dim, W, n, dir);

@@ -301,6 +301,83 @@ __global__ __launch_bounds__(256) void k_q1_lattice_dia(int n, int sub, int o0, 
     }
 }
 
+// A Q1 level operator in the forms the multigrid keeps, one row per thread:
+// all 27 diagonals and the Dirichlet-eliminated upper 14 (tiled, in the
+// levels' precision; the upper ones also in FP64 where asked for) and the
+// damped inverse diagonal; Dirichlet rows are identity rows. Entries, their
+// order of summation and their roundings are those of k_q1_lattice_dia,
+// dirichlet_dia, dia_symmetrize, dia_jacobi_diag and the conversions, in one
+// pass that writes each result once: 64 (PER_POINT: 512) multiply-adds a row
+// with the element tables in scalar registers, where 32 lanes a row each
+// tested all 8 elements. 129^3 and its coarser levels, FP32, one MI355X:
+// 870 us for the separate passes, 122 us.
+template <typename T, bool PER_POINT>
+__global__ __launch_bounds__(256) void k_q1_level(int n, int sub, int o0, int o1, double h,
+                                                  const double* __restrict__ tab, const double* __restrict__ kfine,
+                                                  double omega, T* __restrict__ full, T* __restrict__ up,
+                                                  T* __restrict__ dinv, double* __restrict__ up64,
+                                                  int* __restrict__ bad) {
+    const int W = n + 1, nf = n * sub;
+    const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (i >= (int64_t)W * W * W) return;
+    const int yz = (int)(i / W), x = (int)(i - (int64_t)yz * W), z = yz / W, y = yz - z * W;
+    const bool bnd = x == 0 || y == 0 || z == 0 || x == n || y == n || z == n;
+    double v[27];
+#pragma unroll
+    for (int d = 0; d < 27; ++d) v[d] = 0.0;
+    if (!bnd) {
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+            const int ox = o & 1, oy = (o >> 1) & 1, oz = o >> 2;
+            const int ex = x - 1 + ox, ey = y - 1 + oy, ez = z - 1 + oz;
+            const int a = hex_local(1 - ox, 1 - oy, 1 - oz);
+            if (!PER_POINT) {
+                const double k = kfine ? kfine[((int64_t)ez * n + ey) * n + ex] : 1.0;
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    const int bx = c & 1, by = (c >> 1) & 1, bz = c >> 2;
+                    const int d = (oz + bz) * 9 + (oy + by) * 3 + ox + bx;
+                    v[d] = fma(k, tab[kK + 8 * a + hex_local(bx, by, bz)], v[d]);
+                }
+            } else {
+                double kq[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int cx = ex * sub + ((q & 1) ? o1 : o0), cy = ey * sub + ((q & 2) ? o1 : o0),
+                              cz = ez * sub + ((q & 4) ? o1 : o0);
+                    kq[q] = kfine[((int64_t)cz * nf + cy) * nf + cx];
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) {
+                        const int bx = c & 1, by = (c >> 1) & 1, bz = c >> 2;
+                        const int d = (oz + bz) * 9 + (oy + by) * 3 + ox + bx;
+                        v[d] = fma(kq[q], tab[kG + 64 * q + 8 * a + hex_local(bx, by, bz)], v[d]);
+                    }
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < 27; ++d) v[d] *= h;
+    } else {
+        v[13] = 1.0;
+    }
+#pragma unroll
+    for (int d = 0; d < 27; ++d) full[dia_tiled_index(d, i, 27)] = (T)v[d];
+#pragma unroll
+    for (int u = 0; u < 14; ++u) {
+        const int d = 13 + u, qx = x + d % 3 - 1, qy = y + (d / 3) % 3 - 1, qz = z + d / 9 - 1;
+        const bool drop = u != 0 && (qx == 0 || qy == 0 || qz == 0 || qx == n || qy == n || qz == n);
+        const double w = drop ? 0.0 : v[d];
+        up[dia_tiled_index(u, i, 14)] = (T)w;
+        if (up64) up64[dia_tiled_index(u, i, 14)] = w;
+    }
+    double m = v[13];
+    m *= 1.0 / omega;
+    if (m == 0.0) bad[0] = 1;
+    dinv[i] = m == 0.0 ? (T)0 : (T)(1.0 / m);
+}
+
 __global__ void k_exp_values(int64_t n, const double* __restrict__ theta, double* __restrict__ out) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         out[i] = exp(theta[i]);
@@ -357,6 +434,27 @@ int lattice_pattern(int dim, int W, const int32_t* dof_of_lat, const int32_t* rp
                            rp_lat, col);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
+
+template <typename T>
+int q1_level(int n, int nfine, double h, const double* tab, const double* kfine, double omega, T* full, T* up, T* dinv,
+             double* up64, int* bad, hipStream_t s) {
+    if (n <= 0 || nfine % n != 0) return -1;
+    const int64_t W = n + 1, nb = (W * W * W + 255) / 256;
+    const int sub = nfine / n;
+    const double g = 0.5 / std::sqrt(3.0);
+    const int o0 = (int)std::floor((0.5 - g) * sub), o1 = (int)std::floor((0.5 + g) * sub);
+    if (kfine && sub > 1)
+        hipLaunchKernelGGL((k_q1_level<T, true>), dim3((unsigned)nb), dim3(256), 0, s, n, sub, o0, o1, h, tab, kfine,
+                           omega, full, up, dinv, up64, bad);
+    else
+        hipLaunchKernelGGL((k_q1_level<T, false>), dim3((unsigned)nb), dim3(256), 0, s, n, sub, o0, o1, h, tab, kfine,
+                           omega, full, up, dinv, up64, bad);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+template int q1_level<float>(int, int, double, const double*, const double*, double, float*, float*, float*, double*,
+                             int*, hipStream_t);
+template int q1_level<double>(int, int, double, const double*, const double*, double, double*, double*, double*,
+                              double*, int*, hipStream_t);
 
 int exp_values(int64_t n, const double* theta, double* out, hipStream_t s) {
     if (n <= 0) return 0;

@@ -238,6 +238,15 @@ int dirichlet_dia(int64_t n, int nd, int centre, const uint8_t* dir, TM* dia, hi
 template <typename TA, typename TB>
 int convert(int64_t n, const TA* a, TB* b, hipStream_t s);
 int boundary_flags(int dim, int W, int64_t n, uint8_t* dir, hipStream_t s);
+// five vectors of n entries with h entries on either side: those are set to 0
+template <typename T>
+int zero_halos(int64_t n, int64_t h, T* const (&v)[5], hipStream_t s);
+// a Q1 level operator as the multigrid keeps it: all diagonals, the
+// Dirichlet-eliminated upper ones (also in FP64 into up64 unless null), the
+// damped inverse diagonal; *bad = 1 for a zero diagonal
+template <typename T>
+int q1_level(int n, int nfine, double h, const double* tab, const double* kfine, double omega, T* full, T* up, T* dinv,
+             double* up64, int* bad, hipStream_t s);
 int adjoint_grad_q1_hex(int n, double h, const double* theta, const int32_t* dof_of_lat, int64_t n_inner,
                         const double* u, const double* lambda, double* grad, hipStream_t s);
 int zero_range(int64_t lo, int64_t hi, double* x, hipStream_t s);
