@@ -244,6 +244,11 @@ class GPUSparseMatrix {
         sell_enabled_ = layout >= 1;
         build_spmv_layout();
     }
+    // Q1 values of the n^3 element lattice this pattern belongs to, into the CSR
+    // and the dictionary layout in one pass, with the load vector; false (and
+    // nothing written) when the layout is not a dictionary of this pattern
+    bool set_q1_values(int n, double h, double f_const, const double* tab, const double* kel, const int32_t* lat_of_dof,
+                       double* rhs);
     // the dictionary layout in another numbering of rows and columns (map: row
     // or column -> its number there, a device array): slots and dictionary
     bool dictionary_ready() const { return dict_valid_ && rows_ == cols_; }

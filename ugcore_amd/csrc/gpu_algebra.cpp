@@ -811,6 +811,15 @@ void GPUSparseMatrix::cycle_product(const double* w, const SellEpilogue& e) cons
                           w, rowptr_.get(), has_row_order() ? row_order_.get() : nullptr, e, context().stream));
 }
 
+bool GPUSparseMatrix::set_q1_values(int n, double h, double f_const, const double* tab, const double* kel,
+                                    const int32_t* lat_of_dof, double* rhs) {
+    if (building_ || !dict_valid_ || layout_pattern_id_ != pattern_id_) return false;
+    UGX_LAUNCH(dict_q1_values(n, slice_order_.size() / 64, h, f_const, tab, kel, lat_of_dof, slice_order_.get(),
+                              rowptr_.get(), d_width_.get(), d_dptr_.get(), d_dict_.get(), d_vptr_.get(),
+                              d_iptr_.get(), d_idx_.get(), d_val_.get(), val_.get(), rhs, context().stream));
+    return true;
+}
+
 void GPUSparseMatrix::renumber_dictionary(const int32_t* map, DeviceBuffer<int32_t>& order,
                                           DeviceBuffer<int32_t>& dict) const {
     auto& c = context();
@@ -1862,6 +1871,13 @@ void DomainDiscretization::assemble_linear(GPUSparseMatrix& A, GPUVector& b) {
     if (kind_ == 0) {
         // row by row: every entry and every rhs entry written once
         if (nfine != L.n) throw UGError("assemble_linear: the top level must be the fine level");
+        if (reuse && A.set_q1_values(L.n, hsz, f_const_, q1_tables_device(), exp_theta_device(), L.lat_of_dof.get(),
+                                     b.data())) {
+            A.set_origin(this);
+            sync();
+            t_assemble_ = wall() - t0;
+            return;
+        }
         if (rp_lat_.size() != L.N) {
             rp_lat_.resize(L.N);
             UGX_LAUNCH(rowptr_of_lattice(L.N, L.dof_of_lat.get(), A.rowptr(), rp_lat_.get(), c.stream));

@@ -410,6 +410,137 @@ __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslice
     }
 }
 
+// Q1 values (and load vector) of a lattice operator whose pattern and
+// dictionary are in place, into the CSR and the dictionary layout in one pass,
+// one wave per slice, one row per lane. A lane forms the 27 entries of its row
+// in registers (64 multiply-adds; the same order as k_q1_lattice_csr, so the
+// same bits) and leaves them in LDS by direction. The row's entries are the
+// slice's dictionary positions, so the direction of entry k is the lattice
+// difference between that dictionary column and the row: the layout's pairs are
+// written from there in entry order, and the CSR rows, two at a time, by lanes
+// that own a direction and its rank in the row. Boundary rows are identity
+// rows with a zero load.
+// Bound by the two writes of 8 bytes per entry. One pass for the CSR with 32
+// lanes a row (ranks by shuffles, every lane testing all 8 elements), one for
+// the Dirichlet rows and one that read the CSR back for the layout took 695 us
+// at 129^3 (57,066,625 entries) on one MI355X; this pass 325 us.
+__global__ __launch_bounds__(64) void k_dict_q1_values(int n, int64_t nslices, double h, double fh3,
+                                                       const double* __restrict__ tab,
+                                                       const double* __restrict__ kel,
+                                                       const int32_t* __restrict__ lat_of_dof,
+                                                       const int32_t* __restrict__ order,
+                                                       const int32_t* __restrict__ rowptr,
+                                                       const int32_t* __restrict__ width,
+                                                       const int32_t* __restrict__ dptr,
+                                                       const int32_t* __restrict__ dict,
+                                                       const int64_t* __restrict__ vptr,
+                                                       const int64_t* __restrict__ iptr,
+                                                       const uint32_t* __restrict__ sidx, double* __restrict__ sval,
+                                                       double* __restrict__ val, double* __restrict__ rhs) {
+    constexpr int P = 65;   // row pitch of a direction: the reads along a row hit different banks
+    __shared__ double v[27 * P];
+    __shared__ uint8_t rank[27 * 64];
+    __shared__ int32_t code[256], rb[64];
+    const int lane = threadIdx.x, W = n + 1;
+    const int64_t per = (nslices + 7) / 8;
+    const int64_t t = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);   // consecutive slices on one XCD
+    if ((blockIdx.x >> 3) >= per || t >= nslices) return;
+    auto point = [&](int32_t l, int& x, int& y, int& z) {
+        const int yz = l / W;
+        x = l - yz * W;
+        z = yz / W;
+        y = yz - z * W;
+    };
+    const int32_t r = order[t * 64 + lane];
+    const int w = width[t];
+    const int32_t d0 = dptr[t], nd = dptr[t + 1] - d0;
+    // everything that the chains of dependent loads below end in is requested
+    // up front: positions, dictionary, rows
+    const uint32_t* ip = sidx + iptr[t] + lane;
+    uint32_t word[7];
+#pragma unroll
+    for (int j = 0; j < 7; ++j) word[j] = 4 * j < w ? __builtin_nontemporal_load(ip + 64 * j) : 0u;
+    int32_t lp[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) lp[j] = nd > 0 ? dict[d0 + (lane + 64 * j < nd ? lane + 64 * j : 0)] : 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) lp[j] = lat_of_dof[lp[j]];
+    // lattice points as x | y << 10 | z << 20
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        int x, y, z;
+        point(lp[j], x, y, z);
+        if (lane + 64 * j < nd) code[lane + 64 * j] = x | y << 10 | z << 20;
+    }
+    for (int i = lane; i < 27 * 64; i += 64) rank[i] = 255;
+    int x = 0, y = 0, z = 0, len = 0;
+    rb[lane] = 0;
+    if (r >= 0) {
+        point(lat_of_dof[r], x, y, z);
+        rb[lane] = rowptr[r];
+        len = rowptr[r + 1] - rowptr[r];
+    }
+    const bool inner = r >= 0 && x > 0 && y > 0 && z > 0 && x < n && y < n && z < n;
+    double e[27], f = 0.0;
+#pragma unroll
+    for (int d = 0; d < 27; ++d) e[d] = 0.0;
+    if (inner) {
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+            const int ox = o & 1, oy = (o >> 1) & 1, oz = o >> 2;
+            // local index of a corner in the reference hexahedron
+            auto local = [](int cx, int cy, int cz) { return 4 * cz + (cy ? 3 - cx : cx); };
+            const int a = local(1 - ox, 1 - oy, 1 - oz);
+            const double k = kel ? kel[((int64_t)(z - 1 + oz) * n + y - 1 + oy) * n + x - 1 + ox] : 1.0;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const int bx = c & 1, by = (c >> 1) & 1, bz = c >> 2;
+                const int d = (oz + bz) * 9 + (oy + by) * 3 + ox + bx;
+                e[d] = fma(k, tab[512 + 8 * a + local(bx, by, bz)], e[d]);
+            }
+            f += tab[576 + a];
+        }
+#pragma unroll
+        for (int d = 0; d < 27; ++d) e[d] *= h;
+    } else {
+        e[13] = 1.0;
+    }
+#pragma unroll
+    for (int d = 0; d < 27; ++d) v[d * P + lane] = e[d];
+    if (rhs && r >= 0) rhs[r] = inner ? fh3 * f : 0.0;
+    __syncthreads();
+    // the layout's pairs in entry order, and the rank of every direction
+    dbl2* vp = reinterpret_cast<dbl2*>(sval + vptr[t]) + lane;
+    const int own = (x | y << 10 | z << 20) - (1 | 1 << 10 | 1 << 20);
+#pragma unroll
+    for (int j = 0; j < 7; ++j) {
+        const int k = 4 * j;
+        if (k >= w) break;
+        double q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            q[u] = 0.0;
+            if (k + u < len) {
+                const int df = code[(word[j] >> (8 * u)) & 255u] - own;
+                const int d = ((df >> 20) & 3) * 9 + ((df >> 10) & 3) * 3 + (df & 3);
+                q[u] = v[d * P + lane];
+                rank[d * 64 + lane] = (uint8_t)(k + u);
+            }
+        }
+        const dbl2 p0 = {q[0], q[1]}, p1 = {q[2], q[3]};
+        __builtin_nontemporal_store(p0, vp + 64 * (k >> 1));
+        if (k + 2 < w) __builtin_nontemporal_store(p1, vp + 64 * ((k >> 1) + 1));
+    }
+    __syncthreads();
+    const int d = lane & 31, half = lane >> 5;
+    if (d < 27)
+#pragma unroll 8
+        for (int j = half; j < 64; j += 2) {
+            const int k = rank[d * 64 + j];
+            if (k != 255) val[(int64_t)rb[j] + k] = v[d * P + j];
+        }
+}
+
 // the rows of a lattice in blocks of 64 points: 4x4x4 (3D) or 8x8 (2D). Slot
 // 64*b + l of block b (x fastest over the blocks) holds the DoF of the block's
 // point l (x fastest inside the block), -1 where the block extends past the
@@ -516,6 +647,17 @@ template int dict_spmv_dots<float>(int64_t, int64_t, const int32_t*, const int32
 template int dict_spmv_dots<double>(int64_t, int64_t, const int32_t*, const int32_t*, const int32_t*, const int64_t*,
                                     const int64_t*, const double*, const uint32_t*, const int32_t*, const double*,
                                     double*, const double*, double*, hipStream_t);
+
+int dict_q1_values(int n, int64_t nslices, double h, double f_const, const double* tab, const double* kel,
+                   const int32_t* lat_of_dof, const int32_t* order, const int32_t* rowptr, const int32_t* width,
+                   const int32_t* dptr, const int32_t* dict, const int64_t* vptr, const int64_t* iptr,
+                   const uint32_t* sidx, double* sval, double* val, double* rhs, hipStream_t s) {
+    if (n <= 0 || n >= 1023 || nslices <= 0) return -1;
+    const int64_t per = (nslices + 7) / 8;
+    hipLaunchKernelGGL(k_dict_q1_values, dim3((unsigned)(8 * per)), dim3(64), 0, s, n, nslices, h, f_const * h * h * h,
+                       tab, kel, lat_of_dof, order, rowptr, width, dptr, dict, vptr, iptr, sidx, sval, val, rhs);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
 
 int64_t lattice_block_slots(int dim, int W) {
     const int e = dim == 3 ? 4 : 8;

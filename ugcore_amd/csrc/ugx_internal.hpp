@@ -452,6 +452,13 @@ int dict_fill(int64_t nslices, int64_t nrows, const int32_t* rowptr, const int32
 // the values alone into an existing dictionary layout of the same pattern
 int dict_values(int64_t nslices, int64_t nrows, const int32_t* rowptr, const double* val, const int32_t* order,
                 const int32_t* width, const int64_t* vptr, double* sval, hipStream_t s);
+// the Q1 operator of the n^3 element lattice (tab: q1_lattice_tables, kel per
+// element or null) into an existing lattice pattern's CSR values and
+// dictionary values, and its load vector (nullable)
+int dict_q1_values(int n, int64_t nslices, double h, double f_const, const double* tab, const double* kel,
+                   const int32_t* lat_of_dof, const int32_t* order, const int32_t* rowptr, const int32_t* width,
+                   const int32_t* dptr, const int32_t* dict, const int64_t* vptr, const int64_t* iptr,
+                   const uint32_t* sidx, double* sval, double* val, double* rhs, hipStream_t s);
 // y = alpha*v1 + beta*A*x (mode 0) or y = beta*A*x on rows with entries (mode 1)
 int dict_spmv(int64_t nrows, int64_t nslices, const int32_t* width, const int32_t* dptr, const int32_t* dict,
               const int64_t* vptr, const int64_t* iptr, const double* sval, const uint32_t* sidx,
