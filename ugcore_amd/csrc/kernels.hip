@@ -266,10 +266,8 @@ __global__ __launch_bounds__(64) void k_sell_fill(int64_t nrows, int64_t ncols, 
 // rows: 400,003 rows of about 16 entries, 57 us, bound by the gathers. Where rows
 // are wide and few (Q2 operators and transfers: up to 125 entries, 1 - 560
 // slices), one lane's chain of loads and gathers is the time: 20 - 30 us
-// whatever the size with one wave, 9.8 - 13.7 us with four (one MI355X, 729 -
-// 35,937 rows); with sixteen the chain is one round of eight entries and the
-// solve with these matrices takes 2.57 ms instead of 2.71. sell_waves() draws the
-// line.
+// whatever the size with one wave, 6.3 - 14.9 us with four or sixteen (one
+// MI355X, 729 - 35,937 rows). sell_waves() draws the line.
 constexpr int sell_block(int waves) { return waves == 1 ? 256 : 64 * waves; }
 
 template <typename TM, typename TV, int WAVES>
@@ -2719,12 +2717,13 @@ template int sell_fill<double>(int64_t, int64_t, const int32_t*, const int32_t*,
                                const int64_t*, const int32_t*, int32_t*, double*, hipStream_t, bool);
 
 // Several waves a slice where the slices do not fill the chip by themselves
-// (fewer than 16 waves a CU), so that a wave has at most about eight entries:
-// one wave 23.5 us on 35,937 rows of up to 125 entries, four 13.7, sixteen less
-// again; 7.5 - 9.2 us with one wave on rows of up to 27 entries.
+// (fewer than 16 waves a CU). Rows of up to 125 entries: 568 slices 23.5 us with
+// one wave, 14.9 with four, 18.3 with sixteen; 80 slices 13.0 with four and 11.0
+// with sixteen, 12 slices 11.9 and 7.6: sixteen where a CU has at most one slice.
+// Rows of up to 27 entries: 7.5 - 9.2 us with one wave, 4.0 - 5.5 with four.
 static int sell_waves(int64_t nslices, int max_width) {
     if (nslices >= (int64_t)device_cus() * 16 || max_width <= 8) return 1;
-    return max_width > 32 ? 16 : 4;
+    return max_width > 32 && nslices <= device_cus() ? 16 : 4;
 }
 
 template <typename TM, typename TV, int WAVES>
