@@ -2172,14 +2172,6 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         UGX_LAUNCH(zero_halos<T>(l.N, l.H, base, context().stream));
     }
 
-    void check_diagonal(int lev) {
-        auto& c = context();
-        int bad = 0;
-        UGX_HIP(hipMemcpyAsync(&bad, c.flag, sizeof(int), hipMemcpyDeviceToHost, c.stream));
-        sync();
-        if (bad && lev > base) throw UGError("GMG: Jacobi found a zero diagonal");
-    }
-
     void init() override {
         auto& c = context();
         clear_graphs();
@@ -2223,9 +2215,15 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                                    galerkin[lev - 1].get(), c.stream));
             }
         }
+        // what the kernels find on the way, read once at the end: a zero diagonal
+        // per level, then a singular base matrix
+        std::vector<int> found(top + 2, 0);
+        DeviceBuffer<int> flags((int64_t)found.size());
+        flags.upload(found.data(), (int64_t)found.size());
         for (int lev = base; lev <= top; ++lev) {
             LevelGrid& G = disc->level(lev);
             GmgLevel<T>& l = L[lev];
+            int* bad = flags.get() + lev;
             l.dim = G.dim;
             l.W = G.W;
             l.N = G.N;
@@ -2245,9 +2243,7 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                     surf.resize(dia_tiled_size(l.N, 14));
                     up64 = surf.get();
                 }
-                UGX_HIP(hipMemsetAsync(c.flag, 0, sizeof(int), c.stream));
-                disc->template assemble_level_q1<T>(lev, omega, l.Afull.get(), l.A.get(), l.dinv, up64, c.flag);
-                check_diagonal(lev);
+                disc->template assemble_level_q1<T>(lev, omega, l.Afull.get(), l.A.get(), l.dinv, up64, bad);
                 continue;
             }
             DeviceBuffer<double> A64;
@@ -2266,9 +2262,15 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
             }
             // Jacobi: diagInv = 1/(a_ii * (1/omega)) from the FP64 centre diagonal
             DeviceBuffer<double> dinv64(l.N);
-            UGX_HIP(hipMemsetAsync(c.flag, 0, sizeof(int), c.stream));
-            UGX_LAUNCH((dia_jacobi_diag<double, double>(l.N, l.nd, A64.get(), omega, dinv64.get(), c.flag, c.stream)));
-            if (lev == base) {
+            UGX_LAUNCH((dia_jacobi_diag<double, double>(l.N, l.nd, A64.get(), omega, dinv64.get(), bad, c.stream)));
+            if (lev == base && lu_factors_fit((int)l.N, l.nd)) {
+                lu_n = (int)l.N;
+                lu_linvT.resize(l.N * l.N);
+                lu_uinvT.resize(l.N * l.N);
+                lu_perm.resize(l.N);
+                UGX_LAUNCH(lu_factors(lu_n, l.nd, l.off.data(), A64.get(), lu_linvT.get(), lu_uinvT.get(),
+                                      lu_perm.get(), flags.get() + top + 1, c.stream));
+            } else if (lev == base) {
                 std::vector<double> h((size_t)dia_tiled_size(l.N, l.nd));
                 A64.download(h.data(), (int64_t)h.size());
                 lu_n = (int)l.N;
@@ -2304,7 +2306,6 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                     UGX_LAUNCH((convert<double, T>(A64.size(), A64.get(), l.Afull.get(), c.stream)));
                     UGX_LAUNCH((convert<double, T>(l.N, dinv64.get(), l.dinv, c.stream)));
                 }
-                check_diagonal(lev);
                 continue;
             }
             // symmetric Dirichlet-eliminated storage of the level operator
@@ -2329,8 +2330,11 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                 UGX_LAUNCH((convert<double, T>(A64.size(), A64.get(), l.Afull.get(), c.stream)));
                 UGX_LAUNCH((convert<double, T>(l.N, dinv64.get(), l.dinv, c.stream)));
             }
-            check_diagonal(lev);
         }
+        flags.download(found.data(), (int64_t)found.size());
+        if (found[top + 1]) throw UGError("GMG: base level matrix is singular");
+        for (int lev = base + 1; lev <= top; ++lev)
+            if (found[lev]) throw UGError("GMG: Jacobi found a zero diagonal");
         plan_coarse_cycle();
     }
 

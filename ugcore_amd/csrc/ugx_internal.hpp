@@ -189,6 +189,13 @@ int restrict_defect(int dim, int Wc, int Wf, int64_t n_c, const TV* sdf, const u
 // x = U^{-1} L^{-1} P b with row-major triangular inverses; perm[i] = row of b
 template <typename TV>
 int lu_solve(int n, const double* LinvT, const double* UinvT, const int32_t* perm, const TV* b, TV* x, hipStream_t s);
+// what lu_solve applies, from the base operator in tiled DIA form, on the
+// device (lu_factor.hip): m rows, nd diagonals with lattice offsets off (host);
+// *singular is set where a pivot is below 1e-10 and kept otherwise
+constexpr int kLuDeviceMax = 128;
+bool lu_factors_fit(int m, int nd);
+int lu_factors(int m, int nd, const int32_t* off, const double* A, double* linv, double* uinv, int32_t* perm,
+               int* singular, hipStream_t s);
 
 // ---- the V-cycle below the large levels as one kernel (coarse_cycle.hip) ----
 constexpr int kCoarseMaxLevels = 6, kCoarseRows = 2304;
