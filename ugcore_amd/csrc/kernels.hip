@@ -2720,9 +2720,11 @@ template int sell_fill<double>(int64_t, int64_t, const int32_t*, const int32_t*,
 // (fewer than 16 waves a CU). Rows of up to 125 entries: 568 slices 23.5 us with
 // one wave, 14.9 with four, 18.3 with sixteen; 80 slices 13.0 with four and 11.0
 // with sixteen, 12 slices 11.9 and 7.6: sixteen where a CU has at most one slice.
-// Rows of up to 27 entries: 7.5 - 9.2 us with one wave, 4.0 - 5.5 with four.
-static int sell_waves(int64_t nslices, int max_width) {
-    if (nslices >= (int64_t)device_cus() * 16 || max_width <= 8) return 1;
+// Rows of up to 27 entries in a cycle: 7.5 - 9.2 us with one wave, 4.0 - 5.5 with
+// four; a product keeps one wave there, whose two sums are those of the
+// dictionary layout bit for bit.
+static int sell_waves(int64_t nslices, int max_width, int min_width) {
+    if (nslices >= (int64_t)device_cus() * 16 || max_width <= min_width) return 1;
     return max_width > 32 && nslices <= device_cus() ? 16 : 4;
 }
 
@@ -2740,7 +2742,7 @@ int sell_spmv(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, int
               const TM* sval, double alpha, const TV* v1, double beta, const TV* w, TV* dest, int mode,
               const int32_t* rowptr, const int32_t* order, hipStream_t s) {
     if (nrows <= 0) return 0;
-    const int waves = sell_waves((nrows + 63) / 64, max_width);
+    const int waves = sell_waves((nrows + 63) / 64, max_width, 32);
     auto* f = waves == 16  ? &launch_sell_spmv<TM, TV, 16>
               : waves == 4 ? &launch_sell_spmv<TM, TV, 4>
                            : &launch_sell_spmv<TM, TV, 1>;
@@ -2764,7 +2766,7 @@ int sell_cycle(int64_t nrows, const int64_t* slice_ptr, const int32_t* width, in
                const double* sval, const double* w, const int32_t* rowptr, const int32_t* order,
                const SellEpilogue& e, hipStream_t s) {
     if (nrows <= 0) return 0;
-    const int waves = sell_waves((nrows + 63) / 64, max_width);
+    const int waves = sell_waves((nrows + 63) / 64, max_width, 8);
     auto* f = waves == 16 ? &launch_sell_cycle<16> : waves == 4 ? &launch_sell_cycle<4> : &launch_sell_cycle<1>;
     f(nrows, slice_ptr, width, scol, sval, w, rowptr, order, e, s);
     UGX_CHECK_LAUNCH();
