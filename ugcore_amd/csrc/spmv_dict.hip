@@ -295,18 +295,19 @@ __global__ __launch_bounds__(64) void k_dict_values(int64_t nrows, const int32_t
 
 // y = alpha*v1 + beta*A*x (mode 0), or y = beta*A*x on rows with entries
 // (mode 1); one wave per slice, four slices per workgroup.
-// Bound by HBM: 9 bytes per entry and the dictionaries. Two things keep the
-// stream busy: the first kPre entries of every row and the row numbers are
-// requested before the dictionary and x (a chain of three dependent loads and
-// a barrier that the values do not depend on), and consecutive slices run on
-// one XCD, so the x values that neighbouring lattice blocks share are fetched
-// by one L2 instead of eight. One MI355X: the operator of 97^3 tetrahedral rows
-// 41 us without the two, 37 us with them and the partials below; the 257^3 Q1
-// operator runs at the stream's rate either way (990 us).
+// Bound by HBM: 9 bytes per entry and the dictionaries (257^3 Q1 operator 988 us
+// on one MI355X).
 // DOTS (mode 0): also the workgroup's partial sums of (y, u) and (y, y), in
 // part[block] and part[blocks + block]. x may be FP32 (converted as it is
 // staged); dict and order may number the columns and rows differently from
-// the matrix's own numbering (order and x, y then share that numbering).
+// the matrix's own numbering (order and x, y then share that numbering). These
+// are the products of a solver's step on operators that stay in the caches, where
+// latency counts: the first kPre entries of every row and the row numbers are
+// requested before the dictionary and x (a chain of three dependent loads and a
+// barrier that the values do not depend on), and consecutive slices run on one
+// XCD, whose L2 then holds the x values that neighbouring lattice blocks share
+// (97^3 tetrahedral rows 41 us without the two, 37 us with them and the partials;
+// the product at the stream's rate loses by them, 988 -> 995 us).
 template <typename XT, bool DOTS>
 __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslices, const int32_t* __restrict__ width,
                                                    const int32_t* __restrict__ dptr, const int32_t* __restrict__ dict,
@@ -318,18 +319,25 @@ __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslice
                                                    const double* __restrict__ u, double* __restrict__ part) {
     __shared__ double xl[4][256];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t lb = per_xcd ? (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
+    const int64_t lb =
+        DOTS && per_xcd ? (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
     const int64_t t = lb * 4 + wave;
     double* xs = xl[wave];
     const bool live = t < nslices;
-    const int w = live ? width[t] : 0;
-    const dbl2* vp = reinterpret_cast<const dbl2*>(sval + (live ? vptr[t] : 0)) + lane;
-    const uint32_t* ip = sidx + (live ? iptr[t] : 0) + lane;
-    const int32_t r = live ? order[t * 64 + lane] : -1;
+    int w = 0;
+    const dbl2* vp = reinterpret_cast<const dbl2*>(sval) + lane;
+    const uint32_t* ip = sidx + lane;
+    int32_t r = -1;
+    if (DOTS && live) {
+        w = width[t];
+        vp = reinterpret_cast<const dbl2*>(sval + vptr[t]) + lane;
+        ip += iptr[t];
+        r = order[t * 64 + lane];
+    }
     constexpr int kPre = 8;
     uint32_t pw[kPre / 4];
     dbl2 pv[kPre / 2];
-    const bool pre = w >= kPre;   // the same for every lane of the wave
+    const bool pre = DOTS && w >= kPre;   // the same for every lane of the wave
     if (pre) {
 #pragma unroll
         for (int q = 0; q < kPre / 4; ++q) pw[q] = __builtin_nontemporal_load(ip + 64 * q);
@@ -340,12 +348,17 @@ __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslice
         const int32_t d0 = dptr[t], nd = dptr[t + 1] - d0;
         for (int j = lane; j < nd; j += 64) xs[j] = (double)x[dict[d0 + j]];
         if (lane == 0) xs[255] = 0.0;
+        if (!DOTS) w = width[t];
     }
-    const bool mine = r >= 0 && r < nrows;
+    bool mine = r >= 0 && r < nrows;
     double ur = 0.0;
     if (DOTS) ur = mine ? u[r] : 0.0;
     __syncthreads();
-    if (!DOTS && !live) return;
+    if (!DOTS) {
+        if (!live) return;
+        vp = reinterpret_cast<const dbl2*>(sval + vptr[t]) + lane;
+        ip += iptr[t];
+    }
     double s0 = 0.0, s1 = 0.0;
     int k = 0;
     if (pre) {
@@ -401,6 +414,8 @@ __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslice
         }
         return;
     }
+    r = order[t * 64 + lane];
+    mine = r >= 0 && r < nrows;
     if (!mine) return;
     if (mode == 1) {
         if (rowptr[r + 1] > rowptr[r]) y[r] = beta * sum;
@@ -618,10 +633,9 @@ int dict_spmv(int64_t nrows, int64_t nslices, const int32_t* width, const int32_
               const int32_t* order, double alpha, const double* v1, double beta, const double* x, double* y, int mode,
               const int32_t* rowptr, hipStream_t s) {
     if (nslices <= 0) return 0;
-    const int64_t nb = (nslices + 3) / 4, per = nb >= 64 ? (nb + 7) / 8 : 0;
-    hipLaunchKernelGGL((k_dict_spmv<double, false>), dim3((unsigned)dict_spmv_blocks(nslices)), dim3(256), 0, s, nrows,
-                       nslices, width, dptr, dict, vptr, iptr, sval, sidx, order, alpha, v1, beta, x, y, mode, rowptr,
-                       per, (const double*)nullptr, (double*)nullptr);
+    hipLaunchKernelGGL((k_dict_spmv<double, false>), dim3(nblk(nslices, 4)), dim3(256), 0, s, nrows, nslices, width,
+                       dptr, dict, vptr, iptr, sval, sidx, order, alpha, v1, beta, x, y, mode, rowptr, (int64_t)0,
+                       (const double*)nullptr, (double*)nullptr);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
