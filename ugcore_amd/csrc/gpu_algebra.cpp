@@ -2444,7 +2444,14 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         auto& c = context();
         GmgLevel<T>& f = L[lev];
         GmgLevel<T>& cl = L[lev - 1];
-        if (tets) {
+        const bool fuse_sub = std::is_same<T, float>::value && lev == top && sym && mf && nu2 > 0 &&
+                              q1mf_prolong_sub_fits(f.W);
+        if (fuse_sub) {
+            // with the defect update that follows, in one pass
+            if constexpr (std::is_same<T, float>::value)
+                UGX_LAUNCH(q1mf_prolong_sub<T>(f.W, cell_c.get(), cl.sc, cl.acc_deferred ? cl.dinv : nullptr,
+                                               cl.acc_deferred ? cl.sd : nullptr, f.sd, f.sc, c.stream));
+        } else if (tets) {
             UGX_LAUNCH(prolong_add_tet<T>(cl.W, f.W, f.N, cl.sc, disc->level(lev).pcode.get(), f.dir, f.st, f.sc,
                                           c.stream));
         } else if (cl.acc_deferred) {
@@ -2455,7 +2462,7 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         }
         cl.acc_deferred = false;
         if (nu2 == 0) return;
-        UGX_LAUNCH(op_apply_sub(f, f.st, f.sd, f.sd));
+        if (!fuse_sub) UGX_LAUNCH(op_apply_sub(f, f.st, f.sd, f.sd));
         // matrix-free top level of the lattice entry: the last full smoothing
         // step, the deferred correction update, its conversion and (z, r) in
         // one pass (run_lattice then has nothing left to do)

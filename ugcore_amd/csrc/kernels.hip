@@ -1253,13 +1253,6 @@ __device__ __forceinline__ void q1mf_block(const MfMap& m, const T* __restrict__
     }
 }
 
-// the coarse correction the prolongation reads: sc, or (with dinv) the value
-// the coarse level's deferred last post-smoothing update sc + dinv .* sd would
-// store, with the arithmetic of k_jacobi_accumulate
-template <typename TV>
-__device__ __forceinline__ TV coarse_fold(TV sc, TV dinv, TV sd) {
-    return (TV)((double)sc + (double)dinv * (double)sd);
-}
 template <typename T>
 __global__ __launch_bounds__(256) void k_q1mf_jacobi_step(MfMap m, const T* __restrict__ cell,
                                                           const T* __restrict__ dinv, const T* __restrict__ sd_in,

@@ -40,7 +40,11 @@ namespace {
 //         (a = dinv, b = sd, c = sc) without storing sd_out or sc, then
 //         z64 = (double)(sc_new + dinv .* sd_out) with the arithmetic of
 //         k_jacobi_convert_dot (d64 = r)
-// out0 may alias c (MODE 1, 2): every row is read and then written by the same
+// MODE 6: the coarse grid correction and the defect update after it: staged
+//         t = P c_coarse (a = the coarse correction; with b, c2 its last update
+//         a + b .* c2 folded in), d_out = d_in - A t, sc += t: c = d_in,
+//         out0 = d_out, out1 = sc (k_q1mf_march only)
+// out0 may alias c (MODE 1, 2, 6): every row is read and then written by the same
 // thread. The rows' own inputs and outputs are nontemporal: they leave the L2
 // to the values that neighbouring rows share.
 template <typename T>
@@ -55,6 +59,7 @@ struct Q1Args {
     double* partial;
     const double* d64;
     double* z64;
+    const T* c2;
 };
 
 template <typename T>
@@ -95,6 +100,9 @@ __device__ __forceinline__ void load_row(const Q1Args<T>& q, int64_t i, bool ok,
         in.v = ldn(q.out1 + i);   // sc
     } else if (MODE == 1) {
         in.u = ldn(q.c + i);
+    } else if (MODE == 6) {
+        in.u = ldn(q.c + i);
+        in.v = ldn(q.out1 + i);
     } else if (MODE == 2) {
         in.u = q.alpha != 0.0 ? ldn(q.c + i) : (T)0;
     } else if (MODE == 3) {
@@ -110,7 +118,7 @@ __device__ __forceinline__ void load_row(const Q1Args<T>& q, int64_t i, bool ok,
 }
 template <typename T, int MODE>
 __device__ __forceinline__ void store_row(const Q1Args<T>& q, int64_t i, const RowIn<T>& in, T xi, T s, double& dot) {
-    if (MODE == 0) {
+    if (MODE == 0 || MODE == 6) {
         stn(in.u - s, q.out0 + i);
         stn(in.v + xi, q.out1 + i);
     } else if (MODE == 3 || MODE == 4) {
@@ -287,19 +295,69 @@ __global__ __launch_bounds__(256) void k_q1mf_march(MarchMap m, Q1Args<T> q) {
         // line j0 - 1 + that); the lines' last column by the first NL threads
         const int sy = j0 - 1 + tg;
         T va[SX], vb[SX], vc[SC], xa = (T)0, xb = (T)0;
+        // MODE 6: the coarse values that the thread's staged points lie between
+        // (coarse lines cl0 + j, columns tx/2 and, for odd tx, tx/2 + 1), one new
+        // coarse plane for every second fine one: raw parts in flight, and
+        // the sums over the columns on the coarse planes below and above
+        constexpr int NQ = MODE == 6 ? NL / 2 + 1 : 1;
+        constexpr int Wc = NX / 2 + 1;
+        T ra[NQ][2], rb[NQ][2], rc[NQ][2], xc = (T)0;
+        double lo[NQ], hi[NQ];
+        int fetched = -1;   // MODE 6: the plane in flight
+        const int cl0 = (j0 >> 1) - 1, cx = tx >> 1, ox = tx & 1;
+        auto fetch_coarse = [&](int cp) {
+#pragma unroll
+            for (int j = 0; j < NQ; ++j)
+#pragma unroll
+                for (int o = 0; o < 2; ++o) {
+                    const int cy = cl0 + j;
+                    const bool in = cy >= 0 && cy < Wc && o <= ox;
+                    const int64_t i = ((int64_t)cp * Wc + cy) * Wc + cx + o;
+                    ra[j][o] = in ? q.a[i] : (T)0;
+                    rb[j][o] = in && q.b ? q.b[i] : (T)0;
+                    rc[j][o] = in && q.b ? q.c2[i] : (T)0;
+                }
+        };
+        auto fold_coarse = [&]() {
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) {
+                lo[j] = hi[j];
+                const T v0 = q.b ? coarse_fold<T>(ra[j][0], rb[j][0], rc[j][0]) : ra[j][0];
+                const T v1 = q.b ? coarse_fold<T>(ra[j][1], rb[j][1], rc[j][1]) : ra[j][1];
+                hi[j] = (double)v0 + (double)v1;
+            }
+        };
+        if constexpr (MODE == 6) {
+            fetch_coarse((k0 > 0 ? k0 - 1 : 0) >> 1);
+            fold_coarse();
+            fold_coarse();   // both planes: an even plane takes the upper one over, an odd one replaces it
+        }
         auto fetch = [&](int p, int cz) {
             const bool pin = p >= 0 && p < W, cin = cz >= 0 && cz < NX;
             const int64_t base = (int64_t)p * W2;
+            if constexpr (MODE == 6) {
+                fetched = pin ? p : -1;
+                if (pin && (p & 1)) fetch_coarse((p >> 1) + 1);
+                xa = xb = xc = (T)0;
+                const int ye = j0 - 1 + tid;
+                if (pin && !(p & 1) && tid < NL && ye >= 0 && ye < W && !(ye & 1)) {
+                    const int64_t i = ((int64_t)(p >> 1) * Wc + (ye >> 1)) * Wc + Wc - 1;
+                    xa = q.a[i];
+                    xb = q.b ? q.b[i] : (T)0;
+                    xc = q.b ? q.c2[i] : (T)0;
+                }
+            } else {
 #pragma unroll
-            for (int u = 0; u < SX; ++u) {
-                const int y = sy + u * G;
-                va[u] = vb[u] = (T)0;
-                if (pin && y >= 0 && y < W && tg + u * G < NL)
-                    raw_staged<T, MODE>(q, base + (int64_t)y * W + tx, va[u], vb[u]);
+                for (int u = 0; u < SX; ++u) {
+                    const int y = sy + u * G;
+                    va[u] = vb[u] = (T)0;
+                    if (pin && y >= 0 && y < W && tg + u * G < NL)
+                        raw_staged<T, MODE>(q, base + (int64_t)y * W + tx, va[u], vb[u]);
+                }
+                xa = xb = (T)0;
+                const int ye = j0 - 1 + tid;
+                if (pin && tid < NL && ye >= 0 && ye < W) raw_staged<T, MODE>(q, base + (int64_t)ye * W + NX, xa, xb);
             }
-            xa = xb = (T)0;
-            const int ye = j0 - 1 + tid;
-            if (pin && tid < NL && ye >= 0 && ye < W) raw_staged<T, MODE>(q, base + (int64_t)ye * W + NX, xa, xb);
 #pragma unroll
             for (int u = 0; u < SC; ++u) {
                 const int y = sy + u * G;
@@ -307,10 +365,39 @@ __global__ __launch_bounds__(256) void k_q1mf_march(MarchMap m, Q1Args<T> q) {
             }
         };
         auto put = [&](int b) {
+            if constexpr (MODE == 6) {
+                // plane `fetched`: sums over the planes, then over the lines;
+                // the weight is 2^-(odd coordinates), boundary points are zero
+                // unless they copy a coarse point
+                const int oz = fetched & 1;
+                const bool pin = fetched >= 0, pb = fetched == 0 || fetched == W - 1;
+                if (pin && oz) fold_coarse();
+                if (pin && !oz)
 #pragma unroll
-            for (int u = 0; u < SX; ++u)
-                if (tg + u * G < NL) xs[b][(tg + u * G) * W + tx] = combine<T, MODE>(va[u], vb[u], bcg);
-            if (tid < NL) xs[b][tid * W + NX] = combine<T, MODE>(xa, xb, bcg);
+                    for (int j = 0; j < NQ; ++j) lo[j] = hi[j];
+#pragma unroll
+                for (int u = 0; u < SX; ++u) {
+                    const int m = tg + u * G, y = j0 - 1 + m;   // y is odd where m is even
+                    // between the coarse lines m / 2 and m / 2 + 1 (m even), on
+                    // line (m + 1) / 2 (m odd)
+                    const bool oy = !(m & 1);
+                    auto at = [&](int jj) { return jj < NQ ? (oz ? lo[jj] + hi[jj] : lo[jj]) : 0.0; };
+                    double sum;
+                    if constexpr (G == 1) sum = (u & 1) ? at((u + 1) / 2) : at(u / 2) + at(u / 2 + 1);
+                    else sum = oy ? at(u) + at(u + 1) : at(u + 1);
+                    const int nodd = ox + (oy ? 1 : 0) + oz;
+                    const double w = nodd == 0 ? 1.0 : nodd == 1 ? 0.5 : nodd == 2 ? 0.25 : 0.125;
+                    const bool bnd = tx == 0 || y == 0 || y == W - 1 || pb;
+                    const bool zero = !pin || y < 0 || y >= W || (bnd && nodd != 0);
+                    if (m < NL) xs[b][m * W + tx] = zero ? (T)0 : (T)(w * sum);
+                }
+                if (tid < NL) xs[b][tid * W + NX] = q.b ? coarse_fold<T>(xa, xb, xc) : xa;
+            } else {
+#pragma unroll
+                for (int u = 0; u < SX; ++u)
+                    if (tg + u * G < NL) xs[b][(tg + u * G) * W + tx] = combine<T, MODE>(va[u], vb[u], bcg);
+                if (tid < NL) xs[b][tid * W + NX] = combine<T, MODE>(xa, xb, bcg);
+            }
 #pragma unroll
             for (int u = 0; u < SC; ++u)
                 if (tg + u * G < NC) cs[b][(tg + u * G) * NX + tx] = vc[u];
@@ -443,7 +530,7 @@ bool q1mf_fused_fits(int W) { return W <= kDirectMaxW || W == 129 || W == 257; }
 template <typename T>
 int q1mf_jacobi_step(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s) {
     if (!q1mf_fused_fits(W)) return q1mf_planes_jacobi_step<T>(W, cell, dinv, sd_in, sd_out, sc, s);
-    return q1mf_launch<T, 0>(W, Q1Args<T>{cell, dinv, sd_in, nullptr, sd_out, sc, 0.0, 0.0, nullptr, nullptr, nullptr},
+    return q1mf_launch<T, 0>(W, Q1Args<T>{cell, dinv, sd_in, nullptr, sd_out, sc, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr},
                              s);
 }
 template int q1mf_jacobi_step<float>(int, const float*, const float*, const float*, float*, float*, hipStream_t);
@@ -451,7 +538,7 @@ template int q1mf_jacobi_step<double>(int, const double*, const double*, const d
 
 template <typename T>
 int q1mf_jacobi_first(int W, const T* cell, const T* dinv, const double* d64, T* sd_out, T* sc, hipStream_t s) {
-    return q1mf_launch<T, 3>(W, Q1Args<T>{cell, dinv, nullptr, nullptr, sd_out, sc, 0.0, 0.0, nullptr, d64, nullptr},
+    return q1mf_launch<T, 3>(W, Q1Args<T>{cell, dinv, nullptr, nullptr, sd_out, sc, 0.0, 0.0, nullptr, d64, nullptr, nullptr},
                              s);
 }
 template int q1mf_jacobi_first<float>(int, const float*, const float*, const double*, float*, float*, hipStream_t);
@@ -459,7 +546,7 @@ template int q1mf_jacobi_first<double>(int, const double*, const double*, const 
 
 template <typename T>
 int q1mf_jacobi_first_t(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s) {
-    return q1mf_launch<T, 4>(W, Q1Args<T>{cell, dinv, sd_in, nullptr, sd_out, sc, 0.0, 0.0, nullptr, nullptr, nullptr},
+    return q1mf_launch<T, 4>(W, Q1Args<T>{cell, dinv, sd_in, nullptr, sd_out, sc, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr},
                              s);
 }
 template int q1mf_jacobi_first_t<float>(int, const float*, const float*, const float*, float*, float*, hipStream_t);
@@ -467,7 +554,7 @@ template int q1mf_jacobi_first_t<float>(int, const float*, const float*, const f
 template <typename T>
 int q1mf_apply_sub(int W, const T* cell, const T* x, const T* d_in, T* d_out, hipStream_t s) {
     if (!q1mf_fused_fits(W)) return q1mf_planes_apply_sub<T>(W, cell, x, d_in, d_out, s);
-    return q1mf_launch<T, 1>(W, Q1Args<T>{cell, x, nullptr, d_in, d_out, nullptr, 0.0, 0.0, nullptr, nullptr, nullptr},
+    return q1mf_launch<T, 1>(W, Q1Args<T>{cell, x, nullptr, d_in, d_out, nullptr, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr},
                              s);
 }
 template int q1mf_apply_sub<float>(int, const float*, const float*, const float*, float*, hipStream_t);
@@ -477,7 +564,7 @@ template <typename T>
 int q1mf_jacobi_last(int W, const T* cell, const T* dinv, const T* sd_in, const T* sc, double* z, const double* r,
                      hipStream_t s, double* dot_partial, int* n_partial) {
     if (dot_partial && !n_partial) return -1;
-    return q1mf_launch<T, 7>(W, Q1Args<T>{cell, dinv, sd_in, sc, nullptr, nullptr, 0.0, 0.0, dot_partial, r, z}, s,
+    return q1mf_launch<T, 7>(W, Q1Args<T>{cell, dinv, sd_in, sc, nullptr, nullptr, 0.0, 0.0, dot_partial, r, z, nullptr}, s,
                              n_partial);
 }
 template int q1mf_jacobi_last<float>(int, const float*, const float*, const float*, const float*, double*,
@@ -493,7 +580,7 @@ int q1mf_axpy(int W, const T* cell, double alpha, const T* v, double beta, const
         return q1mf_planes_axpy<T>(W, cell, alpha, v, beta, x, y, s);
     }
     if (dot_partial && !n_partial) return -1;
-    return q1mf_launch<T, 2>(W, Q1Args<T>{cell, x, nullptr, v, y, nullptr, alpha, beta, dot_partial, nullptr, nullptr},
+    return q1mf_launch<T, 2>(W, Q1Args<T>{cell, x, nullptr, v, y, nullptr, alpha, beta, dot_partial, nullptr, nullptr, nullptr},
                              s, n_partial);
 }
 template int q1mf_axpy<double>(int, const double*, double, const double*, double, const double*, double*, hipStream_t,
@@ -504,11 +591,38 @@ template <typename T>
 int q1mf_direction_axpy(int W, const T* cell, const T* p_old, const T* z, const double* beta_dev, T* p_new, T* y,
                         hipStream_t s, double* dot_partial, int* n_partial) {
     if (p_new == p_old || !dot_partial || !n_partial) return -1;
-    return q1mf_launch<T, 5>(W, Q1Args<T>{cell, p_old, z, nullptr, y, p_new, 0.0, 1.0, dot_partial, beta_dev, nullptr},
+    return q1mf_launch<T, 5>(W, Q1Args<T>{cell, p_old, z, nullptr, y, p_new, 0.0, 1.0, dot_partial, beta_dev, nullptr, nullptr},
                              s, n_partial);
 }
 template int q1mf_direction_axpy<double>(int, const double*, const double*, const double*, const double*, double*,
                                          double*, hipStream_t, double*, int*);
+
+// t = P c (the coarse correction, with its last update c += dinv_c .* sd_c
+// folded in where given), d -= A t, sc += t on the marching widths in FP32: the
+// prolongation's separate pass wrote t and read it back. One MI355X, 129^3 ->
+// 257^3: 72 + 73 us in two passes, 116 in this one. FP64 keeps two: the values
+// around a column and their sums take the registers of a resident workgroup
+// (65^3 -> 129^3 38.6 us in two passes, 38.1 in one).
+bool q1mf_prolong_sub_fits(int W) { return W == 129 || W == 257; }
+template <typename T>
+int q1mf_prolong_sub(int W, const T* cell, const T* c_coarse, const T* dinv_c, const T* sd_c, T* d, T* sc,
+                     hipStream_t s) {
+    if ((dinv_c == nullptr) != (sd_c == nullptr)) return -1;
+    MarchMap m{};
+    Q1Args<T> q{cell, c_coarse, dinv_c, d, d, sc, 0.0, 0.0, nullptr, nullptr, nullptr, sd_c};
+    if (W == 129) {
+        const int64_t grid = march_grid<7>(reinterpret_cast<const void*>(&k_q1mf_march<T, 6, 7>), m);
+        hipLaunchKernelGGL((k_q1mf_march<T, 6, 7>), dim3((unsigned)grid), dim3(256), 0, s, m, q);
+    } else if (W == 257) {
+        const int64_t grid = march_grid<8>(reinterpret_cast<const void*>(&k_q1mf_march<T, 6, 8>), m);
+        hipLaunchKernelGGL((k_q1mf_march<T, 6, 8>), dim3((unsigned)grid), dim3(256), 0, s, m, q);
+    } else {
+        return -1;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+template int q1mf_prolong_sub<float>(int, const float*, const float*, const float*, const float*, float*, float*,
+                                     hipStream_t);
 
 // asks the runtime for the residency of the marching kernels at this width, so
 // that no query happens inside a captured cycle
@@ -519,6 +633,11 @@ int q1mf_prepare(int W) {
     q1mf_grid<float, 3>(W, m);
     q1mf_grid<float, 4>(W, m);
     q1mf_grid<float, 7>(W, m);
+    if (W == 129) {
+        march_grid<7>(reinterpret_cast<const void*>(&k_q1mf_march<float, 6, 7>), m);
+    } else if (W == 257) {
+        march_grid<8>(reinterpret_cast<const void*>(&k_q1mf_march<float, 6, 8>), m);
+    }
     q1mf_grid<double, 0>(W, m);
     q1mf_grid<double, 1>(W, m);
     q1mf_grid<double, 2>(W, m);

@@ -95,6 +95,16 @@ int q1mf_prepare(int W);
 // whether q1mf_kernels.hip has a schedule for this lattice width: then every
 // function below applies, otherwise only q1mf_jacobi_step, q1mf_apply_sub and
 // q1mf_axpy without partial sums (the plane-by-plane kernels)
+// the coarse level's deferred last post-smoothing update sc + dinv .* sd would
+// store, with the arithmetic of k_jacobi_accumulate
+template <typename TV>
+__host__ __device__ inline TV coarse_fold(TV sc, TV dinv, TV sd) {
+    return (TV)((double)sc + (double)dinv * (double)sd);
+}
+bool q1mf_prolong_sub_fits(int W);
+template <typename T>
+int q1mf_prolong_sub(int W, const T* cell, const T* c_coarse, const T* dinv_c, const T* sd_c, T* d, T* sc,
+                     hipStream_t s);
 bool q1mf_fused_fits(int W);
 template <typename T>
 int q1mf_planes_jacobi_step(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s);
