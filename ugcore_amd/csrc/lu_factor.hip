@@ -51,13 +51,13 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // A chain of 2 m steps, each bound by its barriers, the pivot search and the
 // issue of its instructions, so few waves (four, one a SIMD; with sixteen, which
 // repeat the search, 490 us) and blocks of 16 columns unrolled, which makes a
-// thread's register for a column a constant. 125 rows: 340 us on one MI355X; the
+// thread's register for a column a constant. 125 rows: 270 us on one MI355X; the
 // host took 650 us, with the device idle and a copy in each direction.
 __global__ __launch_bounds__(256) void k_lu_factors(int m, int nd, BaseOffsets off, const double* __restrict__ A,
                                                     double* __restrict__ linv, double* __restrict__ uinv,
                                                     int32_t* __restrict__ perm, int* __restrict__ singular) {
     extern __shared__ double dense[];   // m x m
-    __shared__ double col[2][128], row[2][128], mul[128];
+    __shared__ double col[2][128], row[2][128], mul[128], diag[128], inv[128];
     __shared__ int32_t at[128], ord[128];   // row at a position, position of a row
     const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15, lane = tid & 63;
     for (int e = tid; e < m * m; e += 256) dense[e] = 0.0;
@@ -123,7 +123,10 @@ __global__ __launch_bounds__(256) void k_lu_factors(int m, int nd, BaseOffsets o
             // the row at position k and the pivot change places
             p0 = lane == p ? k : p0 == k ? q : p0;
             p1 = lane + 64 == p ? k : p1 == k ? q : p1;
-            const double piv = col[0][p];
+            const long long pb = __double_as_longlong(second ? c1 : c0);
+            const double piv = __longlong_as_double(
+                (long long)(uint32_t)__builtin_amdgcn_readlane((int)pb, src) |
+                (long long)__builtin_amdgcn_readlane((int)(pb >> 32), src) << 32);
             bad = bad || fabs(piv) < 1e-10;
             if (tid < 64) {
                 mul[lane] = p0 > k ? c0 / piv : 0.0;
@@ -142,16 +145,15 @@ __global__ __launch_bounds__(256) void k_lu_factors(int m, int nd, BaseOffsets o
             double u[kR];
 #pragma unroll
             for (int b = 0; b < kR; ++b) u[b] = row[0][tj + kT * b];
+            // rows already taken have l = 0 and stay; so does column k of a row
+            // with l = 0, which is zero there or taken
 #pragma unroll
             for (int a = 0; a < kR; ++a) {
                 const double l = mul[ti + kT * a];
-                if (ord[ti + kT * a] > k) {   // not yet taken
+                const double keep = r[a][bk];
 #pragma unroll
-                    for (int b = 0; b < kR; ++b) {
-                        const double t = fma(-l, u[b], r[a][b]);
-                        r[a][b] = b == bk && tj == jk ? -l : t;
-                    }
-                }
+                for (int b = 0; b < kR; ++b) r[a][b] = fma(-l, u[b], r[a][b]);
+                if (tj == jk) r[a][bk] = l != 0.0 ? -l : keep;
             }
         }
     };
@@ -167,6 +169,20 @@ __global__ __launch_bounds__(256) void k_lu_factors(int m, int nd, BaseOffsets o
         if (tid == 0) *singular = 1;
         return;
     }
+    // the diagonal entries and their inverses; a row's position (beyond all for
+    // none)
+    int pos[kR];
+#pragma unroll
+    for (int a = 0; a < kR; ++a) {
+        const int i = ti + kT * a;
+        pos[a] = i < m ? ord[i] : 255;
+#pragma unroll
+        for (int b = 0; b < kR; ++b)
+            if (i < m && tj + kT * b == pos[a]) {
+                diag[pos[a]] = r[a][b];
+                inv[pos[a]] = 1.0 / r[a][b];
+            }
+    }
     __syncthreads();
     auto backward = [&](auto block) __attribute__((always_inline)) {
         constexpr int bk = decltype(block)::value;
@@ -175,18 +191,22 @@ __global__ __launch_bounds__(256) void k_lu_factors(int m, int nd, BaseOffsets o
             const int k = kT * bk + jk, s = jk & 1;
             if (k >= m) continue;
             const int p = __builtin_amdgcn_readfirstlane(at[k]);
+            // the rows above, zero for the others
             if (tj == jk)
 #pragma unroll
-                for (int a = 0; a < kR; ++a) col[s][ti + kT * a] = r[a][bk];
+                for (int a = 0; a < kR; ++a) col[s][ti + kT * a] = pos[a] < k ? r[a][bk] : 0.0;
 #pragma unroll
             for (int a = 0; a < kR; ++a)
                 if ((p >> 4) == a && ti == (p & 15)) {
-                    const double u = __shfl(r[a][bk], (lane & 48) + jk, 64);
+                    // divided by the diagonal entry: its inverse and one correction
+                    const double u = diag[k], v = inv[k];
 #pragma unroll
                     for (int b = bk; b < kR; ++b) {
                         const int c = tj + kT * b;
-                        if (c >= k) r[a][b] = (c == k ? 1.0 : r[a][b]) / u;
-                        row[s][c] = r[a][b];
+                        const double t = r[a][b] * v;
+                        const double x = c == k ? v : fma(fma(-t, u, r[a][b]), v, t);
+                        r[a][b] = c >= k ? x : r[a][b];
+                        row[s][c] = c >= k ? x : 0.0;
                     }
                 }
             __syncthreads();
@@ -195,16 +215,10 @@ __global__ __launch_bounds__(256) void k_lu_factors(int m, int nd, BaseOffsets o
             for (int b = bk; b < kR; ++b) x[b] = row[s][tj + kT * b];
 #pragma unroll
             for (int a = 0; a < kR; ++a) {
-                const int o = ord[ti + kT * a];
-                const double u = col[s][ti + kT * a];
-                if (o >= 0 && o < k) {
+                const double u = col[s][ti + kT * a], keep = r[a][bk];
 #pragma unroll
-                    for (int b = bk; b < kR; ++b) {
-                        const int c = tj + kT * b;
-                        const double t = c == k ? -(u * x[b]) : fma(-u, x[b], r[a][b]);
-                        r[a][b] = c >= k ? t : r[a][b];
-                    }
-                }
+                for (int b = bk; b < kR; ++b) r[a][b] = fma(-u, x[b], r[a][b]);
+                if (tj == jk) r[a][bk] = u != 0.0 ? -(u * x[bk]) : keep;
             }
         }
     };
@@ -222,7 +236,7 @@ __global__ __launch_bounds__(256) void k_lu_factors(int m, int nd, BaseOffsets o
         for (int b = 0; b < kR; ++b) {
             const int i = ti + kT * a, c = tj + kT * b;
             if (i >= m || c >= m) continue;
-            const int o = ord[i];
+            const int o = pos[a];
             linv[o * m + c] = c < o ? r[a][b] : c == o ? 1.0 : 0.0;
             uinv[o * m + c] = c >= o ? r[a][b] : 0.0;
         }
