@@ -1,15 +1,16 @@
-// Q2 (triquadratic Lagrange) hexahedron element matrices on gfx950: one
-// element per wavefront, the B^T D B contraction on the FP64 matrix cores.
+// Q2 (triquadratic Lagrange) hexahedron element matrices on gfx950, two
+// elements per wavefront by sum factorisation.
 //
 // Per element (corners X in the reference hexahedron order, coefficient k,
 // constant source f): Ke[a][b] = sum_q w_q |det J_q| k grad phi_a . grad phi_b
 // and fe[a] = sum_q w_q |det J_q| f phi_a over the 3x3x3 Gauss-Legendre
-// points, with the trilinear geometry of the 8 corners. Written as
-// Ke = B^T C B with B (81 x 27) the physical gradients, one row per point and
-// component, and C = diag(w_q |det J_q| k): each lane forms the two entries
-// of B (padded to 84 x 32) it feeds to each v_mfma_f64_16x16x4f64 step in
-// registers, and the wave accumulates three 16 x 16 tiles of the symmetric Ke
-// over 21 steps of 4 rows (only the Jacobians sit in LDS).
+// points, with the trilinear geometry of the 8 corners. With the symmetric 3x3
+// G_q = w_q |det J_q| k J_q^-1 J_q^-T and phi_a = l_i(x) l_j(y) l_m(z),
+//   Ke = sum_{d,e} sum_qz sum_qy sum_qx G_q[d][e] (d_d phi_a) (d_e phi_b)
+// is summed one direction at a time: 1.5 k multiply-adds for the sums over x
+// (54 lanes), 7.7 k for those over y and z (45 lanes: one per unordered pair of
+// (i, j), nine entries each), where the contraction over all points at once is
+// 64 k on the matrix cores.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,23 +21,12 @@
 namespace ugamd {
 namespace {
 
-constexpr int kQ2Rows = 84;   // 27 points x 3 components, padded to a multiple of 4
-
 __device__ __forceinline__ double q2_gauss(int i) {
     // 3-point Gauss-Legendre on [0, 1]: 1/2 -+ sqrt(3/5)/2
     return i == 0 ? 0.11270166537925831 : i == 1 ? 0.5 : 0.8872983346207417;
 }
 __device__ __forceinline__ double q2_gauss_w(int i) { return i == 1 ? 8.0 / 18.0 : 5.0 / 18.0; }
 
-typedef double q2d4 __attribute__((ext_vector_type(4)));
-
-// grad_xi phi_a and phi_a at Gauss point q (q = qx + 3 qy + 9 qz), evaluated
-// at compile time from the 1D Lagrange polynomials of the nodes 0, 1/2, 1 and
-// the local order
-struct Q2RefGrad {
-    double g[27][27][3];
-    double phi[27][27];   // phi_a at point q
-};
 // Local shape order of LagrangeLSFS<ReferenceHexahedron, 2> (lagrange.cpp:
 // 236-253, lagrange.h:2106-2190): multi-indices of the vertices (2 x corner),
 // the edge midpoints of edges (0,1) (1,2) (2,3) (3,0) (0,4) (1,5) (2,6) (3,7)
@@ -51,128 +41,299 @@ constexpr double q2c_l(int i, double x) {
     return i == 0 ? (1.0 - x) * (1.0 - 2.0 * x) : i == 1 ? 4.0 * x * (1.0 - x) : x * (2.0 * x - 1.0);
 }
 constexpr double q2c_dl(int i, double x) { return i == 0 ? 4.0 * x - 3.0 : i == 1 ? 4.0 - 8.0 * x : 4.0 * x - 1.0; }
-constexpr Q2RefGrad q2_ref_grad() {
-    Q2RefGrad t{};
-    for (int q = 0; q < 27; ++q)
-        for (int a = 0; a < 27; ++a) {
-            const double x0 = q2c_x(q % 3), x1 = q2c_x((q / 3) % 3), x2 = q2c_x(q / 9);
-            const int m0 = kQ2Mi[a][0], m1 = kQ2Mi[a][1], m2 = kQ2Mi[a][2];
-            const double l0 = q2c_l(m0, x0), l1 = q2c_l(m1, x1), l2 = q2c_l(m2, x2);
-            t.g[q][a][0] = q2c_dl(m0, x0) * l1 * l2;
-            t.g[q][a][1] = l0 * q2c_dl(m1, x1) * l2;
-            t.g[q][a][2] = l0 * l1 * q2c_dl(m2, x2);
-            t.phi[q][a] = l0 * l1 * l2;
+// the 1D polynomials and their derivatives at the Gauss points, and the local
+// number of the multi-index i + 3 j + 9 m
+struct Q2Basis {
+    double l[3][3], d[3][3];   // [polynomial][point]
+    int8_t num[27];
+};
+constexpr Q2Basis q2_basis() {
+    Q2Basis t{};
+    for (int i = 0; i < 3; ++i)
+        for (int q = 0; q < 3; ++q) {
+            t.l[i][q] = q2c_l(i, q2c_x(q));
+            t.d[i][q] = q2c_dl(i, q2c_x(q));
         }
+    for (int a = 0; a < 27; ++a) t.num[kQ2Mi[a][0] + 3 * kQ2Mi[a][1] + 9 * kQ2Mi[a][2]] = (int8_t)a;
     return t;
 }
-__constant__ Q2RefGrad kQ2Grad = q2_ref_grad();
+__constant__ Q2Basis kQ2Basis = q2_basis();
 
-constexpr int kQ2Waves = 8;   // elements (wavefronts) per workgroup
+constexpr int kQ2Waves = 4;   // wavefronts per workgroup, two elements each
 
-// the reference gradient and shape tables copied into the workgroup's LDS
-// (their per-lane reads in the matrix steps then cost an LDS access instead
-// of a cached global one); visible after the element routine's first barrier
-__device__ __forceinline__ void q2_stage_table(Q2RefGrad& tab) {
-    const double* src = reinterpret_cast<const double*>(&kQ2Grad);
-    double* dst = reinterpret_cast<double*>(&tab);
-    for (int i = threadIdx.x; i < (int)(sizeof(Q2RefGrad) / sizeof(double)); i += blockDim.x) dst[i] = src[i];
+// a wavefront's scratch
+struct Q2Scratch {
+    double X[2][24];       // corners of the two elements
+    double G[2][6][27];    // xx, yy, zz, xy, xz, yz at point qx + 3 qy + 9 qz
+    double fw[2][27];      // w_q |det J_q| f
+    double K[729];         // sums over x, then the element matrix
+};
+// LDS written by some lanes of a wavefront is read by others: in order, once
+// the compiler keeps it so
+__device__ __forceinline__ void q2_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// The element computation of one wavefront (lane l): corners from src.corner(l)
-// for l < 24 (valid elements) and the coefficient src.k(q) at Gauss point q
-// (x fastest), then sink.ke(i, j, v) for the 729
-// entries and sink.fe(a, v) for the 27 load entries. Every wave of the
-// workgroup calls it once (it holds two barriers); invalid waves work on the
-// unit cube and emit nothing.
-template <class Src, class Sink>
-__device__ __forceinline__ void q2_element_wave(int l, bool valid, const Src& src, Sink& sink, double f_const,
-                                                double* Xs, double (*Jis)[9], double* cs, double* fw, bool want_fe,
-                                                const Q2RefGrad& tab) {
-    if (l < 24) {
-        const int c = l / 3, d = l - 3 * c;
-        const int bit = d == 0 ? (c == 1 || c == 2 || c == 5 || c == 6) : d == 1 ? (c == 2 || c == 3 || c == 6 || c == 7)
-                                                                         : (c >= 4);
-        Xs[l] = valid ? src.corner(l) : (double)bit;
-    }
-    if (l == 27) cs[27] = 0.0;   // the padding rows 81..83 of B
-    __syncthreads();
-    // 1. Jacobian of the trilinear map at point q = lane (x fastest)
-    if (l < 27) {
-        const int qx = l % 3, qy = (l / 3) % 3, qz = l / 9;
-        const double xi[3] = {q2_gauss(qx), q2_gauss(qy), q2_gauss(qz)};
-        double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-        for (int a = 0; a < 8; ++a) {
-            const int cx = (a == 1 || a == 2 || a == 5 || a == 6), cy = (a == 2 || a == 3 || a == 6 || a == 7),
-                      cz = a >= 4;
-            const double fx = cx ? xi[0] : 1.0 - xi[0], fy = cy ? xi[1] : 1.0 - xi[1], fz = cz ? xi[2] : 1.0 - xi[2];
-            const double d[3] = {(cx ? 1.0 : -1.0) * fy * fz, fx * (cy ? 1.0 : -1.0) * fz, fx * fy * (cz ? 1.0 : -1.0)};
-            for (int r = 0; r < 3; ++r)
-                for (int c = 0; c < 3; ++c) J[r][c] += Xs[3 * a + r] * d[c];
-        }
-        const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
-                           J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
-                           J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
-        const double id = 1.0 / det;
-        double* ji = Jis[l];
-        ji[0] = (J[1][1] * J[2][2] - J[1][2] * J[2][1]) * id;
-        ji[1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-        ji[2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-        ji[3] = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) * id;
-        ji[4] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-        ji[5] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-        ji[6] = (J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id;
-        ji[7] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-        ji[8] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-        const double wd = q2_gauss_w(qx) * q2_gauss_w(qy) * q2_gauss_w(qz) * fabs(det);
-        cs[l] = wd * (valid ? src.k(l) : 1.0);
-        fw[l] = wd * f_const;
+// products of two 1D factors at the three points, for the nine pairs of
+// polynomials: first derivative on neither, the first, both (x), and all four (y)
+struct Q2Tables {
+    double x[3][9][3];
+    double y[9][12];   // ll, l d, d l, dd
+    double l[3][3];
+    int mi[27];        // multi-indices of the local shapes, two bits a direction
+};
+__device__ __forceinline__ void q2_fill_tables(Q2Tables& t) {
+    for (int e = threadIdx.x; e < 27; e += blockDim.x) {
+        const int p = e / 3, q = e - 3 * p;
+        const double l1 = kQ2Basis.l[p / 3][q], l2 = kQ2Basis.l[p % 3][q];
+        const double d1 = kQ2Basis.d[p / 3][q], d2 = kQ2Basis.d[p % 3][q];
+        t.x[0][p][q] = t.y[p][q] = l1 * l2;
+        t.y[p][3 + q] = l1 * d2;
+        t.x[1][p][q] = t.y[p][6 + q] = d1 * l2;
+        t.x[2][p][q] = t.y[p][9 + q] = d1 * d2;
+        if (p < 3) t.l[p][q] = kQ2Basis.l[p][q];
+        t.mi[e] = kQ2Mi[e][0] | kQ2Mi[e][1] << 2 | kQ2Mi[e][2] << 4;
     }
     __syncthreads();
-    // load vector: fe[a] = sum_q w_q |det J_q| f phi_a(xi_q)
-    if (want_fe && valid && l < 27) {
-        double s = 0.0;
-        for (int q = 0; q < 27; ++q) s += fw[q] * tab.phi[q][l];
-        sink.fe(l, s);
-    }
-    // 2. Ke = (C B)^T B in the 16 x 16 tiles (0,0), (0,1), (1,1); (1,0) is the
-    //    transpose of (0,1). Step kk covers the rows k = 4 kk .. 4 kk + 3 of B
-    //    (point k / 3, component k % 3; rows 81..83 are zero): lane
-    //    l = 16 lk + li forms B[4 kk + lk][a] = (J_q^-T grad_xi phi_a(xi_q))_(k % 3)
-    //    for the shapes a = li and 16 + li (zero beyond 26) and supplies them
-    //    as A[li][lk] (scaled by C) and B[lk][li] of the 16x4 / 4x16 step.
-    //    Accumulator element v of lane l is row l / 16 + 4 v, column l % 16 of
-    //    the tile (the f64 layout, measured on gfx950).
-    const int li = l & 15, lk = l >> 4;
-    const int a1 = 16 + li < 27 ? 16 + li : 26;
-    const bool has1 = 16 + li < 27;
-    q2d4 acc00 = {0.0, 0.0, 0.0, 0.0}, acc01 = acc00, acc11 = acc00;
-    for (int kk = 0; kk < kQ2Rows / 4; ++kk) {
-        const int k = 4 * kk + lk;
-        const int q = k / 3, r = k - 3 * q;
-        double v0 = 0.0, v1 = 0.0, c = 0.0;
-        if (k < 81) {
-            const double j0 = Jis[q][r], j1 = Jis[q][3 + r], j2 = Jis[q][6 + r];
-            const double* g0 = tab.g[q][li];
-            const double* g1 = tab.g[q][a1];
-            c = cs[q];
-            v0 = j0 * g0[0] + j1 * g0[1] + j2 * g0[2];
-            if (has1) v1 = j0 * g1[0] + j1 * g1[1] + j2 * g1[2];
+}
+
+// a lane's part: its (i, i') and field of the first stage, its (i, j) and
+// (i', j') of the second
+struct Q2Lane {
+    int xrow;      // row of Q2Tables::x
+    int g;         // field of G
+    int p1, p1t;   // (i, i') and (i', i)
+    int py;        // (j, j')
+    uint32_t a, b;   // the local shapes (i, j, m) and (i', j', m), m = 0, 1, 2, a byte each
+    int mi;          // multi-index of shape l % 32, two bits each
+    __device__ __forceinline__ void init(int l) {
+        // fields dd Gxx, ll Gyy, ll Gzz, ll Gyz, dl Gxy, dl Gxz of nine pairs each
+        const int pair = l < 54 ? l % 9 : 0, field = l < 54 ? l / 9 : 0;
+        xrow = (field == 0 ? 2 : field < 4 ? 0 : 1) * 9 + pair;
+        g = field == 3 ? 5 : field == 4 ? 3 : field == 5 ? 4 : field;
+        int u = 0, v = l < 45 ? l : 0;   // the l-th u <= v of 9
+        while (v >= 9 - u) {
+            v -= 9 - u;
+            ++u;
         }
-        acc00 = __builtin_amdgcn_mfma_f64_16x16x4f64(c * v0, v0, acc00, 0, 0, 0);
-        acc01 = __builtin_amdgcn_mfma_f64_16x16x4f64(c * v0, v1, acc01, 0, 0, 0);
-        acc11 = __builtin_amdgcn_mfma_f64_16x16x4f64(c * v1, v1, acc11, 0, 0, 0);
+        v += u;
+        a = kQ2Basis.num[u] | kQ2Basis.num[u + 9] << 8 | kQ2Basis.num[u + 18] << 16;
+        b = kQ2Basis.num[v] | kQ2Basis.num[v + 9] << 8 | kQ2Basis.num[v + 18] << 16;
+        const int s = (l & 31) < 27 ? l & 31 : 0;
+        mi = kQ2Mi[s][0] | kQ2Mi[s][1] << 2 | kQ2Mi[s][2] << 4;
+        p1 = (u % 3) * 3 + v % 3;
+        p1t = (v % 3) * 3 + u % 3;
+        py = (u / 3) * 3 + v / 3;
     }
-    if (!valid) return;
+};
+
+// A lane's inputs of the element of its half (l / 32): corner coordinate l % 32
+// and the coefficient at Gauss point l % 32 (x fastest); the unit cube for an
+// element that is not there
+struct Q2In {
+    double x, k;
+};
+template <class Src>
+__device__ __forceinline__ Q2In q2_load(int l, const bool (&valid)[2], const Src& src) {
+    const int hl = l & 31, c = hl / 3, d = hl - 3 * c;
+    const int bit = d == 0 ? (c == 1 || c == 2 || c == 5 || c == 6) : d == 1 ? (c == 2 || c == 3 || c == 6 || c == 7)
+                                                                     : (c >= 4);
+    const bool mine = l >> 5 ? valid[1] : valid[0];
+    Q2In in;
+    in.x = mine && hl < 24 ? src.corner(hl) : (double)bit;
+    in.k = mine && hl < 27 ? src.k(hl) : 1.0;
+    return in;
+}
+
+// Two elements by one wavefront (lane l): sink.ke(l, K) with the element matrix K
+// in LDS and sink.fe(a, v) for the 27 load entries of each valid element.
+template <class Sink>
+__device__ __forceinline__ void q2_element_pair(int l, const Q2Lane& L, const Q2Tables& tab, const bool (&valid)[2],
+                                                Q2In in, Sink (&sink)[2], double f_const, Q2Scratch& sh,
+                                                bool want_fe) {
+    // what follows from the lane alone is formed again for every pair of elements:
+    // kept across them, it would take the registers of the stages below
+    asm volatile("" : "+v"(l));
+    const int half = l >> 5, hl = l & 31;
+    const bool mine = half ? valid[1] : valid[0];
+    q2_wave_sync();   // the elements before are done with the scratch
+    if (hl < 24) sh.X[half][hl] = in.x;
+    q2_wave_sync();
+    // 1. G at point q = hl: the Jacobian of the trilinear map column by column
+    if (hl < 27) {
+        const double* X = sh.X[half];
+        const int qx = hl % 3, qy = (hl / 3) % 3, qz = hl / 9;
+        const double x1 = q2_gauss(qx), y1 = q2_gauss(qy), z1 = q2_gauss(qz);
+        const double x0 = 1.0 - x1, y0 = 1.0 - y1, z0 = 1.0 - z1;
+        double J[3][3];   // J[c][r] = dX_r / dxi_c
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int i = lk + 4 * v;
-        sink.ke(i, li, acc00[v]);
-        if (has1) {
-            sink.ke(i, 16 + li, acc01[v]);
-            sink.ke(16 + li, i, acc01[v]);
+        for (int r = 0; r < 3; ++r) {
+            const double X0 = X[r], X1 = X[3 + r], X2 = X[6 + r], X3 = X[9 + r], X4 = X[12 + r], X5 = X[15 + r],
+                         X6 = X[18 + r], X7 = X[21 + r];
+            J[0][r] = z0 * (y0 * (X1 - X0) + y1 * (X2 - X3)) + z1 * (y0 * (X5 - X4) + y1 * (X6 - X7));
+            J[1][r] = z0 * (x0 * (X3 - X0) + x1 * (X2 - X1)) + z1 * (x0 * (X7 - X4) + x1 * (X6 - X5));
+            J[2][r] = y0 * (x0 * (X4 - X0) + x1 * (X5 - X1)) + y1 * (x0 * (X7 - X3) + x1 * (X6 - X2));
         }
-        if (16 + i < 27 && has1) sink.ke(16 + i, 16 + li, acc11[v]);
+        double C[3][3];   // rows of det J J^-1
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double* p = J[(d + 1) % 3];
+            const double* q = J[(d + 2) % 3];
+            C[d][0] = p[1] * q[2] - p[2] * q[1];
+            C[d][1] = p[2] * q[0] - p[0] * q[2];
+            C[d][2] = p[0] * q[1] - p[1] * q[0];
+        }
+        const double det = fabs(J[0][0] * C[0][0] + J[0][1] * C[0][1] + J[0][2] * C[0][2]);
+        const double w = q2_gauss_w(qx) * q2_gauss_w(qy) * q2_gauss_w(qz);
+        const double g = w * in.k / det;
+        auto dot = [&](int d, int e) { return g * (C[d][0] * C[e][0] + C[d][1] * C[e][1] + C[d][2] * C[e][2]); };
+        sh.G[half][0][hl] = dot(0, 0);
+        sh.G[half][1][hl] = dot(1, 1);
+        sh.G[half][2][hl] = dot(2, 2);
+        sh.G[half][3][hl] = dot(0, 1);
+        sh.G[half][4][hl] = dot(0, 2);
+        sh.G[half][5][hl] = dot(1, 2);
+        if (want_fe) sh.fw[half][hl] = w * det * f_const;
     }
+    q2_wave_sync();
+    // load vector: fe[a] = sum_q w_q |det J_q| f phi_a(xi_q)
+    if (want_fe && hl < 27) {
+        const double *lx = tab.l[L.mi & 3], *ly = tab.l[L.mi >> 2 & 3], *lz = tab.l[L.mi >> 4];
+        double s = 0.0;
+#pragma unroll 1
+        for (int qz = 0; qz < 3; ++qz) {
+            double sy = 0.0;
+#pragma unroll
+            for (int qy = 0; qy < 3; ++qy) {
+                const double* f = sh.fw[half] + 3 * qy + 9 * qz;
+                const double sx = f[0] * lx[0] + f[1] * lx[1] + f[2] * lx[2];
+                sy = fma(ly[qy], sx, sy);
+            }
+            s = fma(lz[qz], sy, s);
+        }
+        if (mine && half) sink[1].fe(hl, s);
+        if (mine && !half) sink[0].fe(hl, s);
+    }
+#pragma unroll 1
+    for (int el = 0; el < 2; ++el) {
+        if (!(el ? valid[1] : valid[0])) continue;   // the same for the whole wavefront
+        Q2Lane M = L;
+        asm volatile("" : "+v"(M.xrow), "+v"(M.g), "+v"(M.p1), "+v"(M.p1t), "+v"(M.py), "+v"(M.a), "+v"(M.b));
+        // 2. sums over x: T[field][pair][qy + 3 qz]
+        double* T = sh.K;
+        q2_wave_sync();
+        if (l < 54) {
+            const double* G = sh.G[el][M.g];
+            const double* c = tab.x[0][0] + 3 * M.xrow;
+            const double c0 = c[0], c1 = c[1], c2 = c[2];
+            double v[27];
+#pragma unroll
+            for (int p = 0; p < 27; ++p) v[p] = G[p];
+#pragma unroll
+            for (int p = 0; p < 9; ++p) T[l * 9 + p] = fma(c2, v[3 * p + 2], fma(c1, v[3 * p + 1], c0 * v[3 * p]));
+        }
+        q2_wave_sync();
+        // 3. sums over y, then over z: V[m][m'] of the lane's (i, j), (i', j')
+        double V[3][3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) V[m][k] = 0.0;
+        double y[12];
+#pragma unroll
+        for (int q = 0; q < 12; ++q) y[q] = tab.y[M.py][q];
+        const double* Txx = T + M.p1 * 9;
+        const double* Tyy = T + 81 + M.p1 * 9;
+        const double* Tzz = T + 162 + M.p1 * 9;
+        const double* Tyz = T + 243 + M.p1 * 9;
+        const double* Txy = T + 324 + M.p1 * 9;    // derivative on i
+        const double* Tyx = T + 324 + M.p1t * 9;   // derivative on i'
+        const double* Txz = T + 405 + M.p1 * 9;
+        const double* Tzx = T + 405 + M.p1t * 9;
+#pragma unroll
+        for (int qz = 0; qz < 3; ++qz) {
+            // one plane of T in registers at a time: its offset is known once the
+            // plane before is done
+            int o = 3 * qz;
+            asm volatile("" : "+v"(o) : "v"(V[2][2]));
+            double ull = 0.0, uld = 0.0, udl = 0.0, udd = 0.0;   // by the z factors of (a, b)
+#pragma unroll
+            for (int qy = 0; qy < 3; ++qy) {
+                const int p = o + qy;
+                const double yz = Tyz[p];
+                ull = fma(y[qy], Txx[p], ull);
+                ull = fma(y[9 + qy], Tyy[p], ull);
+                ull = fma(y[3 + qy], Txy[p], ull);
+                ull = fma(y[6 + qy], Tyx[p], ull);
+                udd = fma(y[qy], Tzz[p], udd);
+                uld = fma(y[qy], Txz[p], uld);
+                uld = fma(y[6 + qy], yz, uld);
+                udl = fma(y[qy], Tzx[p], udl);
+                udl = fma(y[3 + qy], yz, udl);
+            }
+            // constants that vanish at the middle point drop out
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const double lk = q2c_l(k, q2c_x(qz)), dk = q2c_dl(k, q2c_x(qz));
+                double A = 0.0, D = 0.0;
+                if (lk != 0.0) {
+                    A = ull * lk;
+                    D = udl * lk;
+                }
+                if (dk != 0.0) {
+                    A = fma(uld, dk, A);
+                    D = fma(udd, dk, D);
+                }
+#pragma unroll
+                for (int m = 0; m < 3; ++m) {
+                    const double lm = q2c_l(m, q2c_x(qz)), dm = q2c_dl(m, q2c_x(qz));
+                    if (lm != 0.0) V[m][k] = fma(lm, A, V[m][k]);
+                    if (dm != 0.0) V[m][k] = fma(dm, D, V[m][k]);
+                }
+            }
+        }
+        q2_wave_sync();   // T is read before its place takes the matrix
+        if (l < 45) {
+            int a[3], b[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                a[m] = M.a >> (8 * m) & 255u;
+                b[m] = M.b >> (8 * m) & 255u;
+            }
+            // an entry and its transpose take the same value
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    sh.K[27 * a[m] + b[k]] = V[m][k];
+                    sh.K[27 * b[k] + a[m]] = V[m][k];
+                }
+        }
+        q2_wave_sync();
+        if (el) sink[1].ke(l, sh.K);
+        else sink[0].ke(l, sh.K);
+    }
+}
+
+// adds the element matrix to val at slot(i, j): no two entries of an element
+// share a slot, so a lane's twelve slots and then its twelve values are in flight
+// together
+template <class Slot>
+__device__ __forceinline__ void q2_add(int l, const double* K, double* val, const Slot& slot) {
+    int32_t p[12];
+    double v[12];
+#pragma unroll
+    for (int r = 0; r < 12; ++r) {
+        const int e = l + 64 * r < 729 ? l + 64 * r : 728;
+        const int i = (int)((unsigned)e * 2428u >> 16);   // e / 27
+        p[r] = slot(i, e - 27 * i);
+    }
+#pragma unroll
+    for (int r = 0; r < 12; ++r) v[r] = val[p[r]];
+#pragma unroll
+    for (int r = 0; r < 12; ++r)
+        if (l + 64 * r < 729) val[p[r]] = v[r] + K[l + 64 * r];
 }
 
 struct Q2ArraySrc {
@@ -185,25 +346,44 @@ struct Q2ArraySrc {
 struct Q2ArraySink {
     double* Kout;
     double* fout;
-    __device__ void ke(int i, int j, double v) { Kout[i * 27 + j] = v; }
+    __device__ __forceinline__ void ke(int l, const double* K) {
+        for (int e = l; e < 729; e += 64) Kout[e] = K[e];
+    }
     __device__ void fe(int a, double v) { fout[a] = v; }
 };
 
-__global__ __launch_bounds__(64 * kQ2Waves) void k_q2_hex_elements(int64_t n, const double* __restrict__ X,
+// Every wavefront takes pairs of elements in turn. Bound by the 5.8 kB that an
+// element writes: 64^3 elements (1.64 GB with the inputs) 482 us on one MI355X, 838 us with
+// the contraction over all points on the matrix cores (129 kflop an element in
+// their 16 x 16 x 4 steps, four of ten of their FP64 rate), Jacobians by 27 of 64
+// lanes and every entry stored from where it arose. What is left is latency: three
+// waves a SIMD (a fourth would spill: 748 us), each a chain through LDS.
+__global__ __launch_bounds__(64 * kQ2Waves, 3) void k_q2_hex_elements(int64_t n, const double* __restrict__ X,
                                                                    const double* __restrict__ kcoef, double f_const,
                                                                    double* __restrict__ Ke, double* __restrict__ fe) {
-    const int w = threadIdx.x >> 6;
-    const int64_t e = (int64_t)blockIdx.x * kQ2Waves + w;
-    const bool valid = e < n;   // the last workgroup may hold fewer elements; every wave reaches the barriers
-    __shared__ double Xs_all[kQ2Waves][24];
-    __shared__ double Jis_all[kQ2Waves][27][9];
-    __shared__ double cs_all[kQ2Waves][28], fw_all[kQ2Waves][27];
-    __shared__ Q2RefGrad tab;
-    q2_stage_table(tab);
-    Q2ArraySrc src{X, kcoef, e};
-    Q2ArraySink sink{Ke + (valid ? e : 0) * 729, fe ? fe + (valid ? e : 0) * 27 : nullptr};
-    q2_element_wave(threadIdx.x & 63, valid, src, sink, f_const, Xs_all[w], Jis_all[w], cs_all[w], fw_all[w],
-                    fe != nullptr, tab);
+    __shared__ Q2Scratch sh[kQ2Waves];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    __shared__ Q2Tables tab;
+    q2_fill_tables(tab);
+    Q2Lane L;
+    L.init(l);
+    // the next pair's inputs are in flight while a pair is computed
+    auto load = [&](int64_t p) {
+        const bool valid[2] = {2 * p < n, 2 * p + 1 < n};
+        return q2_load(l, valid, Q2ArraySrc{X, kcoef, 2 * p + (l >> 5)});
+    };
+    const int64_t step = (int64_t)gridDim.x * kQ2Waves;
+    int64_t p = (int64_t)blockIdx.x * kQ2Waves + w;
+    Q2In in = load(p);
+    for (; 2 * p < n; p += step) {
+        const bool valid[2] = {true, 2 * p + 1 < n};
+        const int64_t e1 = valid[1] ? 2 * p + 1 : 2 * p;
+        Q2ArraySink sink[2] = {{Ke + 2 * p * 729, fe ? fe + 2 * p * 27 : nullptr},
+                               {Ke + e1 * 729, fe ? fe + e1 * 27 : nullptr}};
+        const Q2In next = load(p + step);
+        q2_element_pair(l, L, tab, valid, in, sink, f_const, sh[w], fe != nullptr);
+        in = next;
+    }
 }
 
 // ---- assembly on the unit-cube lattice of n^3 elements ----
@@ -249,19 +429,6 @@ __global__ __launch_bounds__(256) void k_q2_lattice_fill(int W, int64_t N, const
     }
 }
 
-// the CSR slot of (r, c): the row's columns are its box [x0,x1] x [y0,y1] x
-// [z0,z1] in (z, y, x) order, so the position follows from the offsets
-__device__ __forceinline__ int32_t q2_slot(int W, const int32_t* __restrict__ rowptr, int32_t r, int32_t c) {
-    const int x = r % W, y = (r / W) % W, z = r / (W * W);
-    const int cx = c % W, cy = (c / W) % W, cz = c / (W * W);
-    int x0, x1, y0, y1, z0, z1;
-    q2_range(x, W, x0, x1);
-    q2_range(y, W, y0, y1);
-    q2_range(z, W, z0, z1);
-    const int nx = x1 - x0 + 1, ny = y1 - y0 + 1;
-    return rowptr[r] + ((cz - z0) * ny + (cy - y0)) * nx + (cx - x0);
-}
-
 struct Q2LatticeSrc {
     int n;
     double h;
@@ -276,39 +443,68 @@ struct Q2LatticeSrc {
     }
     __device__ double k(int) const { return theta ? exp(theta[((int64_t)ez * n + ey) * n + ex]) : 1.0; }
 };
+// Entry (i, j) of element (ex, ey, ez): the row's columns are its box [x0,x1] x
+// [y0,y1] x [z0,z1] in (z, y, x) order, so the CSR slot follows from the
+// multi-indices; decoding node numbers took eight divisions an entry (a colour of
+// 32,768 elements 301 us, 231 so and with a lane's slots in flight together, one
+// MI355X)
 struct Q2CsrSink {
     int W, ex, ey, ez;
     const int32_t* rowptr;
-    const int32_t* col;
     double* val;
     double* rhs;
-    __device__ int32_t node(int a) const {
-        return (int32_t)(((int64_t)(2 * ez + kQ2Mi[a][2]) * W + (2 * ey + kQ2Mi[a][1])) * W + (2 * ex + kQ2Mi[a][0]));
+    const int* mi;
+    __device__ __forceinline__ int32_t node(int m) const {
+        return ((2 * ez + (m >> 4)) * W + 2 * ey + (m >> 2 & 3)) * W + 2 * ex + (m & 3);
     }
-    __device__ void ke(int i, int j, double v) { val[q2_slot(W, rowptr, node(i), node(j))] += v; }
-    __device__ void fe(int a, double v) { rhs[node(a)] += v; }
+    __device__ __forceinline__ int32_t slot(int i, int j) const {
+        const int a = mi[i], b = mi[j];
+        const int x = 2 * ex + (a & 3), y = 2 * ey + (a >> 2 & 3), z = 2 * ez + (a >> 4);
+        const int cx = 2 * ex + (b & 3), cy = 2 * ey + (b >> 2 & 3), cz = 2 * ez + (b >> 4);
+        int x0, x1, y0, y1, z0, z1;
+        q2_range(x, W, x0, x1);
+        q2_range(y, W, y0, y1);
+        q2_range(z, W, z0, z1);
+        const int nx = x1 - x0 + 1, ny = y1 - y0 + 1;
+        return rowptr[(z * W + y) * W + x] + ((cz - z0) * ny + (cy - y0)) * nx + (cx - x0);
+    }
+    __device__ __forceinline__ void ke(int l, const double* K) {
+        q2_add(l, K, val, [&](int i, int j) { return slot(i, j); });
+    }
+    __device__ __forceinline__ void fe(int a, double v) { rhs[node(mi[a])] += v; }
 };
 
 // one colour (element parities px, py, pz): no two of its elements share a node
-__global__ __launch_bounds__(64 * kQ2Waves) void k_q2_lattice_assemble(int n, int color, const double* theta,
+__global__ __launch_bounds__(64 * kQ2Waves, 3) void k_q2_lattice_assemble(int n, int color, const double* theta,
                                                                        double f_const, const int32_t* rowptr,
-                                                                       const int32_t* col, double* val, double* rhs) {
+                                                                       double* val, double* rhs) {
     const int hn = (n + 1) / 2;
-    const int w = threadIdx.x >> 6;
-    const int64_t t = (int64_t)blockIdx.x * kQ2Waves + w;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int64_t p = (int64_t)blockIdx.x * kQ2Waves + w;
     const int px = color & 1, py = (color >> 1) & 1, pz = color >> 2;
-    const int tx = (int)(t % hn), ty = (int)((t / hn) % hn), tz = (int)(t / ((int64_t)hn * hn));
-    const int ex = 2 * tx + px, ey = 2 * ty + py, ez = 2 * tz + pz;
-    const bool valid = t < (int64_t)hn * hn * hn && ex < n && ey < n && ez < n;
-    __shared__ double Xs_all[kQ2Waves][24];
-    __shared__ double Jis_all[kQ2Waves][27][9];
-    __shared__ double cs_all[kQ2Waves][28], fw_all[kQ2Waves][27];
-    __shared__ Q2RefGrad tab;
-    q2_stage_table(tab);
-    Q2LatticeSrc src{n, 1.0 / n, ex, ey, ez, theta};
-    Q2CsrSink sink{2 * n + 1, ex, ey, ez, rowptr, col, val, rhs};
-    q2_element_wave(threadIdx.x & 63, valid, src, sink, f_const, Xs_all[w], Jis_all[w], cs_all[w], fw_all[w],
-                    rhs != nullptr, tab);
+    __shared__ Q2Scratch sh[kQ2Waves];
+    __shared__ Q2Tables tab;
+    q2_fill_tables(tab);
+    Q2Lane L;
+    L.init(l);
+    Q2LatticeSrc src{n, 1.0 / n, 0, 0, 0, theta};   // of the lane's half
+    Q2CsrSink sink[2];
+    bool valid[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int64_t t = 2 * p + h;
+        const int tx = (int)(t % hn), ty = (int)((t / hn) % hn), tz = (int)(t / ((int64_t)hn * hn));
+        const int ex = 2 * tx + px, ey = 2 * ty + py, ez = 2 * tz + pz;
+        valid[h] = t < (int64_t)hn * hn * hn && ex < n && ey < n && ez < n;
+        if (h == l >> 5) {
+            src.ex = ex;
+            src.ey = ey;
+            src.ez = ez;
+        }
+        sink[h] = Q2CsrSink{2 * n + 1, ex, ey, ez, rowptr, val, rhs, tab.mi};
+    }
+    q2_element_pair(l, L, tab, valid, q2_load(l, valid, src), sink, f_const, sh[w],
+                    rhs != nullptr);
 }
 
 // Dirichlet rows (u = 0 on the boundary of the cube): row := unit row on its
@@ -344,35 +540,42 @@ struct Q2SlotSink {
     int64_t ne, pos, e;
     double* val;
     double* rhs;
-    __device__ void ke(int i, int j, double v) {
-        if (val) val[slot[(int64_t)(27 * i + j) * ne + pos]] += v;
+    __device__ __forceinline__ void ke(int l, const double* K) {
+        if (val) q2_add(l, K, val, [&](int i, int j) { return slot[(int64_t)(27 * i + j) * ne + pos]; });
     }
     __device__ void fe(int a, double v) { rhs[dofs[e * 27 + a]] += v; }
 };
 
 // one colour's elements (positions pos0 .. pos0+cnt-1 of the colour order),
 // one element per wavefront
-__global__ __launch_bounds__(64 * kQ2Waves) void k_elem_hex_q2(int64_t ne, const int32_t* __restrict__ order,
+__global__ __launch_bounds__(64 * kQ2Waves, 3) void k_elem_hex_q2(int64_t ne, const int32_t* __restrict__ order,
                                                                const int32_t* __restrict__ dofs,
                                                                const double* __restrict__ coords,
                                                                const double* __restrict__ kel,
                                                                const double* __restrict__ kq, double f_const,
                                                                const int32_t* __restrict__ slot, double* val,
                                                                double* rhs, int64_t pos0, int64_t cnt) {
-    const int w = threadIdx.x >> 6;
-    const int64_t t = (int64_t)blockIdx.x * kQ2Waves + w;
-    const bool valid = t < cnt;   // every wave reaches the barriers of the element routine
-    const int64_t pos = pos0 + (valid ? t : 0);
-    const int64_t e = order[pos];
-    __shared__ double Xs_all[kQ2Waves][24];
-    __shared__ double Jis_all[kQ2Waves][27][9];
-    __shared__ double cs_all[kQ2Waves][28], fw_all[kQ2Waves][27];
-    __shared__ Q2RefGrad tab;
-    q2_stage_table(tab);
-    Q2ElemSrc src{coords, dofs, kel, kq, e};
-    Q2SlotSink sink{slot, dofs, ne, pos, e, val, rhs};
-    q2_element_wave(threadIdx.x & 63, valid, src, sink, f_const, Xs_all[w], Jis_all[w], cs_all[w], fw_all[w],
-                    rhs != nullptr, tab);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int64_t p = (int64_t)blockIdx.x * kQ2Waves + w;
+    __shared__ Q2Scratch sh[kQ2Waves];
+    __shared__ Q2Tables tab;
+    q2_fill_tables(tab);
+    Q2Lane L;
+    L.init(l);
+    Q2ElemSrc src{coords, dofs, kel, kq, 0};   // of the lane's half
+    Q2SlotSink sink[2];
+    bool valid[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int64_t t = 2 * p + h;
+        valid[h] = t < cnt;
+        const int64_t pos = pos0 + (valid[h] ? t : 0);
+        const int64_t e = order[pos];
+        if (h == l >> 5) src.e = e;
+        sink[h] = Q2SlotSink{slot, dofs, ne, pos, e, val, rhs};
+    }
+    q2_element_pair(l, L, tab, valid, q2_load(l, valid, src), sink, f_const, sh[w],
+                    rhs != nullptr);
 }
 
 }  // namespace
@@ -381,8 +584,10 @@ int q2_hex_elements(int64_t n, const double* X, const double* k, double f_const,
                     hipStream_t s) {
     if (n <= 0) return 0;
     if (!X || !Ke || n > (int64_t)INT32_MAX) return -1;
-    hipLaunchKernelGGL(k_q2_hex_elements, dim3((unsigned)((n + kQ2Waves - 1) / kQ2Waves)), dim3(64 * kQ2Waves), 0, s,
-                       n, X, k, f_const, Ke, fe);
+    const int64_t need = (n + 2 * kQ2Waves - 1) / (2 * kQ2Waves);
+    const int64_t fit = (int64_t)device_cus() * resident_blocks(reinterpret_cast<const void*>(&k_q2_hex_elements), 0);
+    hipLaunchKernelGGL(k_q2_hex_elements, dim3((unsigned)std::min(need, fit)), dim3(64 * kQ2Waves), 0, s, n, X, k,
+                       f_const, Ke, fe);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -404,8 +609,8 @@ int q2_lattice_assemble(int n, const double* theta, double f_const, const int32_
     const int hn = (n + 1) / 2;
     const int64_t per = (int64_t)hn * hn * hn;
     for (int color = 0; color < 8; ++color)
-        hipLaunchKernelGGL(k_q2_lattice_assemble, dim3((unsigned)((per + kQ2Waves - 1) / kQ2Waves)),
-                           dim3(64 * kQ2Waves), 0, s, n, color, theta, f_const, rowptr, col, val, rhs);
+        hipLaunchKernelGGL(k_q2_lattice_assemble, dim3((unsigned)((per + 2 * kQ2Waves - 1) / (2 * kQ2Waves))),
+                           dim3(64 * kQ2Waves), 0, s, n, color, theta, f_const, rowptr, val, rhs);
     const int W = 2 * n + 1;
     const int64_t N = (int64_t)W * W * W;
     hipLaunchKernelGGL(k_q2_lattice_dirichlet, dim3((unsigned)std::min<int64_t>((N + 255) / 256, 65536)), dim3(256),
@@ -417,7 +622,7 @@ int elem_assemble_q2_colour(int64_t ne, const int32_t* order, const int32_t* dof
                             const double* kel, const double* kq, double f_const, const int32_t* slot, double* val,
                             double* rhs, int64_t pos0, int64_t cnt, hipStream_t s) {
     if (cnt <= 0) return 0;
-    hipLaunchKernelGGL(k_elem_hex_q2, dim3((unsigned)((cnt + kQ2Waves - 1) / kQ2Waves)), dim3(64 * kQ2Waves), 0, s,
+    hipLaunchKernelGGL(k_elem_hex_q2, dim3((unsigned)((cnt + 2 * kQ2Waves - 1) / (2 * kQ2Waves))), dim3(64 * kQ2Waves), 0, s,
                        ne, order, dofs, coords, kel, kq, f_const, slot, val, rhs, pos0, cnt);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
