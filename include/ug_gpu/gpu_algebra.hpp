@@ -873,10 +873,14 @@ class AssembledMultiGridCycle : public ILinearIterator {
     // direction update) and q = A p_new with (q, p_new) into qp_out[0] in one
     // pass; p_new and p_old are distinct lattice vectors with the halo; false
     // when the top level is not matrix-free
+    // (rho_old, device: the factor is beta[0] / rho_old[0]). With np_out the
+    // products of these two stay in `partial` where the next CG update sums
+    // them itself: np_out[0] of them, 0 where they were summed.
     bool surface_direction_axpy_lattice(double* q, const double* p_old, const double* z, const double* beta,
-                                        double* p_new, double* qp_out, double* partial);
+                                        double* p_new, double* qp_out, double* partial,
+                                        const double* rho_old = nullptr, int* np_out = nullptr);
     bool surface_axpy_lattice(double* y, double alpha, const double* v, double beta, const double* x,
-                              double* yx_out = nullptr, double* partial = nullptr);
+                              double* yx_out = nullptr, double* partial = nullptr, int* np_out = nullptr);
     static constexpr int max_partials() { return 65536; }
     struct Impl;
 

@@ -1031,7 +1031,7 @@ bool CG::apply_lattice(GPUVector& x, const GPUVector& src, AssembledMultiGridCyc
     if (kind == 2) gmg.surface_axpy_lattice(rl, 1.0, rl, -1.0, xl);   // r = b - A x
     // p = z = B r, rho = (z, r): the first z is written where p lives (the
     // loop's z buffer is written afresh before it is read)
-    gmg.apply_lattice(pl, rl, sc + 0, part, rf_first);
+    gmg.apply_lattice(pl, rl, sc + 4, part, rf_first);
     conv_->set_name(name());
     conv_->start_defect(dev_dot(N, rl, rl, true));
     // second direction buffer: the fused update writes p_new beside p_old
@@ -1041,16 +1041,17 @@ bool CG::apply_lattice(GPUVector& x, const GPUVector& src, AssembledMultiGridCyc
     }
     double* pl2 = ws_p2_.get() + H;
     bool q_ready = false;   // q = A p and lambda already formed with the direction update
+    int nl = 0;             // lambda's partial sums left to cg_update (in part)
     bool ok = true;
     while (!conv_->iteration_ended()) {
         // q = A p, lambda = (q, p)
-        if (!q_ready && !gmg.surface_axpy_lattice(ql, 0.0, ql, 1.0, pl, sc + 1, part)) {
+        if (!q_ready && !gmg.surface_axpy_lattice(ql, 0.0, ql, 1.0, pl, sc + 1, part, &nl)) {
+            nl = 0;
             gmg.surface_axpy_lattice(ql, 0.0, ql, 1.0, pl);
             UGX_LAUNCH(dot<double>(N, ql, pl, c.red_partial, sc + 1, false, c.stream));
         }
         q_ready = false;
-        UGX_LAUNCH(cg_update(N, sc, pl, ql, xl, rl, part, c.stream, rfl));
-        UGX_HIP(hipMemcpyAsync(c.red_host, sc + 5, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+        UGX_LAUNCH(cg_update(N, sc, pl, ql, xl, rl, c.red_partial, c.red_host, c.stream, rfl, nl, part));
         sync();
         if (c.red_host[1] != 0.0) {   // lambda == 0: breakdown (x, r unchanged)
             ok = false;
@@ -1059,9 +1060,8 @@ bool CG::apply_lattice(GPUVector& x, const GPUVector& src, AssembledMultiGridCyc
         conv_->update_defect(std::sqrt(c.red_host[0]));
         if (conv_->iteration_ended()) break;
         gmg.apply_lattice(zl, rl, sc + 4, part, rfl);   // z = B r, rho_new = (z, r)
-        UGX_LAUNCH(cg_beta(sc, c.stream));          // beta = rho_new / rho, rho = rho_new
-        // p = z + beta p, fused with the next q = A p when the operator allows
-        if (gmg.surface_direction_axpy_lattice(ql, pl, zl, sc + 3, pl2, sc + 1, part)) {
+        // p = z + rho_new / rho p, fused with the next q = A p when the operator allows
+        if (gmg.surface_direction_axpy_lattice(ql, pl, zl, sc + 4, pl2, sc + 1, part, sc + 0, &nl)) {
             std::swap(pl, pl2);
             q_ready = true;
         } else {
@@ -1114,12 +1114,11 @@ bool CG::apply_return_defect(GPUVector& x, GPUVector& b) {
     conv_->set_name(name());
     conv_->start(r);
     p = z;
-    UGX_LAUNCH(dot<double>(n, z.data(), r.data(), c.red_partial, sc + 0, false, c.stream));
+    UGX_LAUNCH(dot<double>(n, z.data(), r.data(), c.red_partial, sc + 4, false, c.stream));
     while (!conv_->iteration_ended()) {
         op_->apply(q, p);
         UGX_LAUNCH(dot<double>(n, q.data(), p.data(), c.red_partial, sc + 1, false, c.stream));
-        UGX_LAUNCH(cg_update(n, sc, p.data(), q.data(), x.data(), r.data(), c.red_partial, c.stream));
-        UGX_HIP(hipMemcpyAsync(c.red_host, sc + 5, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+        UGX_LAUNCH(cg_update(n, sc, p.data(), q.data(), x.data(), r.data(), c.red_partial, c.red_host, c.stream));
         sync();
         if (c.red_host[1] != 0.0 && n) return false;   // lambda == 0 (x, r unchanged)
         conv_->update_defect(std::sqrt(c.red_host[0]));
@@ -1130,7 +1129,6 @@ bool CG::apply_return_defect(GPUVector& x, GPUVector& b) {
             z = r;
         }
         UGX_LAUNCH(dot<double>(n, z.data(), r.data(), c.red_partial, sc + 4, false, c.stream));
-        UGX_LAUNCH(cg_beta(sc, c.stream));
         UGX_LAUNCH(cg_direction(n, sc, p.data(), z.data(), c.stream));
     }
     return conv_->post();
@@ -2004,9 +2002,10 @@ struct AssembledMultiGridCycle::Impl {
     virtual void cycle_buffers(void*& defect, void*& correction) = 0;
     virtual void run_cycle() = 0;
     virtual bool surface_axpy(double* y, double alpha, const double* v, double beta, const double* x, double* yx_out,
-                              double* partial) = 0;
+                              double* partial, int* np_out) = 0;
     virtual bool surface_direction_axpy(double* q, const double* p_old, const double* z, const double* beta,
-                                        double* p_new, double* qp_out, double* partial) = 0;
+                                        double* p_new, double* qp_out, double* partial, const double* rho_old,
+                                        int* np_out) = 0;
     virtual int64_t halo() const = 0;
 };
 
@@ -2682,8 +2681,17 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         UGX_HIP(hipGraphLaunch(cycle_exec, c.stream));
     }
 
+    void keep_or_sum(int np, double* partial, double* out, int* np_out) {
+        if (np_out && cg_update_sums(L[top].N, np)) {
+            *np_out = np;
+            return;
+        }
+        if (np_out) *np_out = 0;
+        UGX_LAUNCH(sum_partials(np, partial, out, context().stream));
+    }
+
     bool surface_axpy(double* y, double alpha, const double* v, double beta, const double* x, double* yx_out,
-                      double* partial) override {
+                      double* partial, int* np_out) override {
         GmgLevel<T>& t = L[top];
         auto& c = context();
         if (mf) {
@@ -2691,7 +2699,7 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                 int np = AssembledMultiGridCycle::max_partials();
                 if (q1mf_axpy<double>(t.W, cell_c64.get(), alpha, v, beta, x, y, c.stream, partial, &np) != 0)
                     return false;
-                UGX_LAUNCH(sum_partials(np, partial, yx_out, c.stream));
+                keep_or_sum(np, partial, yx_out, np_out);
                 return true;
             }
             UGX_LAUNCH(q1mf_axpy<double>(t.W, cell_c64.get(), alpha, v, beta, x, y, c.stream));
@@ -2705,14 +2713,14 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
     // p_new = z + beta p_old and q = A p_new with (q, p_new) in one pass
     // (matrix-free top level only)
     bool surface_direction_axpy(double* q, const double* p_old, const double* z, const double* beta, double* p_new,
-                                double* qp_out, double* partial) override {
+                                double* qp_out, double* partial, const double* rho_old, int* np_out) override {
         if (!mf) return false;
         auto& c = context();
         int np = AssembledMultiGridCycle::max_partials();
-        if (q1mf_direction_axpy<double>(L[top].W, cell_c64.get(), p_old, z, beta, p_new, q, c.stream, partial, &np) !=
-            0)
+        if (q1mf_direction_axpy<double>(L[top].W, cell_c64.get(), p_old, z, beta, p_new, q, c.stream, partial, &np,
+                                        rho_old) != 0)
             return false;
-        UGX_LAUNCH(sum_partials(np, partial, qp_out, c.stream));
+        keep_or_sum(np, partial, qp_out, np_out);
         return true;
     }
 
@@ -2791,14 +2799,14 @@ void AssembledMultiGridCycle::apply_lattice(double* c_lat, const double* d_lat, 
 bool AssembledMultiGridCycle::lattice_uses_f32_defect() const { return impl_ && impl_->uses_f32_defect(); }
 bool AssembledMultiGridCycle::surface_direction_axpy_lattice(double* q, const double* p_old, const double* z,
                                                              const double* beta, double* p_new, double* qp_out,
-                                                             double* partial) {
+                                                             double* partial, const double* rho_old, int* np_out) {
     if (!impl_) throw UGError("GMG: not initialised");
-    return impl_->surface_direction_axpy(q, p_old, z, beta, p_new, qp_out, partial);
+    return impl_->surface_direction_axpy(q, p_old, z, beta, p_new, qp_out, partial, rho_old, np_out);
 }
 bool AssembledMultiGridCycle::surface_axpy_lattice(double* y, double alpha, const double* v, double beta,
-                                                   const double* x, double* yx_out, double* partial) {
+                                                   const double* x, double* yx_out, double* partial, int* np_out) {
     if (!impl_) throw UGError("GMG: not initialised");
-    return impl_->surface_axpy(y, alpha, v, beta, x, yx_out, partial);
+    return impl_->surface_axpy(y, alpha, v, beta, x, yx_out, partial, np_out);
 }
 
 bool AssembledMultiGridCycle::init(std::shared_ptr<MatrixOperator> J) {

@@ -642,7 +642,8 @@ __global__ __launch_bounds__(256) void k_nonzero_partial(int64_t n, const double
 // one workgroup of 1024: thread t sums partial[t], partial[t + 1024], ... in
 // that order (eight loads in flight), then the waves and the 16 wave sums are
 // combined in a fixed order, so the result does not depend on timing
-__global__ __launch_bounds__(1024) void k_sum_partials(int np, const double* partial, double* out, int sqrt_flag) {
+// the sum of np partials by a workgroup of 1024, in its thread 0
+__device__ __forceinline__ double sum_1024(int np, const double* __restrict__ partial) {
     double s = 0.0;
     int i = threadIdx.x;
     for (; i + 7 * 1024 < np; i += 8 * 1024) {
@@ -657,34 +658,63 @@ __global__ __launch_bounds__(1024) void k_sum_partials(int np, const double* par
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double r = 0.0;
+    double r = 0.0;
+    if (threadIdx.x == 0)
         for (int w = 0; w < 16; ++w) r += sh[w];
-        out[0] = sqrt_flag ? sqrt(r) : r;
-    }
+    return r;
+}
+__global__ __launch_bounds__(1024) void k_sum_partials(int np, const double* partial, double* out, int sqrt_flag) {
+    const double r = sum_1024(np, partial);
+    if (threadIdx.x == 0) out[0] = sqrt_flag ? sqrt(r) : r;
 }
 
 // ---------------------------------------------------------------------------
 // CG building blocks with the scalars kept in device memory
-// (sc[0] rho, sc[1] lambda, sc[2] alpha, sc[3] beta, sc[4] rho_new, sc[5] |r|^2,
-//  sc[6] = 1 after a breakdown lambda == 0)
+// (sc[0] rho of the step before, sc[1] lambda, sc[2] alpha, sc[4] rho, sc[5]
+//  |r|^2, sc[6] = 1 after a breakdown lambda == 0)
+// On the small lattices a step is bound by its launches, so the scalars are
+// formed where they are used: lambda by every workgroup of the update from the
+// operator's partial sums, beta = rho / rho_old by the direction update, and the
+// kernel that sums |r|^2 keeps rho and hands the host its two values. The 33^3
+// solve: 97 us a step with a kernel for each of them and a copy, 90 so.
 // ---------------------------------------------------------------------------
-__global__ void k_cg_beta(double* sc) {
-    if (threadIdx.x != 0) return;
-    sc[3] = sc[4] / sc[0];
-    sc[0] = sc[4];
+// the sum of np partials, the same in every thread of a workgroup of 256
+__device__ __forceinline__ double block_sum_partials(int np, const double* __restrict__ partial) {
+    __shared__ double sh[4];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < np; i += 256) s += partial[i];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// |r|^2 = sum of the partials, the breakdown flag beside it in pinned host
+// memory, and rho kept for the next step
+__global__ __launch_bounds__(1024) void k_cg_norm(int np, const double* __restrict__ partial, double* __restrict__ sc,
+                                                  double* __restrict__ host) {
+    const double s = sum_1024(np, partial);
+    if (threadIdx.x == 0) {
+        sc[5] = s;
+        sc[0] = sc[4];
+        host[0] = s;
+        host[1] = sc[6];
+    }
 }
 
 // alpha = rho / lambda (0, with the breakdown flag, when lambda == 0), formed
-// by every thread and recorded by the first; x += alpha p ; r -= alpha q ;
+// by every thread and recorded by the first (lambda: the sum of nl partials,
+// or sc[1] where nl is 0); x += alpha p ; r -= alpha q ;
 // partial sums of r.r
 __global__ __launch_bounds__(256) void k_cg_update(int64_t n, double* __restrict__ sc,
                                                    const double* __restrict__ p, const double* __restrict__ q,
                                                    double* __restrict__ x, double* __restrict__ r,
-                                                   double* __restrict__ partial, float* __restrict__ rf) {
-    const double lambda = sc[1];
-    const double alpha = lambda == 0.0 ? 0.0 : sc[0] / lambda;
+                                                   double* __restrict__ partial, float* __restrict__ rf, int nl,
+                                                   const double* __restrict__ lpart) {
+    const double lambda = nl > 0 ? block_sum_partials(nl, lpart) : sc[1];
+    const double alpha = lambda == 0.0 ? 0.0 : sc[4] / lambda;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (nl > 0) sc[1] = lambda;
         sc[2] = alpha;
         if (lambda == 0.0) sc[6] = 1.0;
     }
@@ -717,7 +747,7 @@ __global__ __launch_bounds__(256) void k_cg_update(int64_t n, double* __restrict
 // p = beta p + z
 __global__ __launch_bounds__(256) void k_cg_direction(int64_t n, const double* __restrict__ sc, double* __restrict__ p,
                                                       const double* __restrict__ z) {
-    const double beta = sc[3];
+    const double beta = sc[4] / sc[0];
     UGX_STREAM_LOOP(n) {
         double pv[kStreamE], zv[kStreamE];
 #pragma unroll
@@ -2165,17 +2195,17 @@ int sum_partials(int np, const double* partial, double* out, hipStream_t s) {
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, np, partial, out, 0);
     UGX_CHECK_LAUNCH();
 }
-int cg_beta(double* sc, hipStream_t s) {
-    hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(64), 0, s, sc);
-    UGX_CHECK_LAUNCH();
-}
 int cg_update(int64_t n, double* sc, const double* p, const double* q, double* x, double* r, double* partial,
-              hipStream_t s, float* rf) {
+              double* host, hipStream_t s, float* rf, int nl, const double* lpart) {
     const int g = red_grid(n);
-    hipLaunchKernelGGL(k_cg_update, dim3(g), dim3(256), 0, s, n, sc, p, q, x, r, partial, rf);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, g, partial, sc + 5, 0);
+    hipLaunchKernelGGL(k_cg_update, dim3(g), dim3(256), 0, s, n, sc, p, q, x, r, partial, rf, nl, lpart);
+    hipLaunchKernelGGL(k_cg_norm, dim3(1), dim3(1024), 0, s, g, partial, sc, host);
     UGX_CHECK_LAUNCH();
 }
+// every workgroup of the update reads the partials again. One MI355X: 65^3
+// (580,000 reads) 6.9 us against 5.6 with a sum of 3.0 before it; 129^3 (4.3
+// million) 21.1 against 18.1 and 4.1, no gain
+bool cg_update_sums(int64_t n, int nl) { return (int64_t)red_grid(n) * nl <= (1 << 20); }
 int cg_direction(int64_t n, const double* sc, double* p, const double* z, hipStream_t s) {
     hipLaunchKernelGGL(k_cg_direction, dim3(stream_grid(n)), dim3(256), 0, s, n, sc, p, z);
     UGX_CHECK_LAUNCH();

@@ -33,7 +33,8 @@ namespace {
 //         correction: sd = (T)d64, st = dinv.*sd; sd_out = sd - A st; sc = st
 // MODE 4: the same from a defect already in T (b = sd)
 // MODE 5: the CG direction update fused with the operator: staged
-//         p_new = fma(beta, p_old, z) (a = p_old, b = z, beta = *d64),
+//         p_new = fma(beta, p_old, z) (a = p_old, b = z, beta = *d64, or
+//         *d64 / *c where c is given),
 //         out1 = p_new, out0 = y = A p_new, partials of (y, p_new)
 // MODE 7: the last post-smoothing step of a cycle fused with the correction
 //         update that ends it, its conversion and the (z, r) partials: MODE 0
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(256) void k_q1mf_direct(int W, int64_t nblocks, Q1A
     const int i = (int)(lb * 256) + (int)threadIdx.x;
     double dot = 0.0;
     if (i < W2 * W) {
-        const T bcg = MODE == 5 ? (T)*q.d64 : (T)0;
+        const T bcg = MODE == 5 ? (T)(q.c ? *q.d64 / (double)*q.c : *q.d64) : (T)0;
         const int yz = i / W, x = i - yz * W, z = yz / W, y = yz - z * W;
         RowIn<T> in{};
         load_row<T, MODE>(q, i, true, in);
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(256) void k_q1mf_march(MarchMap m, Q1Args<T> q) {
         const int j0 = (m.glo[xcd] + slot - chunk * g) * TY;
         const int k0 = (int)((int64_t)chunk * W / m.nchunks), k1 = (int)((int64_t)(chunk + 1) * W / m.nchunks);
         const int tid = threadIdx.x, tx = tid & (NX - 1), tg = tid >> SH;
-        const T bcg = MODE == 5 ? (T)*q.d64 : (T)0;
+        const T bcg = MODE == 5 ? (T)(q.c ? *q.d64 / (double)*q.c : *q.d64) : (T)0;
         // staging: slot u of a thread is column tx of line tg + u G (lattice
         // line j0 - 1 + that); the lines' last column by the first NL threads
         const int sy = j0 - 1 + tg;
@@ -589,13 +590,13 @@ template int q1mf_axpy<double>(int, const double*, double, const double*, double
 // p_new must not alias p_old (other workgroups still stage p_old)
 template <typename T>
 int q1mf_direction_axpy(int W, const T* cell, const T* p_old, const T* z, const double* beta_dev, T* p_new, T* y,
-                        hipStream_t s, double* dot_partial, int* n_partial) {
+                        hipStream_t s, double* dot_partial, int* n_partial, const double* rho_old) {
     if (p_new == p_old || !dot_partial || !n_partial) return -1;
-    return q1mf_launch<T, 5>(W, Q1Args<T>{cell, p_old, z, nullptr, y, p_new, 0.0, 1.0, dot_partial, beta_dev, nullptr, nullptr},
+    return q1mf_launch<T, 5>(W, Q1Args<T>{cell, p_old, z, rho_old, y, p_new, 0.0, 1.0, dot_partial, beta_dev, nullptr, nullptr},
                              s, n_partial);
 }
 template int q1mf_direction_axpy<double>(int, const double*, const double*, const double*, const double*, double*,
-                                         double*, hipStream_t, double*, int*);
+                                         double*, hipStream_t, double*, int*, const double*);
 
 // t = P c (the coarse correction, with its last update c += dinv_c .* sd_c
 // folded in where given), d -= A t, sc += t on the marching widths in FP32: the

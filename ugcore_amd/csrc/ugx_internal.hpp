@@ -57,15 +57,17 @@ int count_nonzero(int64_t n, const double* a, double* partial, double* out, hipS
 // number of partial sums dot() writes for n entries (one per workgroup of its
 // grid, at most 65536)
 int dot_partials(int64_t n);
-// CG with device scalars sc[0..6] = rho, lambda, alpha, beta, rho_new, |r|^2,
-// breakdown flag
+// CG with device scalars sc[0..6] = rho of the step before, lambda, alpha, -,
+// rho, |r|^2, breakdown flag
 int sum_partials(int np, const double* partial, double* out, hipStream_t s);
-int cg_beta(double* sc, hipStream_t s);
-// alpha = sc[0] / sc[1] into sc[2] (0 and sc[6] = 1 when sc[1] == 0), then the
+// alpha = sc[4] / sc[1] into sc[2] (0 and sc[6] = 1 when sc[1] == 0), then the
 // update; rf (nullable): also writes (float) r, the FP32 cycle's copy of the defect
+// lambda from the nl partials at lpart where nl > 0 (cg_update_sums(n, nl); not
+// in `partial`), else from sc[1]; host: pinned, takes |r|^2 and the breakdown flag
 int cg_update(int64_t n, double* sc, const double* p, const double* q, double* x, double* r, double* partial,
-              hipStream_t s,
-              float* rf = nullptr);
+              double* host, hipStream_t s, float* rf = nullptr, int nl = 0, const double* lpart = nullptr);
+bool cg_update_sums(int64_t n, int nl);
+// p = z + sc[4] / sc[0] p
 int cg_direction(int64_t n, const double* sc, double* p, const double* z, hipStream_t s);
 template <typename T>
 int convert_dot(int64_t n, const T* c, double* z, const double* r, double* partial, double* out, hipStream_t s);
@@ -122,7 +124,7 @@ int q1mf_jacobi_first(int W, const T* cell, const T* dinv, const double* d64, T*
 // p_old distinct, both with the halo
 template <typename T>
 int q1mf_direction_axpy(int W, const T* cell, const T* p_old, const T* z, const double* beta_dev, T* p_new, T* y,
-                        hipStream_t s, double* dot_partial, int* n_partial);
+                        hipStream_t s, double* dot_partial, int* n_partial, const double* rho_old = nullptr);
 // the same from a defect already in T (with the halo)
 template <typename T>
 int q1mf_jacobi_first_t(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s);
