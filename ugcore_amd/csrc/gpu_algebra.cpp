@@ -2399,6 +2399,8 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         for (auto& l : L) l.acc_deferred = false;
     }
     bool first_step_fused() const { return mf && nu1 > 0 && top > base && q1mf_fused_fits(L[top].W); }
+    // the same with the stored operator of the triangular hierarchy
+    bool first_step_stored() const { return !mf && nu1 > 0 && top > base && sym_ok && L[top].dim == 2; }
 
     void base_solve(int lev) {
         auto& c = context();
@@ -2411,7 +2413,10 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         GmgLevel<T>& f = L[lev];
         GmgLevel<T>& cl = L[lev - 1];
         for (int nu = 0; nu < nu1; ++nu) {
-            if (nu == 0 && lev == top && (first_defect || first_defect_f32)) {
+            if (nu == 0 && lev == top && first_defect && !mf) {
+                UGX_LAUNCH(dias9_first<T>((int)f.W, f.A.get(), f.dinv, first_defect, f.sd2, f.sc, c.stream));
+                first_defect = nullptr;
+            } else if (nu == 0 && lev == top && (first_defect || first_defect_f32)) {
                 if constexpr (std::is_same<T, float>::value) {
                     if (first_defect_f32)
                         UGX_LAUNCH(q1mf_jacobi_first_t<T>(f.W, cell_c.get(), f.dinv, first_defect_f32, f.sd2, f.sc,
@@ -2559,6 +2564,8 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         if (first_step_fused()) {
             first_defect = d_lat;
             if (std::is_same<T, float>::value) first_defect_f32 = d_lat_f32;
+        } else if (first_step_stored()) {
+            first_defect = d_lat;
         } else {
             UGX_LAUNCH((convert<double, T>(t.N, d_lat, t.sd, c.stream)));
             UGX_LAUNCH(vec_set<T>(t.N, t.sc, 0.0, c.stream));
@@ -2703,6 +2710,12 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
                 return true;
             }
             UGX_LAUNCH(q1mf_axpy<double>(t.W, cell_c64.get(), alpha, v, beta, x, y, c.stream));
+            return true;
+        }
+        if (yx_out && t.dim == 2 && alpha == 0.0 && beta == 1.0) {
+            int np = AssembledMultiGridCycle::max_partials();
+            if (dias9_product_dot((int)t.W, surf.get(), x, y, partial, &np, c.stream) != 0) return false;
+            keep_or_sum(np, partial, yx_out, np_out);
             return true;
         }
         if (yx_out) return false;

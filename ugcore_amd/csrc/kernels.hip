@@ -1382,9 +1382,9 @@ __global__ void k_dia_jacobi_diag(int64_t n, int nd, const TM* dia, double omega
 }
 
 // ---------------------------------------------------------------------------
-// Matrix-free P1 transfer between lattice levels (3D: hexahedra, 2D: triangles
-// with diagonals along (1,1)). Weights are the exact dyadic P entries; the
-// Dirichlet adjustment is applied exactly as on the assembled matrices.
+// Matrix-free P1 transfer between the lattice levels of hexahedra. Weights are
+// the exact dyadic P entries; the Dirichlet adjustment is applied exactly as on
+// the assembled matrices.
 // ---------------------------------------------------------------------------
 
 // prolongation with accumulation: st_f = sum_c P(f,c) sc_c ; sc_f += st_f
@@ -1404,44 +1404,30 @@ struct CoarseCorr {
 };
 
 template <typename TV>
-__global__ __launch_bounds__(256) void k_prolong_add(int dim, int Wc, int Wf, int64_t n_f, CoarseCorr<TV> scc,
+__global__ __launch_bounds__(256) void k_prolong_add(int Wc, int Wf, int64_t n_f, CoarseCorr<TV> scc,
                                                      const uint8_t* __restrict__ dir_f, TV* __restrict__ st,
                                                      TV* __restrict__ sc, FastDiv fw) {
     const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
     if (i >= n_f) return;
     const uint32_t q1 = fdiv((uint32_t)i, fw);
     const int x = (int)((uint32_t)i - q1 * (uint32_t)Wf);
-    const uint32_t q2 = dim == 3 ? fdiv(q1, fw) : 0u;
+    const uint32_t q2 = fdiv(q1, fw);
     const int y = (int)(q1 - q2 * (uint32_t)Wf);
     const int z = (int)q2;
     const int x0 = x >> 1, y0 = y >> 1, z0 = z >> 1;
     const int ox = x & 1, oy = y & 1, oz = z & 1;
     double v = 0.0;
     // Dirichlet DoFs lie on the lattice boundary: only there is the flag read
-    const bool bnd = x == 0 || y == 0 || x == Wf - 1 || y == Wf - 1 || (dim == 3 && (z == 0 || z == Wf - 1));
-    if (dim == 3) {
-        const int nodd = ox + oy + oz;
-        if (bnd && dir_f[i] && nodd != 0) {
-            v = 0.0;   // Dirichlet rows of P are zeroed except vertex copies
-        } else {
-            const double w = nodd == 0 ? 1.0 : nodd == 1 ? 0.5 : nodd == 2 ? 0.25 : 0.125;
-            for (int dz = 0; dz <= oz; ++dz)
-                for (int dy = 0; dy <= oy; ++dy)
-                    for (int dx = 0; dx <= ox; ++dx)
-                        v = fma(w, (double)scc(((int64_t)(z0 + dz) * Wc + (y0 + dy)) * Wc + (x0 + dx)), v);
-        }
+    const bool bnd = x == 0 || y == 0 || x == Wf - 1 || y == Wf - 1 || z == 0 || z == Wf - 1;
+    const int nodd = ox + oy + oz;
+    if (bnd && dir_f[i] && nodd != 0) {
+        v = 0.0;   // Dirichlet rows of P are zeroed except vertex copies
     } else {
-        // triangle mesh: odd coordinates lie on axis edges or on the (1,1) diagonal
-        const int nodd = ox + oy;
-        if (bnd && dir_f[i] && nodd != 0) {
-            v = 0.0;
-        } else if (nodd == 0) {
-            v = (double)scc((int64_t)y0 * Wc + x0);
-        } else if (nodd == 1) {
-            v = 0.5 * (double)scc((int64_t)y0 * Wc + x0) + 0.5 * (double)scc((int64_t)(y0 + oy) * Wc + (x0 + ox));
-        } else {
-            v = 0.5 * (double)scc((int64_t)y0 * Wc + x0) + 0.5 * (double)scc((int64_t)(y0 + 1) * Wc + (x0 + 1));
-        }
+        const double w = nodd == 0 ? 1.0 : nodd == 1 ? 0.5 : nodd == 2 ? 0.25 : 0.125;
+        for (int dz = 0; dz <= oz; ++dz)
+            for (int dy = 0; dy <= oy; ++dy)
+                for (int dx = 0; dx <= ox; ++dx)
+                    v = fma(w, (double)scc(((int64_t)(z0 + dz) * Wc + (y0 + dy)) * Wc + (x0 + dx)), v);
     }
     // c += t in the vector precision (mg_solver_impl.hpp:1905)
     const TV t = (TV)v;
@@ -1507,7 +1493,7 @@ __global__ __launch_bounds__(256) void k_prolong_add3(int Wc, int Wf, int64_t n_
 }
 
 template <typename TV>
-__global__ __launch_bounds__(256) void k_restrict(int dim, int Wc, int Wf, int64_t n_c, const TV* __restrict__ sdf,
+__global__ __launch_bounds__(256) void k_restrict(int Wc, int Wf, int64_t n_c, const TV* __restrict__ sdf,
                                                   const uint8_t* __restrict__ dir_c, const uint8_t* __restrict__ dir_f,
                                                   TV* __restrict__ sdc, FastDiv fw, TV* __restrict__ zc) {
     const int64_t c = blockIdx.x * (int64_t)256 + threadIdx.x;
@@ -1515,14 +1501,14 @@ __global__ __launch_bounds__(256) void k_restrict(int dim, int Wc, int Wf, int64
     if (zc) zc[c] = (TV)0;   // the coarse correction starts from zero
     const uint32_t q1 = fdiv((uint32_t)c, fw);
     const int x = (int)((uint32_t)c - q1 * (uint32_t)Wc);
-    const uint32_t q2 = dim == 3 ? fdiv(q1, fw) : 0u;
+    const uint32_t q2 = fdiv(q1, fw);
     const int y = (int)(q1 - q2 * (uint32_t)Wc);
     const int z = (int)q2;
     const int fx = 2 * x, fy = 2 * y, fz = 2 * z;
     const int nf = Wf - 1;
     // Dirichlet DoFs lie on the lattice boundary: away from it no flag is read
-    const bool inner = x >= 2 && y >= 2 && x <= Wc - 3 && y <= Wc - 3 && (dim == 2 || (z >= 2 && z <= Wc - 3));
-    if (dim == 3 && inner) {
+    const bool inner = x >= 2 && y >= 2 && x <= Wc - 3 && y <= Wc - 3 && z >= 2 && z <= Wc - 3;
+    if (inner) {
         double s = 0.0;
 #pragma unroll
         for (int dz = -1; dz <= 1; ++dz)
@@ -1538,38 +1524,25 @@ __global__ __launch_bounds__(256) void k_restrict(int dim, int Wc, int Wf, int64
         return;
     }
     if (dir_c[c]) {
-        const int64_t f = dim == 3 ? ((int64_t)fz * Wf + fy) * Wf + fx : (int64_t)fy * Wf + fx;
-        sdc[c] = sdf[f];
+        sdc[c] = sdf[((int64_t)fz * Wf + fy) * Wf + fx];
         return;
     }
     double s = 0.0;
-    if (dim == 3) {
-        for (int dz = -1; dz <= 1; ++dz) {
-            const int zz = fz + dz;
-            if (zz < 0 || zz > nf) continue;
-            for (int dy = -1; dy <= 1; ++dy) {
-                const int yy = fy + dy;
-                if (yy < 0 || yy > nf) continue;
-                for (int dx = -1; dx <= 1; ++dx) {
-                    const int xx = fx + dx;
-                    if (xx < 0 || xx > nf) continue;
-                    const int nodd = (dx != 0) + (dy != 0) + (dz != 0);
-                    const int64_t f = ((int64_t)zz * Wf + yy) * Wf + xx;
-                    if (dir_f[f] && nodd != 0) continue;   // zeroed P rows
-                    const double w = nodd == 0 ? 1.0 : nodd == 1 ? 0.5 : nodd == 2 ? 0.25 : 0.125;
-                    s += w * (double)sdf[f];
-                }
+    for (int dz = -1; dz <= 1; ++dz) {
+        const int zz = fz + dz;
+        if (zz < 0 || zz > nf) continue;
+        for (int dy = -1; dy <= 1; ++dy) {
+            const int yy = fy + dy;
+            if (yy < 0 || yy > nf) continue;
+            for (int dx = -1; dx <= 1; ++dx) {
+                const int xx = fx + dx;
+                if (xx < 0 || xx > nf) continue;
+                const int nodd = (dx != 0) + (dy != 0) + (dz != 0);
+                const int64_t f = ((int64_t)zz * Wf + yy) * Wf + xx;
+                if (dir_f[f] && nodd != 0) continue;   // zeroed P rows
+                const double w = nodd == 0 ? 1.0 : nodd == 1 ? 0.5 : nodd == 2 ? 0.25 : 0.125;
+                s += w * (double)sdf[f];
             }
-        }
-    } else {
-        const int dxs[7] = {0, 1, -1, 0, 0, 1, -1};
-        const int dys[7] = {0, 0, 0, 1, -1, 1, -1};
-        for (int k = 0; k < 7; ++k) {
-            const int xx = fx + dxs[k], yy = fy + dys[k];
-            if (xx < 0 || xx > nf || yy < 0 || yy > nf) continue;
-            const int64_t f = (int64_t)yy * Wf + xx;
-            if (dir_f[f] && k != 0) continue;
-            s += (k == 0 ? 1.0 : 0.5) * (double)sdf[f];
         }
     }
     sdc[c] = (TV)s;
@@ -2545,8 +2518,9 @@ int prolong_add(int dim, int Wc, int Wf, int64_t n_f, const TV* scc, const uint8
     if (n_f <= 0) return 0;
     if (n_f >= ((int64_t)1 << 32)) return -1;
     if ((dinv_c == nullptr) != (sd_c == nullptr)) return -1;
+    if (dim == 2) return prolong2<TV>(Wc, Wf, scc, dinv_c, sd_c, dir_f, st, sc, s);
     const CoarseCorr<TV> corr{scc, dinv_c, sd_c};
-    if (dim == 3 && Wf == 2 * Wc - 1) {
+    if (Wf == 2 * Wc - 1) {
         // measured on one MI355X within the 256^3 GMG-CG solve (both kernels
         // with XCD-grouped blocks): 129^3 -> 257^3 FP32 tiled 76 us against
         // 81 us for the per-coarse-point kernel, 65^3 -> 129^3 15 against
@@ -2566,7 +2540,7 @@ int prolong_add(int dim, int Wc, int Wf, int64_t n_f, const TV* scc, const uint8
                            sc, make_fastdiv((uint32_t)Wc));
         UGX_CHECK_LAUNCH();
     }
-    hipLaunchKernelGGL(k_prolong_add<TV>, dim3((n_f + 255) / 256), dim3(256), 0, s, dim, Wc, Wf, n_f, corr, dir_f, st,
+    hipLaunchKernelGGL(k_prolong_add<TV>, dim3((n_f + 255) / 256), dim3(256), 0, s, Wc, Wf, n_f, corr, dir_f, st,
                        sc, make_fastdiv((uint32_t)Wf));
     UGX_CHECK_LAUNCH();
 }
@@ -2614,7 +2588,8 @@ int restrict_defect(int dim, int Wc, int Wf, int64_t n_c, const TV* sdf, const u
                     TV* sdc, hipStream_t s, TV* zero_c) {
     if (n_c <= 0) return 0;
     if (n_c >= ((int64_t)1 << 32)) return -1;
-    if (dim == 3 && Wf == 2 * Wc - 1 && Wc >= 65) {
+    if (dim == 2) return restrict2<TV>(Wc, Wf, sdf, dir_c, dir_f, sdc, zero_c, s);
+    if (Wf == 2 * Wc - 1 && Wc >= 65) {
         // large levels: the z-marching restriction (short-lived staging
         // workgroups left the tiled kernel at about 1.1 TB/s at 257^3)
         RzMap rm;
@@ -2637,7 +2612,7 @@ int restrict_defect(int dim, int Wc, int Wf, int64_t n_c, const TV* sdf, const u
             UGX_CHECK_LAUNCH();
         }
     }
-    hipLaunchKernelGGL(k_restrict<TV>, dim3((n_c + 255) / 256), dim3(256), 0, s, dim, Wc, Wf, n_c, sdf, dir_c, dir_f, sdc,
+    hipLaunchKernelGGL(k_restrict<TV>, dim3((n_c + 255) / 256), dim3(256), 0, s, Wc, Wf, n_c, sdf, dir_c, dir_f, sdc,
                        make_fastdiv((uint32_t)Wc), zero_c);
     UGX_CHECK_LAUNCH();
 }

@@ -201,6 +201,20 @@ int restrict_defect(int dim, int Wc, int Wf, int64_t n_c, const TV* sdf, const u
 // x = U^{-1} L^{-1} P b with row-major triangular inverses; perm[i] = row of b
 template <typename TV>
 int lu_solve(int n, const double* LinvT, const double* UinvT, const int32_t* perm, const TV* b, TV* x, hipStream_t s);
+// ---- the triangular hierarchy's lattice kernels (lattice2d_kernels.hip) ----
+template <typename TV>
+int prolong2(int Wc, int Wf, const TV* c, const TV* dinv, const TV* sd, const uint8_t* dir_f, TV* st, TV* sc,
+             hipStream_t s);
+template <typename TV>
+int restrict2(int Wc, int Wf, const TV* sdf, const uint8_t* dir_c, const uint8_t* dir_f, TV* sdc, TV* zero_c,
+              hipStream_t s);
+// y = A x (symmetric storage) with the partial sums of (y, x); n_partial in:
+// capacity, out: number written
+int dias9_product_dot(int W, const double* U, const double* x, double* y, double* partial, int* n_partial,
+                      hipStream_t s);
+template <typename T>
+int dias9_first(int W, const T* U, const T* dinv, const double* d64, T* sd, T* sc, hipStream_t s);
+
 // what lu_solve applies, from the base operator in tiled DIA form, on the
 // device (lu_factor.hip): m rows, nd diagonals with lattice offsets off (host);
 // *singular is set where a pivot is below 1e-10 and kept otherwise
