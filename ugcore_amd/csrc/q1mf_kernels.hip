@@ -46,8 +46,10 @@ namespace {
 //         a + b .* c2 folded in), d_out = d_in - A t, sc += t: c = d_in,
 //         out0 = d_out, out1 = sc (k_q1mf_march only)
 // out0 may alias c (MODE 1, 2, 6): every row is read and then written by the same
-// thread. The rows' own inputs and outputs are nontemporal: they leave the L2
-// to the values that neighbouring rows share.
+// thread. Every access is an ordinary one: a line of 257 values begins and ends
+// inside a cache line, which the next line's wave completes, and nontemporal
+// stores sent it out in parts (1.12 - 1.15 of the bytes; 256^3 solve 8.93 ms, 8.79
+// so; 128^3 FP64 2.79 and 2.69; the rows' inputs were nontemporal too).
 template <typename T>
 struct Q1Args {
     const T* cell;
@@ -62,15 +64,6 @@ struct Q1Args {
     double* z64;
     const T* c2;
 };
-
-template <typename T>
-__device__ __forceinline__ T ldn(const T* p) {
-    return __builtin_nontemporal_load(p);
-}
-template <typename T>
-__device__ __forceinline__ void stn(T v, T* p) {
-    __builtin_nontemporal_store(v, p);
-}
 
 // the value that entry j contributes to its neighbours' rows, from its two
 // loaded parts
@@ -97,22 +90,22 @@ template <typename T, int MODE>
 __device__ __forceinline__ void load_row(const Q1Args<T>& q, int64_t i, bool ok, RowIn<T>& in) {
     if (!ok) return;
     if (MODE == 0) {
-        in.u = ldn(q.b + i);      // sd
-        in.v = ldn(q.out1 + i);   // sc
+        in.u = q.b[i];      // sd
+        in.v = q.out1[i];   // sc
     } else if (MODE == 1) {
-        in.u = ldn(q.c + i);
+        in.u = q.c[i];
     } else if (MODE == 6) {
-        in.u = ldn(q.c + i);
-        in.v = ldn(q.out1 + i);
+        in.u = q.c[i];
+        in.v = q.out1[i];
     } else if (MODE == 2) {
-        in.u = q.alpha != 0.0 ? ldn(q.c + i) : (T)0;
+        in.u = q.alpha != 0.0 ? q.c[i] : (T)0;
     } else if (MODE == 3) {
-        in.u = (T)ldn(q.d64 + i);
+        in.u = (T)q.d64[i];
     } else if (MODE == 4) {
-        in.u = ldn(q.b + i);
+        in.u = q.b[i];
     } else if (MODE == 7) {
-        in.u = ldn(q.b + i);   // sd
-        in.v = ldn(q.c + i);   // sc
+        in.u = q.b[i];   // sd
+        in.v = q.c[i];   // sc
         in.w = q.a[i];         // dinv
         in.r = q.partial ? q.d64[i] : 0.0;
     }
@@ -120,22 +113,22 @@ __device__ __forceinline__ void load_row(const Q1Args<T>& q, int64_t i, bool ok,
 template <typename T, int MODE>
 __device__ __forceinline__ void store_row(const Q1Args<T>& q, int64_t i, const RowIn<T>& in, T xi, T s, double& dot) {
     if (MODE == 0 || MODE == 6) {
-        stn(in.u - s, q.out0 + i);
-        stn(in.v + xi, q.out1 + i);
+        q.out0[i] = in.u - s;
+        q.out1[i] = in.v + xi;
     } else if (MODE == 3 || MODE == 4) {
-        stn(in.u - s, q.out0 + i);
-        stn(xi, q.out1 + i);
+        q.out0[i] = in.u - s;
+        q.out1[i] = xi;
     } else if (MODE == 1) {
-        stn(in.u - s, q.out0 + i);
+        q.out0[i] = in.u - s;
     } else if (MODE == 7) {
         const T sd = in.u - s, sc = in.v + xi;
         const double z = (double)(T)((double)sc + (double)in.w * (double)sd);
-        stn(z, q.z64 + i);
+        q.z64[i] = z;
         dot += z * in.r;
     } else {
         const T y = (T)((q.alpha == 0.0 ? 0.0 : q.alpha * (double)in.u) + q.beta * (double)s);
-        stn(y, q.out0 + i);
-        if (MODE == 5) stn(xi, q.out1 + i);
+        q.out0[i] = y;
+        if (MODE == 5) q.out1[i] = xi;
         dot += (double)y * (double)xi;
     }
 }
@@ -264,9 +257,9 @@ __global__ __launch_bounds__(256) void k_q1mf_direct(int W, int64_t nblocks, Q1A
 // at once (a chunk starts with one extra layer).
 // 257^3, one MI355X, against the schedule it replaced (two lines per workgroup
 // with rows spread over the threads, 29 LDS reads and 43 multiply-adds a row,
-// two barriers a plane): FP32 first step 101 -> 88 us, second 100 -> 100, last with
-// its conversion 143 -> 122, d -= A x 87 -> 73, FP64 direction update with the
-// operator 186 -> 164.
+// two barriers a plane): FP32 first step 101 -> 80 us, second 100 -> 99, last with
+// its conversion 143 -> 120, d -= A x 87 -> 73, FP64 direction update with the
+// operator 186 -> 160.
 struct MarchMap {
     int32_t nchunks;
     int32_t glo[8], gsz[8];   // first band and bands of every XCD
@@ -601,7 +594,7 @@ template int q1mf_direction_axpy<double>(int, const double*, const double*, cons
 // t = P c (the coarse correction, with its last update c += dinv_c .* sd_c
 // folded in where given), d -= A t, sc += t on the marching widths in FP32: the
 // prolongation's separate pass wrote t and read it back. One MI355X, 129^3 ->
-// 257^3: 72 + 73 us in two passes, 116 in this one. FP64 keeps two: the values
+// 257^3: 72 + 73 us in two passes, 111 in this one. FP64 keeps two: the values
 // around a column and their sums take the registers of a resident workgroup
 // (65^3 -> 129^3 38.6 us in two passes, 38.1 in one).
 bool q1mf_prolong_sub_fits(int W) { return W == 129 || W == 257; }
