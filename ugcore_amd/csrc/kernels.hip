@@ -2253,13 +2253,19 @@ static int64_t make_row_map(int64_t n, int nd, const int32_t* off, RowMap& m) {
 
 // LDS-staged launch plan for symmetric 27-point operators on full 3D lattices:
 // bands of TY lines, grouped per XCD. Returns the grid size, 0 if not eligible.
-static int64_t make_staged_map(int64_t n, int nd, const int32_t* off, size_t elem, StagedMap& m, size_t& lds) {
+// Lattices below min_w keep the unstaged kernels: at 65^3 the rows' 81 loads come
+// from the caches, and only the FP64 Jacobi step, with two vectors of 8 bytes
+// around every row, gains by staging (14.7 -> 12.2 us; FP32 7.2 -> 9.5, FP64
+// d -= A x 10.6 -> 11.3, one MI355X). Three lines of 65 rows fill a workgroup
+// once.
+static int64_t make_staged_map(int64_t n, int nd, const int32_t* off, size_t elem, StagedMap& m, size_t& lds,
+                               int min_w = 128) {
     if (nd != 27) return 0;
     const int64_t W = (int64_t)off[25] - off[22];
-    if (W < 128 || off[22] != W * W || n != W * W * W) return 0;
+    if (W < min_w || off[22] != W * W || n != W * W * W) return 0;
     m = StagedMap{};
     m.W = (int32_t)W;
-    m.TY = 4;
+    m.TY = W < 128 ? 3 : 4;
     const int64_t nb = (W + m.TY - 1) / m.TY;
     int32_t maxg = 0;
     for (int c = 0; c < 8; ++c) {
@@ -2391,7 +2397,7 @@ int dias_jacobi_step(int64_t n, int nd, const int32_t* off, const TM* U, const T
     StagedMap sm;
     size_t lds = 0;
     typedef typename Acc<TV>::type T;
-    if (const int64_t grid = make_staged_map(n, nd, off, sizeof(T), sm, lds)) {
+    if (const int64_t grid = make_staged_map(n, nd, off, sizeof(T), sm, lds, sizeof(T) == 8 ? 64 : 128)) {
         hipLaunchKernelGGL((k_dias27_staged_jacobi_step<TM, TV>), dim3(grid), dim3(256), lds, s, n, make_offsets(off, nd), sm, U, dinv, sd_in, sd_out, sc);
         UGX_CHECK_LAUNCH();
     }
