@@ -139,12 +139,10 @@ def bench_poisson_2d(U, seed, reps):
 
 
 def bench_q2_elements(U, seed, reps, n_cells=64):
-    """Q2 hexahedron element matrices (one element per wavefront, FP64 matrix
-    cores) for the n_cells^3 elements of a jittered lattice, k = exp(theta)
-    per element: elements/s, the HBM rate of the element-matrix output, and
-    the FP64 rate of the contraction (27 x 27 x 81 useful multiply-adds per
-    element; 63 MFMA 16x16x4 steps issued: three of the four 16 x 16 tiles of
-    the symmetric matrix, 21 steps each)"""
+    """Q2 hexahedron element matrices (FP64, sums one direction at a time) for the
+    n_cells^3 elements of a jittered lattice, k = exp(theta) per element:
+    elements/s, the HBM rate of inputs and outputs, and the FP64 rate in terms of
+    the contraction over all points (27 x 27 x 81 multiply-adds per element)"""
     rng = np.random.default_rng(seed)
     n = n_cells ** 3
     h = 1.0 / n_cells
@@ -161,8 +159,9 @@ def bench_q2_elements(U, seed, reps, n_cells=64):
     bytes_ = n * 8 * (24 + 1 + 729 + 27)
     res = {"elements": n, "ms": t * 1e3, "elements_per_s": n / t, "GBps": bytes_ / t / 1e9,
            "frac_of_8TBps": bytes_ / t / 1e9 / HBM_PEAK_GBS,
-           "useful_fp64_TFLOPs": n * 2 * 27 * 27 * 81 / t / 1e12,
-           "mfma_issued_fp64_TFLOPs": n * 63 * 16 * 16 * 4 * 2 / t / 1e12}
+           # the contraction over all points at once; the kernel sums one
+           # direction at a time, in about a seventh of these operations
+           "useful_fp64_TFLOPs": n * 2 * 27 * 27 * 81 / t / 1e12}
     log(f"[bench] Q2 element matrices {n_cells}^3: {t*1e3:.3f} ms, {res['GBps']:.0f} GB/s written+read, "
         f"{res['useful_fp64_TFLOPs']:.2f} TFLOP/s useful FP64")
     del dx, dk, ke, fe
@@ -547,7 +546,7 @@ def main():
     lat_bytes = n ** 3 * 8 + N * (8 + 8)   # matrix-free: per-element coefficient, x, y
 
     # the CG's direction update fused with its operator (the lattice CG's
-    # k_q1mf_z<double,5>): p_new = z + beta p_old, q = A p_new, (q, p_new)
+    # k_q1mf_march<double,5>): p_new = z + beta p_old, q = A p_new, (q, p_new)
     zl = U.DeviceArray(np.concatenate([np.zeros(H), np.random.default_rng(2).normal(size=N), np.zeros(H)]))
     pl2 = U.DeviceArray(np.zeros(N + 2 * H))
     beta_d = U.DeviceArray(np.array([0.5]))
@@ -602,12 +601,13 @@ def main():
                 "launch_ms": t * 1e3, "launches_per_solve": launches, "traffic": measured_traffic(kernel),
                 "measured_stream_triad_GBps": triad_gbs}
 
-    cands = [roofline("k_q1mf_z<float,0>", smooth_bytes, t_smooth, smooth_launches)]
+    mf_kernel = "k_q1mf_direct" if n < 65 else "k_q1mf_march"
+    cands = [roofline(f"{mf_kernel}<float,0>", smooth_bytes, t_smooth, smooth_launches)]
     if lattice:
-        cands.append(roofline("k_q1mf_z<double,5>", dir_bytes, t_dir, max(iters["f32"] - 1, 0)))
-        cands.append(roofline("k_q1mf_z<double,2>", lat_bytes, t_lat, 1))
+        cands.append(roofline(f"{mf_kernel}<double,5>", dir_bytes, t_dir, max(iters["f32"] - 1, 0)))
+        cands.append(roofline(f"{mf_kernel}<double,2>", lat_bytes, t_lat, 1))
     else:
-        op_kernel = {"dict": "k_dict_spmv", "sell": "k_sell_spmv<double,double>"}.get(
+        op_kernel = {"dict": "k_dict_spmv<double,false>", "sell": "k_sell_spmv<double,double,1>"}.get(
             layout, f"k_spmv_csr<double,double,{best_lanes}>")
         cands.append(roofline(op_kernel, spmv_bytes, t_spmv, iters["f32"]))
     # the kernel with the largest share of the solve
