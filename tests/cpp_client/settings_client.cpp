@@ -1,0 +1,97 @@
+// A program over the C++ interface (include/ug_gpu/gpu_algebra.hpp) for what
+// only that interface can do: settings changed between two uses of one object.
+//   settings_client base_level   a matrix multigrid whose base level is lowered
+// Prints what it compares; exit status 0 if every comparison holds.
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <memory>
+#include <vector>
+
+#include "ug_gpu/gpu_algebra.hpp"
+
+using namespace ug::gpu;
+
+namespace {
+
+std::vector<double> values(const GPUVector& v) {
+    std::vector<double> h((size_t)v.size());
+    v.download(h.data());
+    return h;
+}
+
+GPUVector vector_of(int64_t n, int seed) {
+    std::vector<double> h((size_t)n);
+    uint32_t s = 12345u + 977u * (uint32_t)seed;
+    for (auto& x : h) {
+        s = s * 1664525u + 1013904223u;
+        x = (double)(s >> 8) / (1 << 24) - 0.5;
+    }
+    GPUVector v(n);
+    v.upload(h.data());
+    return v;
+}
+
+bool equal(const char* what, const GPUVector& a, const GPUVector& b) {
+    const auto x = values(a), y = values(b);
+    bool same = x.size() == y.size();
+    for (size_t i = 0; same && i < x.size(); ++i) same = x[i] == y[i];
+    double n2 = 0.0;
+    for (double v : x) n2 += v * v;
+    std::printf("%s: %s (norm %.6e)\n", what, same ? "equal" : "DIFFERENT", std::sqrt(n2));
+    std::fflush(stdout);
+    return same && n2 > 0.0 && std::isfinite(n2);
+}
+
+// the level matrices of a Q2 hierarchy
+struct Q2Levels {
+    std::vector<std::shared_ptr<GPUSparseMatrix>> A, P, R;
+    explicit Q2Levels(int refs) {
+        Q2Discretization q(refs);
+        q.set_source(1.0);
+        for (int l = 0; l <= refs; ++l) {
+            for (auto* v : {&A, &P, &R}) v->push_back(std::make_shared<GPUSparseMatrix>());
+            GPUVector b(q.num_dofs(l));
+            q.assemble_linear(l, *A[l], b);
+            if (l == 0) continue;
+            q.prolongation(l, *P[l]);
+            q.restriction(l, *P[l], *R[l]);
+        }
+    }
+};
+
+// one object: initialised and applied with the base level `high`, then with
+// the base level `low`; the second correction is that of a new object
+bool base_level(int refs, int high, int low) {
+    Q2Levels q(refs);
+    auto J = std::make_shared<MatrixOperator>(q.A[refs]);
+    const int64_t n = q.A[refs]->num_rows();
+    const GPUVector d = vector_of(n, refs);
+    GPUVector c(n), ref(n);
+    MatrixMultiGrid g;
+    g.set_levels(q.A, q.P, q.R);
+    for (int base : {high, low, high}) {
+        g.set_base_level(base);
+        if (!g.init(J) || !g.apply(c, d)) return false;
+        MatrixMultiGrid fresh;
+        fresh.set_levels(q.A, q.P, q.R);
+        fresh.set_base_level(base);
+        if (!fresh.init(J) || !fresh.apply(ref, d)) return false;
+        char what[64];
+        std::snprintf(what, sizeof(what), "refs %d base level %d", refs, base);
+        if (!equal(what, c, ref)) return false;
+    }
+    return true;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    bool ok = false;
+    try {
+        if (argc > 1 && !std::strcmp(argv[1], "base_level")) ok = base_level(2, 1, 0) && base_level(3, 2, 0);
+    } catch (const std::exception& e) {
+        std::printf("error: %s\n", e.what());
+    }
+    return ok ? 0 : 1;
+}

@@ -195,3 +195,48 @@ def test_pybind_q2_multigrid_solve_equals_the_ctypes_path():
     assert S2.apply(x2, b2)
     assert S.steps() == S2.steps()
     assert np.array_equal(x.numpy(), x2.numpy())
+
+
+@pytest.mark.parametrize("cycle", [1, 2])
+def test_matrix_multigrid_initialised_again_with_other_sizes(cycle):
+    """the same object after its level matrices took larger (then smaller) ones
+    of another hierarchy of the same depth: every correction is, bit for bit,
+    that of a new object"""
+    print(f"case matrix multigrid initialised again cycle={cycle}", flush=True)
+    u = U()
+    rng = np.random.default_rng(cycle)
+    q = u.Q2Discretization(3)
+    q.set_theta(0.4 * rng.normal(size=8 ** 3))
+    q.set_source(1.0)
+    A, P, R, _ = q.hierarchy()
+    data = [[(m.download_csr(), m.num_cols()) if m is not None else None for m in ms] for ms in (A, P, R)]
+    mats = [[u.SparseMatrix() if l or k == 0 else None for l in range(3)] for k in range(3)]
+    G = u.MatrixMultiGrid(*mats, base_level=0, cycle=cycle)
+    for first in (0, 1, 0):
+        for k in range(3):
+            for l in range(3):
+                if mats[k][l] is not None:
+                    (rp, col, val), cols = data[k][first + l]
+                    mats[k][l].upload_csr(rp, col, val, n_cols=cols)
+        G.init(mats[0][-1])
+        F = u.MatrixMultiGrid(*mats, base_level=0, cycle=cycle)
+        F.init(mats[0][-1])
+        n = mats[0][-1].num_rows()
+        d = u.Vector(values=rng.normal(size=n))
+        c, ref = u.Vector(n), u.Vector(n)
+        for _ in range(2):
+            G.apply(c, d)
+            F.apply(ref, d)
+            assert np.array_equal(c.numpy(), ref.numpy()), first
+        assert np.linalg.norm(ref.numpy()) > 0
+
+
+def test_matrix_multigrid_base_level_lowered():
+    """another base level on the same object (an option of the C++ interface)"""
+    print("case matrix multigrid base level lowered", flush=True)
+    import os
+    import subprocess
+    client = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp_client", "_build", "settings_client")
+    r = subprocess.run([client, "base_level"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.count("equal") == 6

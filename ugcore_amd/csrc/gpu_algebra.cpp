@@ -2890,6 +2890,7 @@ bool MatrixMultiGrid::init(std::shared_ptr<MatrixOperator> J) {
     sc_.assign(top_ + 1, GPUVector());
     sd_.assign(top_ + 1, GPUVector());
     st_.assign(top_ + 1, GPUVector());
+    st2_.clear();   // fused_ready() allocates them at the new sizes
     smoother_.clear();
     smoother_.resize(top_ + 1);
     for (int l = base_; l <= top_; ++l) {
