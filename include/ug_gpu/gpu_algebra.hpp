@@ -756,6 +756,7 @@ class MatrixMultiGrid : public ILinearIterator {
     void presmooth_and_restriction(int lev);
     void prolongation_and_postsmooth(int lev);
     void base_solve(int lev);
+    void require_initialised_sizes();
     GPUSparseMatrix& Aop(int lev) { return lev == top_ ? op_->get_matrix() : *A_[lev]; }
     std::vector<std::shared_ptr<GPUSparseMatrix>> A_, P_, R_;
     int base_ = 0, top_ = -1, nu1_ = 2, nu2_ = 2, cycle_ = 1;

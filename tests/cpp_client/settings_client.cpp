@@ -81,6 +81,18 @@ bool base_level(int refs, int high, int low) {
         std::snprintf(what, sizeof(what), "refs %d base level %d", refs, base);
         if (!equal(what, c, ref)) return false;
     }
+    // another base level without a new init is refused
+    for (int base : {low, refs + 1, -1}) {
+        g.set_base_level(base);
+        bool refused = false;
+        try {
+            g.apply(c, d);
+        } catch (const UGError&) {
+            refused = true;
+        }
+        std::printf("base level %d without init: %s\n", base, refused ? "refused" : "ACCEPTED");
+        if (!refused) return false;
+    }
     return true;
 }
 

@@ -240,3 +240,41 @@ def test_matrix_multigrid_base_level_lowered():
     r = subprocess.run([client, "base_level"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.count("equal") == 6
+
+
+@pytest.mark.parametrize("which,level", [(0, 1), (0, 2), (1, 2), (2, 2), (1, 1)])
+def test_matrix_multigrid_refuses_levels_replaced_after_init(which, level):
+    """a level matrix (0: operator, 1: prolongation, 2: restriction) replaced by
+    a larger one needs a new init: apply raises and launches nothing"""
+    print(f"case matrix multigrid level replaced which={which} level={level}", flush=True)
+    u = U()
+    rng = np.random.default_rng(level)
+    q = u.Q2Discretization(3)
+    q.set_source(1.0)
+    A, P, R, _ = q.hierarchy()
+    mats = [[u.SparseMatrix() if l or k == 0 else None for l in range(3)] for k in range(3)]
+
+    def fill(k, l, shift):
+        m = (A, P, R)[k][l + shift]
+        rp, col, val = m.download_csr()
+        mats[k][l].upload_csr(rp, col, val, n_cols=m.num_cols())
+
+    for k in range(3):
+        for l in range(3):
+            if mats[k][l] is not None:
+                fill(k, l, 0)
+    G = u.MatrixMultiGrid(*mats, base_level=0)
+    G.init(mats[0][-1])
+    n = mats[0][-1].num_rows()
+    d, c = u.Vector(values=rng.normal(size=n)), u.Vector(n)
+    G.apply(c, d)
+    want = c.numpy()
+    fill(which, level, 1)
+    c.set(-7.0)
+    with pytest.raises(u.UGError):
+        G.apply(c, d)
+    assert np.all(c.numpy() == -7.0)
+    fill(which, level, 0)
+    G.init(mats[0][-1])
+    G.apply(c, d)
+    assert np.array_equal(c.numpy(), want)

@@ -2927,6 +2927,7 @@ bool MatrixMultiGrid::init(std::shared_ptr<MatrixOperator> J) {
 
 bool MatrixMultiGrid::apply(GPUVector& c, const GPUVector& d) {
     if (top_ < 0 || (int)sc_.size() != top_ + 1) throw UGError("MatrixMultiGrid: not initialised");
+    require_initialised_sizes();
     if (d.size() != sd_[top_].size() || c.size() != sd_[top_].size()) throw UGError("GMG::apply: size mismatch");
     // mg_solver_impl.hpp:175-275
     if (&c != &d && top_ > base_ && fused_ready()) {
@@ -2946,6 +2947,19 @@ bool MatrixMultiGrid::apply(GPUVector& c, const GPUVector& d) {
     lmgc(top_, cycle_);
     c += sc_[top_];
     return true;
+}
+
+// The level vectors, smoothers and base factors are of the sizes that init()
+// found: a level matrix replaced since by one of another size, or another base
+// level, needs a new init(). The fused products check nothing themselves.
+void MatrixMultiGrid::require_initialised_sizes() {
+    bool ok = op_ && base_ >= 0 && base_ <= top_ && lu_n_ == sd_[base_].size();
+    for (int l = base_ + 1; ok && l <= top_; ++l) {
+        const int64_t n = sd_[l].size(), nc = sd_[l - 1].size();
+        ok = smoother_[l] && P_[l] && R_[l] && Aop(l).num_rows() == n && Aop(l).num_cols() == n &&
+             P_[l]->num_rows() == n && P_[l]->num_cols() == nc && R_[l]->num_rows() == nc && R_[l]->num_cols() == n;
+    }
+    if (!ok) throw UGError("MatrixMultiGrid::apply: size mismatch, a level or the base level changed after init");
 }
 
 bool MatrixMultiGrid::fused_ready() {
