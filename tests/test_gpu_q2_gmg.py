@@ -278,3 +278,52 @@ def test_matrix_multigrid_refuses_levels_replaced_after_init(which, level):
     G.init(mats[0][-1])
     G.apply(c, d)
     assert np.array_equal(c.numpy(), want)
+
+
+def test_restriction_with_an_empty_row_adds_nothing():
+    """a coarse DoF that nothing is restricted to keeps its level's defect
+    (apply_ignore_zero_rows), which is zero after init, whatever the memory of
+    that vector held before"""
+    print("case matrix multigrid empty restriction row", flush=True)
+    u = U()
+    import scipy.sparse as sp
+    rng = np.random.default_rng(4)
+    sizes = [9, 19, 39]
+    mats = [[None] * 3 for _ in range(3)]
+
+    def up(M):
+        M = M.tocsr()
+        M.sort_indices()
+        m = u.SparseMatrix()
+        m.upload_csr(M.indptr, M.indices, M.data, n_cols=M.shape[1])
+        return m
+
+    csr = [sp.diags([-np.ones(n - 1), 2.5 * np.ones(n), -np.ones(n - 1)], [-1, 0, 1]) for n in sizes]
+    for l, n in enumerate(sizes):
+        mats[0][l] = up(csr[l])
+        if l:
+            m = sizes[l - 1]
+            Pm = sp.lil_matrix((n, m))
+            for j in range(m):
+                Pm[2 * j + 1, j] = 1.0
+                Pm[2 * j, j] = Pm[2 * j + 2, j] = 0.5
+            Rm = Pm.T.tocsr()
+            Rm.data[Rm.indptr[3]:Rm.indptr[4]] = 0.0
+            Rm.eliminate_zeros()
+            mats[1][l], mats[2][l] = up(Pm), up(Rm)
+    dv = rng.normal(size=sizes[-1])
+    got = []
+    for layout in ("sell", "csr"):          # the fused and the separate steps
+        mats[1][2].set_spmv_layout(layout)
+        for value in (0.0, np.nan, 3.0):
+            old = [u.Vector(values=np.full(n, value)) for n in sizes for _ in range(8)]
+            u.synchronize()
+            del old                         # what the next buffers of these sizes hold
+            G = u.MatrixMultiGrid(*mats, base_level=0)
+            G.init(mats[0][-1])
+            c = u.Vector(sizes[-1])
+            G.apply(c, u.Vector(values=dv))
+            got.append(c.numpy())
+    for g in got[1:]:
+        assert np.linalg.norm(g - got[0]) <= 1e-13 * np.linalg.norm(got[0])
+    assert np.linalg.norm(got[0]) > 0

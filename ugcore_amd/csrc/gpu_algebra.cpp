@@ -2896,6 +2896,7 @@ bool MatrixMultiGrid::init(std::shared_ptr<MatrixOperator> J) {
     for (int l = base_; l <= top_; ++l) {
         sc_[l].resize(rows(l));
         sd_[l].resize(rows(l));
+        sd_[l].set(0.0);   // rows that no restriction writes keep it
         st_[l].resize(rows(l));
         if (l > base_) {
             smoother_[l].reset(new Jacobi(omega_));
