@@ -849,7 +849,9 @@ class AssembledMultiGridCycle : public ILinearIterator {
     // (any entries, the correction zeroed) into `correction`, both N entries
     // in the precision of the levels.
     bool krylov_ready(const GPUSparseMatrix& A) const;
-    Precision precision() const { return prec_; }
+    // of the levels as init() made them (a later set_precision counts from the
+    // next init on)
+    Precision precision() const;
     void krylov_buffers(void*& defect, void*& correction);
     void krylov_cycle();
     int64_t lattice_size() const;

@@ -1,6 +1,8 @@
 // A program over the C++ interface (include/ug_gpu/gpu_algebra.hpp) for what
 // only that interface can do: settings changed between two uses of one object.
 //   settings_client base_level   a matrix multigrid whose base level is lowered
+//   settings_client precision    a multigrid whose precision is set after init,
+//                                in a BiCGStab solve
 // Prints what it compares; exit status 0 if every comparison holds.
 #include <cmath>
 #include <cstdio>
@@ -96,12 +98,45 @@ bool base_level(int refs, int high, int low) {
     return true;
 }
 
+// the precision set on the multigrid after init counts from the next init on:
+// the solve in between is the one before it, the one behind it that of a new
+// multigrid of that precision
+bool precision(int refs, Precision from, Precision to) {
+    auto disc = std::make_shared<DomainDiscretization>(2, refs);
+    disc->set_velocity(20.0, 10.0, 5.0);
+    auto A = std::make_shared<GPUSparseMatrix>();
+    GPUVector b;
+    disc->assemble_linear(*A, b);
+    auto J = std::make_shared<MatrixOperator>(A);
+    auto gmg = std::make_shared<AssembledMultiGridCycle>(disc);
+    gmg->set_precision(from);
+    BiCGStab S;
+    S.set_preconditioner(gmg);
+    if (!S.init(J)) return false;
+    GPUVector x(b.size()), y(b.size());
+    auto solve = [&](BiCGStab& s, GPUVector& v) {
+        v.set(0.0);
+        return s.apply(v, b);
+    };
+    if (!solve(S, x)) return false;
+    gmg->set_precision(to);
+    if (gmg->precision() != from || !solve(S, y) || !equal("precision set, no init", x, y)) return false;
+    if (!S.init(J) || gmg->precision() != to || !solve(S, y)) return false;
+    auto fresh = std::make_shared<AssembledMultiGridCycle>(disc);
+    fresh->set_precision(to);
+    BiCGStab F;
+    F.set_preconditioner(fresh);
+    return F.init(J) && solve(F, x) && equal("precision after init", x, y);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     bool ok = false;
     try {
         if (argc > 1 && !std::strcmp(argv[1], "base_level")) ok = base_level(2, 1, 0) && base_level(3, 2, 0);
+        if (argc > 1 && !std::strcmp(argv[1], "precision"))
+            ok = precision(1, Precision::F32, Precision::F64) && precision(2, Precision::F64, Precision::F32);
     } catch (const std::exception& e) {
         std::printf("error: %s\n", e.what());
     }

@@ -99,3 +99,15 @@ def test_limits_and_non_finite_defects():
     bad[3] = np.nan
     assert not S.apply(u.Vector(N), u.Vector(values=bad))
     assert S.steps() <= 1
+
+
+def test_precision_set_after_init():
+    """counts from the next init on (the C++ interface's setter)"""
+    print("case bicgstab precision set after init", flush=True)
+    sys.stdout.flush()
+    import os
+    import subprocess
+    client = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp_client", "_build", "settings_client")
+    r = subprocess.run([client, "precision"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.count("equal") == 4

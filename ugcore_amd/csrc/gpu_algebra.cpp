@@ -1999,6 +1999,7 @@ struct AssembledMultiGridCycle::Impl {
     virtual void apply_lattice(double* c_lat, const double* d_lat, double* cd_out, double* partial,
                                const float* d_lat_f32) = 0;
     virtual bool uses_f32_defect() const = 0;
+    virtual Precision precision() const = 0;
     virtual void cycle_buffers(void*& defect, void*& correction) = 0;
     virtual void run_cycle() = 0;
     virtual bool surface_axpy(double* y, double alpha, const double* v, double beta, const double* x, double* yx_out,
@@ -2642,6 +2643,8 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         UGX_HIP(hipGraphLaunch(exec, c.stream));
     }
 
+    Precision precision() const override { return std::is_same<T, float>::value ? Precision::F32 : Precision::F64; }
+
     void cycle_buffers(void*& defect, void*& correction) override {
         if (!cycle_in) cycle_in = L[top].sd;
         defect = cycle_in;
@@ -2791,6 +2794,7 @@ bool AssembledMultiGridCycle::krylov_ready(const GPUSparseMatrix& A) const {
     return impl_ && !transposed_ && !disc_->symmetric() && mat_ == &A && A.version() == mat_version_ &&
            A.origin() == disc_.get();
 }
+Precision AssembledMultiGridCycle::precision() const { return impl_ ? impl_->precision() : prec_; }
 void AssembledMultiGridCycle::krylov_buffers(void*& defect, void*& correction) {
     if (!impl_) throw UGError("GMG: not initialised");
     impl_->cycle_buffers(defect, correction);
