@@ -63,3 +63,25 @@ def test_breakdown_leaves_the_solution():
     x = u.Vector(n)
     assert not S.apply(x, u.Vector(values=np.ones(n)))
     assert not x.numpy().any()
+
+
+@pytest.mark.parametrize("rows,cols", [(40, 70), (40, 41)])
+def test_rectangular_operator_is_refused(rows, cols):
+    """a Jacobi-preconditioned CG on a matrix with more columns than rows: the
+    product z.r of vectors of different lengths is an error"""
+    print(f"case cg rectangular {rows}x{cols}", flush=True)
+    import ugcore_amd as u
+    rng = np.random.default_rng(rows)
+    M = np.zeros((rows, cols))
+    M[np.arange(rows), np.arange(rows)] = 4.0
+    M[np.arange(rows), (np.arange(rows) + 1) % cols] = -1.0
+    c = np.argsort(M == 0, axis=1, kind="stable")[:, :2]
+    c.sort(axis=1)
+    A = u.SparseMatrix()
+    A.upload_csr(2 * np.arange(rows + 1), c.reshape(-1), np.take_along_axis(M, c, 1).reshape(-1), n_cols=cols)
+    S = u.CG(u.Jacobi(1.0), max_steps=20)
+    S.init(A)
+    x = u.Vector(cols)
+    with pytest.raises(u.UGError):
+        S.apply(x, u.Vector(values=rng.normal(size=rows)))
+    assert not x.numpy().any()

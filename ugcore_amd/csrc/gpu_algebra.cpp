@@ -1113,6 +1113,7 @@ bool CG::apply_return_defect(GPUVector& x, GPUVector& b) {
     }
     conv_->set_name(name());
     conv_->start(r);
+    if (z.size() != n) throw UGError("CG: size mismatch of solution and right-hand side");   // a rectangular operator
     p = z;
     UGX_LAUNCH(dot<double>(n, z.data(), r.data(), c.red_partial, sc + 4, false, c.stream));
     while (!conv_->iteration_ended()) {
