@@ -293,85 +293,10 @@ __global__ __launch_bounds__(64) void k_dict_values(int64_t nrows, const int32_t
     }
 }
 
-// y = alpha*v1 + beta*A*x (mode 0), or y = beta*A*x on rows with entries
-// (mode 1); one wave per slice, four slices per workgroup.
-// Bound by HBM: 9 bytes per entry and the dictionaries (257^3 Q1 operator 988 us
-// on one MI355X).
-// DOTS (mode 0): also the workgroup's partial sums of (y, u) and (y, y), in
-// part[block] and part[blocks + block]. x may be FP32 (converted as it is
-// staged); dict and order may number the columns and rows differently from
-// the matrix's own numbering (order and x, y then share that numbering). These
-// are the products of a solver's step on operators that stay in the caches, where
-// latency counts: the first kPre entries of every row and the row numbers are
-// requested before the dictionary and x (a chain of three dependent loads and a
-// barrier that the values do not depend on), and consecutive slices run on one
-// XCD, whose L2 then holds the x values that neighbouring lattice blocks share
-// (97^3 tetrahedral rows 41 us without the two, 37 us with them and the partials;
-// the product at the stream's rate loses by them, 988 -> 995 us).
-template <typename XT, bool DOTS>
-__global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslices, const int32_t* __restrict__ width,
-                                                   const int32_t* __restrict__ dptr, const int32_t* __restrict__ dict,
-                                                   const int64_t* __restrict__ vptr, const int64_t* __restrict__ iptr,
-                                                   const double* __restrict__ sval, const uint32_t* __restrict__ sidx,
-                                                   const int32_t* __restrict__ order, double alpha, const double* v1,
-                                                   double beta, const XT* __restrict__ x, double* y, int mode,
-                                                   const int32_t* __restrict__ rowptr, int64_t per_xcd,
-                                                   const double* __restrict__ u, double* __restrict__ part) {
-    __shared__ double xl[4][256];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t lb =
-        DOTS && per_xcd ? (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
-    const int64_t t = lb * 4 + wave;
-    double* xs = xl[wave];
-    const bool live = t < nslices;
-    int w = 0;
-    const dbl2* vp = reinterpret_cast<const dbl2*>(sval) + lane;
-    const uint32_t* ip = sidx + lane;
-    int32_t r = -1;
-    if (DOTS && live) {
-        w = width[t];
-        vp = reinterpret_cast<const dbl2*>(sval + vptr[t]) + lane;
-        ip += iptr[t];
-        r = order[t * 64 + lane];
-    }
-    constexpr int kPre = 8;
-    uint32_t pw[kPre / 4];
-    dbl2 pv[kPre / 2];
-    const bool pre = DOTS && w >= kPre;   // the same for every lane of the wave
-    if (pre) {
-#pragma unroll
-        for (int q = 0; q < kPre / 4; ++q) pw[q] = __builtin_nontemporal_load(ip + 64 * q);
-#pragma unroll
-        for (int q = 0; q < kPre / 2; ++q) pv[q] = __builtin_nontemporal_load(vp + 64 * q);
-    }
-    if (live) {
-        const int32_t d0 = dptr[t], nd = dptr[t + 1] - d0;
-        for (int j = lane; j < nd; j += 64) xs[j] = (double)x[dict[d0 + j]];
-        if (lane == 0) xs[255] = 0.0;
-        if (!DOTS) w = width[t];
-    }
-    bool mine = r >= 0 && r < nrows;
-    double ur = 0.0;
-    if (DOTS) ur = mine ? u[r] : 0.0;
-    __syncthreads();
-    if (!DOTS) {
-        if (!live) return;
-        vp = reinterpret_cast<const dbl2*>(sval + vptr[t]) + lane;
-        ip += iptr[t];
-    }
-    double s0 = 0.0, s1 = 0.0;
-    int k = 0;
-    if (pre) {
-#pragma unroll
-        for (int q = 0; q < kPre / 4; ++q) {
-            const uint32_t word = pw[q];
-            s0 = fma(pv[2 * q].x, xs[word & 255u], s0);
-            s1 = fma(pv[2 * q].y, xs[(word >> 8) & 255u], s1);
-            s0 = fma(pv[2 * q + 1].x, xs[(word >> 16) & 255u], s0);
-            s1 = fma(pv[2 * q + 1].y, xs[word >> 24], s1);
-        }
-        k = kPre;
-    }
+// the sum of a lane's row from entry k (a multiple of 4) to the slice's width w,
+// on top of s0 and s1
+__device__ __forceinline__ double dict_row_sum(const dbl2* vp, const uint32_t* ip, int w, const double* xs, int k,
+                                               double s0, double s1) {
     for (; k + 4 <= w; k += 4) {
         const uint32_t word = __builtin_nontemporal_load(ip + 64 * (k >> 2));
         const dbl2 a = __builtin_nontemporal_load(vp + 64 * (k >> 1));
@@ -393,35 +318,137 @@ __global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslice
             s0 = fma(b.x, xs[(word >> 16) & 255u], s0);
         }
     }
-    const double sum = s0 + s1;
-    if (DOTS) {
-        // mode 0 without v1: y = beta A x
-        double yr = mine ? 0.0 + beta * sum : 0.0, yu = yr * ur, yy = yr * yr;
-        if (mine) y[r] = yr;
-        for (int o = 32; o > 0; o >>= 1) {
-            yu += __shfl_down(yu, o, 64);
-            yy += __shfl_down(yy, o, 64);
-        }
-        __shared__ double sh[2][4];
-        if (lane == 0) {
-            sh[0][wave] = yu;
-            sh[1][wave] = yy;
-        }
-        __syncthreads();
-        if (threadIdx.x < 2) {
-            const double* q = sh[threadIdx.x];
-            part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = (q[0] + q[1]) + (q[2] + q[3]);
-        }
-        return;
+    return s0 + s1;
+}
+
+// y = alpha*v1 + beta*A*x (mode 0), or y = beta*A*x on rows with entries
+// (mode 1); one wave per slice, four slices per workgroup.
+// Bound by HBM: 9 bytes per entry and the dictionaries (257^3 Q1 operator 988 us
+// on one MI355X). A kernel of its own: as one template with the form below its
+// further arguments cost the products that stay in the caches (33^3 Q1 6.35 us
+// against 6.15, 65^3 17.15 and 16.99, 49^3 tetrahedral rows 8.09 and 7.92).
+__global__ __launch_bounds__(256) void k_dict_spmv(int64_t nrows, int64_t nslices, const int32_t* __restrict__ width,
+                                                   const int32_t* __restrict__ dptr, const int32_t* __restrict__ dict,
+                                                   const int64_t* __restrict__ vptr, const int64_t* __restrict__ iptr,
+                                                   const double* __restrict__ sval, const uint32_t* __restrict__ sidx,
+                                                   const int32_t* __restrict__ order, double alpha, const double* v1,
+                                                   double beta, const double* __restrict__ x, double* y, int mode,
+                                                   const int32_t* __restrict__ rowptr) {
+    __shared__ double xl[4][256];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t t = (int64_t)blockIdx.x * 4 + wave;
+    double* xs = xl[wave];
+    int w = 0;
+    if (t < nslices) {
+        const int32_t d0 = dptr[t], nd = dptr[t + 1] - d0;
+        for (int j = lane; j < nd; j += 64) xs[j] = x[dict[d0 + j]];
+        if (lane == 0) xs[255] = 0.0;
+        w = width[t];
     }
-    r = order[t * 64 + lane];
-    mine = r >= 0 && r < nrows;
-    if (!mine) return;
+    __syncthreads();
+    if (t >= nslices) return;
+    const dbl2* vp = reinterpret_cast<const dbl2*>(sval + vptr[t]) + lane;
+    const uint32_t* ip = sidx + iptr[t] + lane;
+    const double sum = dict_row_sum(vp, ip, w, xs, 0, 0.0, 0.0);
+    const int32_t r = order[t * 64 + lane];
+    if (r < 0 || r >= nrows) return;
     if (mode == 1) {
         if (rowptr[r + 1] > rowptr[r]) y[r] = beta * sum;
     } else {
         const double base = (alpha == 0.0) ? 0.0 : alpha * v1[r];
         y[r] = base + beta * sum;
+    }
+}
+
+// y = A x with the workgroup's partial sums of (y, u) and (y, y), in part[block]
+// and part[blocks + block]. x may be FP32 (converted as it is staged); dict and
+// order may number the columns and rows differently from the matrix's own
+// numbering (order and x, y then share that numbering). These are the products
+// of a solver's step on operators that stay in the caches, where latency counts:
+// the first kPre entries of every row and the row numbers are requested before
+// the dictionary and x (a chain of three dependent loads and a barrier that the
+// values do not depend on), and consecutive slices run on one XCD, whose L2 then
+// holds the x values that neighbouring lattice blocks share (97^3 tetrahedral
+// rows, one MI355X: 41 us without the two, 37 us with them and the partials; the
+// product at the stream's rate loses by them, 988 -> 995 us, so k_dict_spmv has
+// neither).
+template <typename XT>
+__global__ __launch_bounds__(256) void k_dict_spmv_dots(int64_t nrows, int64_t nslices,
+                                                        const int32_t* __restrict__ width,
+                                                        const int32_t* __restrict__ dptr,
+                                                        const int32_t* __restrict__ dict,
+                                                        const int64_t* __restrict__ vptr,
+                                                        const int64_t* __restrict__ iptr,
+                                                        const double* __restrict__ sval,
+                                                        const uint32_t* __restrict__ sidx,
+                                                        const int32_t* __restrict__ order,
+                                                        const XT* __restrict__ x, double* __restrict__ y,
+                                                        int64_t per_xcd, const double* __restrict__ u,
+                                                        double* __restrict__ part) {
+    __shared__ double xl[4][256];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t lb = per_xcd ? (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
+    const int64_t t = lb * 4 + wave;
+    double* xs = xl[wave];
+    const bool live = t < nslices;
+    int w = 0;
+    const dbl2* vp = reinterpret_cast<const dbl2*>(sval) + lane;
+    const uint32_t* ip = sidx + lane;
+    int32_t r = -1;
+    if (live) {
+        w = width[t];
+        vp = reinterpret_cast<const dbl2*>(sval + vptr[t]) + lane;
+        ip += iptr[t];
+        r = order[t * 64 + lane];
+    }
+    constexpr int kPre = 8;
+    uint32_t pw[kPre / 4];
+    dbl2 pv[kPre / 2];
+    const bool pre = w >= kPre;   // the same for every lane of the wave
+    if (pre) {
+#pragma unroll
+        for (int q = 0; q < kPre / 4; ++q) pw[q] = __builtin_nontemporal_load(ip + 64 * q);
+#pragma unroll
+        for (int q = 0; q < kPre / 2; ++q) pv[q] = __builtin_nontemporal_load(vp + 64 * q);
+    }
+    if (live) {
+        const int32_t d0 = dptr[t], nd = dptr[t + 1] - d0;
+        for (int j = lane; j < nd; j += 64) xs[j] = (double)x[dict[d0 + j]];
+        if (lane == 0) xs[255] = 0.0;
+    }
+    const bool mine = r >= 0 && r < nrows;
+    const double ur = mine ? u[r] : 0.0;
+    __syncthreads();
+    double s0 = 0.0, s1 = 0.0;
+    int k = 0;
+    if (pre) {
+#pragma unroll
+        for (int q = 0; q < kPre / 4; ++q) {
+            const uint32_t word = pw[q];
+            s0 = fma(pv[2 * q].x, xs[word & 255u], s0);
+            s1 = fma(pv[2 * q].y, xs[(word >> 8) & 255u], s1);
+            s0 = fma(pv[2 * q + 1].x, xs[(word >> 16) & 255u], s0);
+            s1 = fma(pv[2 * q + 1].y, xs[word >> 24], s1);
+        }
+        k = kPre;
+    }
+    const double sum = dict_row_sum(vp, ip, w, xs, k, s0, s1);
+    const double yr = mine ? 0.0 + sum : 0.0;
+    double yu = yr * ur, yy = yr * yr;
+    if (mine) y[r] = yr;
+    for (int o = 32; o > 0; o >>= 1) {
+        yu += __shfl_down(yu, o, 64);
+        yy += __shfl_down(yy, o, 64);
+    }
+    __shared__ double sh[2][4];
+    if (lane == 0) {
+        sh[0][wave] = yu;
+        sh[1][wave] = yy;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const double* q = sh[threadIdx.x];
+        part[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = (q[0] + q[1]) + (q[2] + q[3]);
     }
 }
 
@@ -633,9 +660,8 @@ int dict_spmv(int64_t nrows, int64_t nslices, const int32_t* width, const int32_
               const int32_t* order, double alpha, const double* v1, double beta, const double* x, double* y, int mode,
               const int32_t* rowptr, hipStream_t s) {
     if (nslices <= 0) return 0;
-    hipLaunchKernelGGL((k_dict_spmv<double, false>), dim3(nblk(nslices, 4)), dim3(256), 0, s, nrows, nslices, width,
-                       dptr, dict, vptr, iptr, sval, sidx, order, alpha, v1, beta, x, y, mode, rowptr, (int64_t)0,
-                       (const double*)nullptr, (double*)nullptr);
+    hipLaunchKernelGGL(k_dict_spmv, dim3(nblk(nslices, 4)), dim3(256), 0, s, nrows, nslices, width, dptr, dict, vptr,
+                       iptr, sval, sidx, order, alpha, v1, beta, x, y, mode, rowptr);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -650,9 +676,8 @@ int dict_spmv_dots(int64_t nrows, int64_t nslices, const int32_t* width, const i
                    const int32_t* order, const XT* x, double* y, const double* u, double* part, hipStream_t s) {
     if (nslices <= 0) return -1;
     const int64_t nb = (nslices + 3) / 4, per = nb >= 64 ? (nb + 7) / 8 : 0;
-    hipLaunchKernelGGL((k_dict_spmv<XT, true>), dim3((unsigned)dict_spmv_blocks(nslices)), dim3(256), 0, s, nrows,
-                       nslices, width, dptr, dict, vptr, iptr, sval, sidx, order, 0.0, (const double*)nullptr, 1.0, x,
-                       y, 0, (const int32_t*)nullptr, per, u, part);
+    hipLaunchKernelGGL(k_dict_spmv_dots<XT>, dim3((unsigned)dict_spmv_blocks(nslices)), dim3(256), 0, s, nrows,
+                       nslices, width, dptr, dict, vptr, iptr, sval, sidx, order, x, y, per, u, part);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 template int dict_spmv_dots<float>(int64_t, int64_t, const int32_t*, const int32_t*, const int32_t*, const int64_t*,
