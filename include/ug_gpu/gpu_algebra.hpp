@@ -52,6 +52,9 @@ struct DeviceContext {
 DeviceContext& context();            // initialises the device on first use
 DeviceContext* context_if_ready();   // nullptr before the first context() (allocates nothing)
 void sync();
+// returns the memory of released buffers, which the library keeps for its next
+// ones, to the device; the bytes
+int64_t trim_memory();
 
 // Device memory of the library's objects, from a pool of released blocks
 // (gpu_algebra.cpp, BlockPool). Internal buffers are used on the library's

@@ -28,6 +28,11 @@ int ugx_init(void);                                  /* selects/initialises the 
 const char* ugx_last_error(void);
 void* ugx_stream(void);                              /* the library's hipStream_t */
 int ugx_synchronize(void);
+/* The memory of released objects is kept for the next ones (at most a sixteenth
+ * of the device's). This returns all of it to the device, for allocations
+ * outside the library; the bytes, or a negative value on error. Objects in use
+ * keep theirs. */
+int64_t ugx_trim_memory(void);
 
 /* ---- device buffers and timing (plumbing for callers without a GPU framework) */
 void* ugx_malloc(int64_t bytes);

@@ -3,7 +3,8 @@
 results again and again, a vector's memory handed out anew starts at zero and
 is not written by work queued before, also when the old owner's last work was
 still running, and torch work on a vector's memory on another stream is
-finished before that memory serves another vector."""
+finished before that memory serves another vector; what is kept is bounded and
+goes back to the device on request while other objects live."""
 import sys
 
 import numpy as np
@@ -77,3 +78,42 @@ def test_work_on_another_stream_ends_before_reuse():
         w = U.Vector(n)                         # the same size: most likely the same memory
         assert not w.numpy().any()
     assert keep.size() == n
+
+
+def test_kept_memory_goes_back_on_request():
+    print("case trim memory", flush=True)
+    sys.stdout.flush()
+    import ugcore_amd as U
+    import torch
+    keep = U.Vector(1000)
+    keep.set(2.0)
+    n = 1 << 27                                 # 1 GiB
+    U.trim_memory()
+    v = U.Vector(n)
+    U.synchronize()
+    used = torch.cuda.mem_get_info()[0]
+    del v
+    assert torch.cuda.mem_get_info()[0] <= used + (n << 2)      # kept
+    assert U.trim_memory() >= 8 * n
+    # up to the chunks of a few MB that the runtime takes for itself in between
+    assert torch.cuda.mem_get_info()[0] >= used + 8 * n - (32 << 20)
+    assert U.trim_memory() == 0
+    assert np.all(keep.numpy() == 2.0)
+    w = U.Vector(n)                             # allocated anew, zero
+    assert not w.numpy().any()
+
+
+def test_the_number_of_kept_blocks_is_bounded():
+    print("case block count", flush=True)
+    sys.stdout.flush()
+    import ugcore_amd as U
+    keep = U.Vector(64)
+    U.trim_memory()
+    for _ in range(2):
+        vs = [U.Vector(64) for _ in range(1500)]
+        assert not any(v.numpy().any() for v in vs[::100])
+        for k, v in enumerate(vs):
+            v.set(float(k))
+        del vs, v
+    assert 0 < U.trim_memory() <= 512 * 512
+    assert not keep.numpy().any()

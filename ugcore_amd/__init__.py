@@ -68,6 +68,7 @@ _SIGNATURES = {
     "ugx_last_error": (C.c_char_p, []),
     "ugx_stream": (_P, []),
     "ugx_synchronize": (_I, []),
+    "ugx_trim_memory": (_I64, []),
     "ugx_malloc": (_P, [_I64]),
     "ugx_free": (_I, [_P]),
     "ugx_memcpy_htod": (_I, [_P, _P, _I64]),
@@ -265,6 +266,12 @@ def init():
 
 def synchronize():
     _check(lib().ugx_synchronize(), "ugx_synchronize")
+
+
+def trim_memory():
+    """returns the memory of released objects, which the library keeps for its
+    next ones, to the device (for torch, say); the number of bytes"""
+    return _check(lib().ugx_trim_memory(), "ugx_trim_memory")
 
 
 class DeviceArray:

@@ -129,13 +129,27 @@ int ugx_synchronize(void) {
     });
 }
 
+int64_t ugx_trim_memory(void) {
+    int64_t bytes = 0;
+    const int rc = guard([&] {
+        bytes = trim_memory();
+        return 0;
+    });
+    return rc < 0 ? rc : bytes;
+}
+
 // ---- device buffers / events ---------------------------------------------------
 
 void* ugx_malloc(int64_t bytes) {
     return guard_ptr([&] {
         context();
         void* p = nullptr;
-        if (bytes <= 0 || hipMalloc(&p, (size_t)bytes) != hipSuccess) throw UGError("ugx_malloc failed");
+        if (bytes > 0 && hipMalloc(&p, (size_t)bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            trim_memory();
+            if (hipMalloc(&p, (size_t)bytes) != hipSuccess) p = nullptr;
+        }
+        if (!p) throw UGError("ugx_malloc failed");
         return p;
     });
 }

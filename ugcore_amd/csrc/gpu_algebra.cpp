@@ -67,16 +67,21 @@ namespace {
 
 // Released blocks are kept for the next buffer of about their size instead of
 // going through hipFree and hipMalloc, which map and unmap the memory: a
-// multigrid set-up allocates and frees about 60 buffers (2 GB at 128^3), and
-// renewing operator and multigrid at 128^3 took 44.4 ms that way against
-// 3.0 ms from the pool (three problems in turn on one MI355X).
+// multigrid set-up allocates and frees about 60 buffers (2 GB at 128^3).
+// Renewing operator and multigrid at 128^3 on one MI355X, without and with the
+// pool: 9.9 and 3.0 ms where one problem is renewed again and again, 44.4 and
+// 3.0 ms where three are in turn.
 //
 // A block released by an internal buffer may still be in use by kernels
 // queued on the library's stream: later work on that stream may have it at
 // once, a shared buffer only when the stream has been waited for since (the
-// epoch of its release lies before the last wait). Kept blocks amount to at
-// most a sixteenth of the device's memory (the oldest go first), are given up
-// when hipMalloc fails, and are all returned when the last buffer is released.
+// epoch of its release lies before the last wait). What is kept belongs to
+// nobody, so it is bounded and given back: at most 512 blocks (three
+// hierarchies; the search is linear), a sixteenth of the device's memory and
+// about as much as the device has free besides (asked whenever the pool has
+// grown by a gigabyte, 3.3 us), the oldest go first; all of it where an
+// allocation of the library fails, on trim_memory(), and when the last buffer
+// is released.
 class BlockPool {
    public:
     void* take(size_t bytes, bool shared, size_t* got) {
@@ -96,7 +101,7 @@ class BlockPool {
         if (!p) {
             if (hipMalloc(&p, need) != hipSuccess) {
                 (void)hipGetLastError();
-                trim(0);
+                trim(0, 0);
                 UGX_HIP(hipMalloc(&p, need));
             }
             *got = need;
@@ -118,7 +123,20 @@ class BlockPool {
         }
         free_.push_back(Block{p, o.bytes, o.device, idle ? 0 : epoch_});
         kept_ += o.bytes;
-        trim(sizes_.empty() ? 0 : limit_);
+        size_t most = sizes_.empty() ? 0 : limit_;
+        if (most > 0 && kept_ > asked_ + kAsk) {
+            size_t fr = 0, total = 0;
+            if (hipMemGetInfo(&fr, &total) == hipSuccess && fr < kept_) most = std::min(most, (fr + kept_) / 2);
+            asked_ = kept_;
+        }
+        trim(most, kMaxBlocks);
+    }
+    // everything kept goes back to the device; the bytes
+    size_t give_back() {
+        std::lock_guard<std::mutex> lock(mu_);
+        const size_t n = kept_;
+        trim(0, 0);
+        return n;
     }
     // around a wait for the library's stream: blocks released before begin
     // have nothing pending after end
@@ -132,7 +150,7 @@ class BlockPool {
     }
 
    private:
-    static constexpr size_t kUnit = 512;
+    static constexpr size_t kUnit = 512, kMaxBlocks = 512, kAsk = (size_t)1 << 30;
     struct Block {
         void* p;
         size_t bytes;
@@ -164,20 +182,25 @@ class BlockPool {
         void* p = best->p;
         *got = best->bytes;
         kept_ -= best->bytes;
+        asked_ = std::min(asked_, kept_);
         free_.erase(best);
         return p;
     }
-    void trim(size_t most) {
-        while (kept_ > most && !free_.empty()) {
-            kept_ -= free_.front().bytes;
-            (void)hipFree(free_.front().p);   // waits for the device
-            free_.erase(free_.begin());
+    // the oldest blocks go until at most so many bytes and blocks are kept
+    void trim(size_t most, size_t blocks) {
+        size_t n = 0;
+        for (; n < free_.size() && (kept_ > most || free_.size() - n > blocks); ++n) {
+            kept_ -= free_[n].bytes;
+            (void)hipFree(free_[n].p);   // waits for the device
         }
+        free_.erase(free_.begin(), free_.begin() + (std::ptrdiff_t)n);
+        asked_ = std::min(asked_, kept_);
     }
     std::mutex mu_;
     std::vector<Block> free_;   // oldest first
     std::unordered_map<void*, Owned> sizes_;
     size_t kept_ = 0, limit_ = 0;
+    size_t asked_ = 0;   // kept_ when the device's free memory was asked for last
     uint64_t epoch_ = 1, waited_ = 1;
 };
 
@@ -195,6 +218,8 @@ void sync() {
     UGX_HIP(hipStreamSynchronize(s));
     block_pool().end_wait(e);
 }
+
+int64_t trim_memory() { return (int64_t)block_pool().give_back(); }
 
 template <typename T>
 void DeviceBuffer<T>::resize(int64_t n) {

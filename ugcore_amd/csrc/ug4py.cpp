@@ -317,6 +317,11 @@ PYBIND11_MODULE(ug4py, m) {
     static py::exception<UGError> exc(m, "UGError");
     m.def("init", [] { check(ugx_init(), "init"); });
     m.def("synchronize", [] { check(ugx_synchronize(), "synchronize"); });
+    m.def("trim_memory", [] {
+        const int64_t n = ugx_trim_memory();
+        check(n < 0 ? -1 : 0, "trim_memory");
+        return n;
+    }, "returns the memory of released objects to the device; the bytes");
     m.def("stream", [] { return (uintptr_t)ugx_stream(); }, "the library's hipStream_t");
 
     py::class_<Vector>(m, "Vector")
