@@ -547,7 +547,6 @@ class ElementDiscretization {
     DeviceBuffer<int32_t> dofs_, rowptr_, col_, dir_;
     DeviceBuffer<int32_t> order_, slot_;                   // Q2: elements by colour, slots
     DeviceBuffer<int32_t> eptr_, src_, inc_ptr_, inc_t_;   // others: lists of local entries / vertices
-    DeviceBuffer<double> ke_, fe_;                         // workspace: local matrices and vectors
     DeviceBuffer<double> coords_, kel_, kq_, f_dof_;
     std::vector<int64_t> colour_start_;
     double f_const_ = 0.0;

@@ -85,3 +85,37 @@ def test_gathered_assembly(kind, ne, hub):
         ed.assemble_defect(d, U.Vector(values=u))
         assert np.all(np.abs(d.numpy() - rd) <= (64 + m) * eps * np.maximum(sd, 1e-30))
     assert m[n - 1] == 0 and b.numpy()[n - 1] == 0.0 and d.numpy()[n - 1] == 0.0
+
+
+def test_local_matrices_are_not_kept():
+    """between assemblies the discretisation holds its mesh, its pattern and its
+    lists, not the 512 bytes per Q1 hexahedron of the local matrices"""
+    print("case element workspace", flush=True)
+    sys.stdout.flush()
+    import torch
+    import ugcore_amd as U
+    n = 64
+    W, ne = n + 1, n ** 3
+    z, y, x = np.meshgrid(*[np.arange(n)] * 3, indexing="ij")
+    at = lambda dx, dy, dz: (((z + dz) * W + y + dy) * W + x + dx).reshape(-1)
+    E = np.stack([at(*c) for c in ((0, 0, 0), (1, 0, 0), (1, 1, 0), (0, 1, 0), (0, 0, 1), (1, 0, 1), (1, 1, 1),
+                                   (0, 1, 1))], 1)
+    X = np.stack(np.meshgrid(*[np.arange(W) / n] * 3, indexing="ij")[::-1], -1).reshape(-1, 3)
+    keep = U.Vector(8)
+    ed = U.ElementDiscretization("hexahedron_q1", E, X)
+    A, b, d = U.SparseMatrix(), U.Vector(W ** 3), U.Vector(W ** 3)
+    for _ in range(2):
+        ed.assemble_linear(A, b)
+        ed.assemble_defect(d, b)
+    U.synchronize()
+    U.trim_memory()
+    with_ed = torch.cuda.mem_get_info()[0]
+    nnz = ed.nnz()
+    del ed
+    U.trim_memory()
+    held = torch.cuda.mem_get_info()[0] - with_ed
+    # element table, list of local entries, vertex lists; pattern and entry
+    # pointers; coordinates and pointers; blocks are up to 1/8 larger than asked
+    lists = ne * (4 * 8 + 4 * 64 + 4 * 8) + 8 * nnz + 32 * W ** 3
+    assert held <= 1.125 * lists + (32 << 20) < lists + 512 * ne, (held, lists)
+    assert keep.size() == 8

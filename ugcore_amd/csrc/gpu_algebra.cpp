@@ -1698,8 +1698,9 @@ void ElementDiscretization::run(double* val, double* vec, const double* u) {
                                                c.stream));
         return;
     }
-    if (val) ke_.resize(ne_ * nv_ * nv_);
-    if (vec) fe_.resize(ne_ * nv_);
+    // for this call alone: 8 nv^2 bytes per element (the set-up took six times
+    // that), back in the pool before the layout is built
+    DeviceBuffer<double> ke(val ? ne_ * nv_ * nv_ : 0), fe(vec ? ne_ * nv_ : 0);
     ugamd::ElemLaunch L;
     L.ne = ne_;
     L.dofs = dofs_.get();
@@ -1710,11 +1711,11 @@ void ElementDiscretization::run(double* val, double* vec, const double* u) {
     for (int k = 0; k < 3; ++k) L.vel[k] = vel_[k];
     L.conv = conv_ ? 1 : 0;
     L.u = u;
-    L.ke = val ? ke_.get() : nullptr;
-    L.fe = vec ? fe_.get() : nullptr;
+    L.ke = ke.get();
+    L.fe = fe.get();
     UGX_LAUNCH(elem_local(type_, L, c.stream));
-    UGX_LAUNCH(elem_gather(nnz_, eptr_.get(), src_.get(), ke_.get(), val, ndofs_, inc_ptr_.get(), inc_t_.get(),
-                           fe_.get(), vec, c.stream));
+    UGX_LAUNCH(elem_gather(nnz_, eptr_.get(), src_.get(), ke.get(), val, ndofs_, inc_ptr_.get(), inc_t_.get(),
+                           fe.get(), vec, c.stream));
 }
 
 bool ElementDiscretization::give_pattern(GPUSparseMatrix& A) {
