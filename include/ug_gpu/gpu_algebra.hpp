@@ -485,10 +485,10 @@ class BiCGStab : public ILinearOperatorInverse {
 // P1 tetrahedra with FV1 and optional full-upwind convection, Q1 hexahedra with
 // FE (2x2x2 Gauss); -div(k grad u) (+ div(v u)) = f, k per element, f constant
 // or per DoF (hexahedra: constant), homogeneous Dirichlet values on the listed
-// DoFs. The CSR pattern (every element coupling, rows sorted), the local
-// entries of every CSR entry (Q2: the slot of every local entry) and an element
-// colouring are built once on the device; an assembly forms the local matrices
-// and adds them up per entry, Q2 in one launch per colour; no atomics
+// DoFs. The CSR pattern (every element coupling, rows sorted) and the local
+// entries of every CSR entry (Q2: an element colouring and the slot of every
+// local entry) are built once on the device; an assembly forms the local
+// matrices and adds them up per entry, Q2 in one launch per colour; no atomics
 // (elem_assembly.hip).
 class ElementDiscretization {
    public:
@@ -509,7 +509,10 @@ class ElementDiscretization {
     int64_t num_elems() const { return ne_; }
     int64_t num_dofs() const { return ndofs_; }
     int64_t nnz() const { return nnz_; }
-    int num_colours() const { return (int)colour_start_.size() - 1; }
+    // of an element colouring (no two elements of a colour share a DoF); the
+    // assembly of Q2 hexahedra uses one, for other types it is made by this call.
+    // An error where an element meets more than 63 colours.
+    int num_colours() const;
     // diffusion k per element (host or device array of num_elems; nullptr: 1)
     void set_diffusion(const double* k, bool on_device = false);
     // Q2: k at the 3x3x3 Gauss points of every element (num_elems x 27, x
@@ -535,6 +538,7 @@ class ElementDiscretization {
 
    private:
     void build();
+    int colour_elements(DeviceBuffer<int32_t>& colour) const;
     // val and vec (each may be null): the matrix values and the right-hand
     // side, or with u the defect sum_e (A_e u_e - f_e)
     void run(double* val, double* vec, const double* u);
@@ -548,7 +552,8 @@ class ElementDiscretization {
     DeviceBuffer<int32_t> order_, slot_;                   // Q2: elements by colour, slots
     DeviceBuffer<int32_t> eptr_, src_, inc_ptr_, inc_t_;   // others: lists of local entries / vertices
     DeviceBuffer<double> coords_, kel_, kq_, f_dof_;
-    std::vector<int64_t> colour_start_;
+    std::vector<int64_t> colour_start_;                    // Q2
+    mutable int num_colours_ = -1;                         // not coloured yet
     double f_const_ = 0.0;
     bool has_k_ = false, has_kq_ = false, has_f_dof_ = false;
     double vel_[3] = {0.0, 0.0, 0.0};

@@ -230,12 +230,16 @@ int ugx_disc_assemble_defect(void* disc, void* d, void* u);
  * num_elems * nv^2 < 2^31.
  * The CSR pattern holds every element coupling (rows sorted by column, zero
  * couplings kept, as AddLocalMatrixToGlobal's insertion, local_algebra.h:766-789);
- * it, the CSR slot of every local entry and an element colouring are built
- * once on the device here; each assembly is one atomic-free launch per colour. */
+ * it and the list of local entries that make up each of its entries are built
+ * once on the device here (Q2: an element colouring and the CSR slot of every
+ * local entry). An assembly is two launches without atomics, all local matrices
+ * and then their sums per entry; Q2: one launch per colour. */
 void* ugx_elemdisc_create(int elem_type, int64_t num_elems, const int32_t* elem_dofs, int64_t num_dofs,
                           const double* dof_coords);
 void ugx_elemdisc_destroy(void* e);
 int64_t ugx_elemdisc_nnz(void* e);
+/* of a colouring without common DoFs (Q2: the assembly's); negative with an error
+ * where an element meets more than 63 colours */
 int ugx_elemdisc_num_colours(void* e);
 /* diffusion k per element (host array of num_elems; NULL: 1) */
 int ugx_elemdisc_set_diffusion(void* e, const double* k_host);

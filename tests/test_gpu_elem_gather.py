@@ -119,3 +119,36 @@ def test_local_matrices_are_not_kept():
     lists = ne * (4 * 8 + 4 * 64 + 4 * 8) + 8 * nnz + 32 * W ** 3
     assert held <= 1.125 * lists + (32 << 20) < lists + 512 * ne, (held, lists)
     assert keep.size() == 8
+
+
+@pytest.mark.parametrize("m", [40, 64, 65, 300])
+def test_any_number_of_elements_may_share_a_dof(m):
+    """a fan of m triangles around one DoF: the assembly needs no colours (more
+    than 63 of them are an error of num_colours alone)"""
+    print(f"case fan of {m} triangles", flush=True)
+    sys.stdout.flush()
+    import ugcore_amd as U
+    t = 2 * np.pi * np.arange(m) / m
+    X = np.concatenate([[[0.0, 0.0]], np.stack([np.cos(t), np.sin(t)], 1)])
+    E = np.stack([np.zeros(m, int), 1 + np.arange(m), 1 + (np.arange(m) + 1) % m], 1)
+    ed = U.ElementDiscretization("triangle_fv1", E, X)
+    ed.set_source(2.0)
+    A, b = U.SparseMatrix(), U.Vector(m + 1)
+    ed.assemble_linear(A, b)
+    if m <= 64:
+        assert ed.num_colours() == m                    # every two share the centre
+    else:
+        with pytest.raises(U.UGError, match="63 neighbouring colours"):
+            ed.num_colours()
+    Ke, fe, _, vol = p1(X[E], np.ones(m))
+    R, S, rb = np.zeros((m + 1, m + 1)), np.zeros((m + 1, m + 1)), np.zeros(m + 1)
+    for a in range(3):
+        np.add.at(rb, E[:, a], 2.0 * fe[:, a])
+        for c in range(3):
+            np.add.at(R, (E[:, a], E[:, c]), Ke[:, a, c])
+            np.add.at(S, (E[:, a], E[:, c]), np.abs(Ke).max(axis=(1, 2)))
+    rp, col, val = A.download_csr()
+    row = np.repeat(np.arange(m + 1), np.diff(rp))
+    # 64 operations at the condition of a fan triangle's Jacobian (about m), then a sum of up to m terms
+    assert np.all(np.abs(val - R[row, col]) <= (64 * m + m) * 2.0 ** -52 * S[row, col])
+    assert np.all(np.abs(b.numpy() - rb) <= (64 * m + m) * 2.0 ** -52 * rb.max())

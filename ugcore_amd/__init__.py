@@ -1006,7 +1006,7 @@ class ElementDiscretization:
         return lib().ugx_elemdisc_nnz(self.h)
 
     def num_colours(self):
-        return lib().ugx_elemdisc_num_colours(self.h)
+        return _check(lib().ugx_elemdisc_num_colours(self.h), "num_colours")
 
     def set_diffusion(self, k):
         if k is None:

@@ -546,7 +546,9 @@ void* ugx_elemdisc_create(int elem_type, int64_t num_elems, const int32_t* elem_
 }
 void ugx_elemdisc_destroy(void* e) { delete (ElemH*)e; }
 int64_t ugx_elemdisc_nnz(void* e) { return ((ElemH*)e)->e->nnz(); }
-int ugx_elemdisc_num_colours(void* e) { return ((ElemH*)e)->e->num_colours(); }
+int ugx_elemdisc_num_colours(void* e) {
+    return guard([&] { return ((ElemH*)e)->e->num_colours(); });
+}
 int ugx_elemdisc_set_diffusion(void* e, const double* k) {
     return guard([&] {
         ((ElemH*)e)->e->set_diffusion(k, false);

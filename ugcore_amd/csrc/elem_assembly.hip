@@ -15,10 +15,10 @@
 //   * for every CSR entry the list of local entries (e, a, b) that make it up
 //     (the sorted positions of its key, elements ascending), and for every DoF
 //     the list of local vertices (e, a);
-//   * a colouring of the elements such that no two elements of one colour
-//     share a DoF (Jones-Plassmann rounds over the DoF -> element incidence,
-//     each local maximum of a hashed priority taking the lowest colour its
-//     coloured neighbours leave free), and for Q2 hexahedra the elements sorted
+//   * for Q2 hexahedra instead a colouring of the elements such that no two
+//     elements of one colour share a DoF (Jones-Plassmann rounds over the DoF ->
+//     element incidence, each local maximum of a hashed priority taking the
+//     lowest colour its coloured neighbours leave free), and the elements sorted
 //     by colour with the slot of every local entry.
 // An assembly of the other element types is two launches without atomics: all
 // local matrices (one element per thread) into a workspace, then one thread
@@ -27,8 +27,8 @@
 // the caches; one launch per colour instead leaves the chip idle (tetrahedra
 // need about 27 colours) and reads and writes every value once per element.
 // 263,958 tetrahedra (48,132 DoFs), matrix, load vector and defect on one
-// MI355X: 786 us in colours, 120 us. Q2 hexahedra have 5.8 KB local matrices
-// from the matrix cores and keep the launch per colour.
+// MI355X: 786 us in colours, 120 us. Q2 hexahedra have local matrices of 5.8 KB
+// and keep the launch per colour.
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>

@@ -1552,10 +1552,41 @@ ElementDiscretization::ElementDiscretization(int elem_type, int64_t num_elems, c
     build();
 }
 
+// the colour of every element (no two of one colour share a DoF); the number of
+// colours: 1 + the largest
+int ElementDiscretization::colour_elements(DeviceBuffer<int32_t>& colour) const {
+    auto& c = context();
+    DeviceBuffer<int32_t> flags(2);
+    UGX_HIP(hipMemsetAsync(colour.get(), 0xff, sizeof(int32_t) * (size_t)ne_, c.stream));
+    UGX_HIP(hipMemsetAsync(flags.get(), 0, sizeof(int32_t) * 2, c.stream));
+    int32_t done[2] = {0, 0};
+    int rounds = 0;
+    while (done[0] < ne_) {
+        UGX_LAUNCH(elem_colour_round(ne_, nv_, dofs_.get(), inc_ptr_.get(), inc_t_.get(), colour.get(), flags.get(),
+                                     flags.get() + 1, c.stream));
+        flags.download(done, 2);
+        if (done[1]) throw UGError("ElementDiscretization: an element has more than 63 neighbouring colours");
+        if (++rounds > 100000) throw UGError("ElementDiscretization: the colouring does not terminate");
+    }
+    int ncol = 0;
+    std::vector<int32_t> h((size_t)ne_);
+    colour.download(h.data(), ne_);
+    for (int32_t x : h) ncol = std::max(ncol, x + 1);
+    return ncol;
+}
+
+int ElementDiscretization::num_colours() const {
+    if (num_colours_ < 0) {
+        DeviceBuffer<int32_t> colour(ne_);
+        num_colours_ = ne_ > 0 ? colour_elements(colour) : 0;
+    }
+    return num_colours_;
+}
+
 void ElementDiscretization::build() {
     auto& c = context();
     const int64_t n = ne_ * nv_ * nv_;
-    // the pattern and the slot of every local entry
+    // the pattern, and the lists of the local entries (Q2: their slots)
     size_t sort_b = 0, scan_b = 0;
     if (elem_pattern_temp_bytes(ne_, nv_, ndofs_, &sort_b, &scan_b) != 0)
         throw UGError("ElementDiscretization: sort set-up failed");
@@ -1580,47 +1611,34 @@ void ElementDiscretization::build() {
     run.release();
     idx.release();
     idx2.release();
-    // DoF -> element incidence, then the colouring rounds
+    // DoF -> element incidence
     const int64_t ni = ne_ * nv_;
     size_t inc_b = 0;
     if (elem_incidence_temp_bytes(ni, ndofs_, &inc_b) != 0 || elem_incidence_temp_bytes(ne_, 64, &sort_b) != 0)
         throw UGError("ElementDiscretization: sort set-up failed");
     DeviceBuffer<uint32_t> ikey(std::max(ni, ne_)), ikey2(std::max(ni, ne_));
-    DeviceBuffer<int32_t> iidx(std::max(ni, ne_)), inc_t(ni), inc_ptr(ndofs_ + 1), colour(ne_), flags(2), order(ne_);
+    DeviceBuffer<int32_t> iidx(std::max(ni, ne_));
     DeviceBuffer<uint8_t> itemp((int64_t)std::max(inc_b, sort_b));
-    UGX_LAUNCH(elem_incidence(ne_, nv_, ndofs_, dofs_.get(), ikey.get(), ikey2.get(), iidx.get(), inc_t.get(),
-                              itemp.get(), inc_b, inc_ptr.get(), c.stream));
-    UGX_HIP(hipMemsetAsync(colour.get(), 0xff, sizeof(int32_t) * (size_t)std::max<int64_t>(ne_, 1), c.stream));
-    UGX_HIP(hipMemsetAsync(flags.get(), 0, sizeof(int32_t) * 2, c.stream));
-    int32_t done[2] = {0, 0};
-    int rounds = 0;
-    while (done[0] < ne_) {
-        UGX_LAUNCH(elem_colour_round(ne_, nv_, dofs_.get(), inc_ptr.get(), inc_t.get(), colour.get(), flags.get(),
-                                     flags.get() + 1, c.stream));
-        flags.download(done, 2);
-        if (done[1]) throw UGError("ElementDiscretization: an element has more than 63 neighbouring colours");
-        if (++rounds > 100000) throw UGError("ElementDiscretization: the colouring does not terminate");
-    }
-    // the number of colours: 1 + the largest colour
-    int ncol = 0;
-    if (ne_ > 0) {
-        std::vector<int32_t> col_h(ne_);
-        colour.download(col_h.data(), ne_);
-        for (int32_t x : col_h) ncol = std::max(ncol, x + 1);
-    }
-    DeviceBuffer<int32_t> colour_ptr(ncol + 1);
-    UGX_LAUNCH(elem_colour_order(ne_, ncol, colour.get(), ikey.get(), ikey2.get(), iidx.get(), order.get(),
-                                 itemp.get(), sort_b, colour_ptr.get(), c.stream));
-    std::vector<int32_t> cp(ncol + 1);
-    colour_ptr.download(cp.data(), ncol + 1);
-    colour_start_.assign(cp.begin(), cp.end());
+    inc_ptr_.resize(ndofs_ + 1);
+    inc_t_.resize(ni);
+    UGX_LAUNCH(elem_incidence(ne_, nv_, ndofs_, dofs_.get(), ikey.get(), ikey2.get(), iidx.get(), inc_t_.get(),
+                              itemp.get(), inc_b, inc_ptr_.get(), c.stream));
     if (q2) {
-        order_ = std::move(order);
+        // the elements sorted by colour, the slots in that order
+        DeviceBuffer<int32_t> colour(ne_);
+        const int ncol = ne_ > 0 ? colour_elements(colour) : 0;
+        num_colours_ = ncol;
+        DeviceBuffer<int32_t> colour_ptr(ncol + 1);
+        order_.resize(ne_);
+        UGX_LAUNCH(elem_colour_order(ne_, ncol, colour.get(), ikey.get(), ikey2.get(), iidx.get(), order_.get(),
+                                     itemp.get(), sort_b, colour_ptr.get(), c.stream));
+        std::vector<int32_t> cp(ncol + 1);
+        colour_ptr.download(cp.data(), ncol + 1);
+        colour_start_.assign(cp.begin(), cp.end());
         slot_.resize(n);
         UGX_LAUNCH(elem_slots_by_position(ne_, nv_, order_.get(), slot_local.get(), slot_.get(), c.stream));
-    } else {
-        inc_ptr_ = std::move(inc_ptr);
-        inc_t_ = std::move(inc_t);
+        inc_ptr_.release();
+        inc_t_.release();
     }
     sync();
 }
