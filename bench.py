@@ -607,7 +607,7 @@ def main():
         cands.append(roofline(f"{mf_kernel}<double,5>", dir_bytes, t_dir, max(iters["f32"] - 1, 0)))
         cands.append(roofline(f"{mf_kernel}<double,2>", lat_bytes, t_lat, 1))
     else:
-        op_kernel = {"dict": "k_dict_spmv<double,false>", "sell": "k_sell_spmv<double,double,1>"}.get(
+        op_kernel = {"dict": "k_dict_spmv", "sell": "k_sell_spmv<double,double,1>"}.get(
             layout, f"k_spmv_csr<double,double,{best_lanes}>")
         cands.append(roofline(op_kernel, spmv_bytes, t_spmv, iters["f32"]))
     # the kernel with the largest share of the solve

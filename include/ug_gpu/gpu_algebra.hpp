@@ -464,8 +464,8 @@ class BiCGStab : public ILinearOperatorInverse {
    private:
     // the same iteration on lattice-ordered vectors: the cycle starts from the
     // defect that the vector update wrote in its precision and is replayed as
-    // a graph, the operator product sums its dot products, and the host reads
-    // two scalars per half step
+    // a graph, the operator product sums its dot products, and the host waits for the
+    // scalars of a half step (one copy of three or four) once per half step
     template <typename T>
     bool apply_lattice(GPUVector& x, GPUVector& b, AssembledMultiGridCycle& gmg);
     int num_restarts_ = 0;
@@ -699,8 +699,8 @@ class DomainDiscretization {
 // elements, as the reference evaluates a coefficient function), f constant.
 // Every level has the reference's LEVEL DoF order (vertices, edges, faces,
 // volumes; subset by subset in creation order), its operator is assembled by
-// the element loop (ElementDiscretization, Q2 element matrices on the matrix
-// cores) and the transfers are StdTransfer's (q2_hierarchy.hip). With
+// the element loop (ElementDiscretization, Q2 element matrices by sum
+// factorisation) and the transfers are StdTransfer's (q2_hierarchy.hip). With
 // MatrixMultiGrid they give the Q2 geometric multigrid.
 class Q2Discretization {
    public:

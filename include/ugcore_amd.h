@@ -225,7 +225,7 @@ int ugx_disc_assemble_defect(void* disc, void* d, void* u);
  * 2x2x2 Gauss (nv 8, dim 3); 3: Q2 hexahedra, FE with 3x3x3 Gauss (nv 27 in
  * the shape order of LagrangeLSFS<ReferenceHexahedron, 2>, lagrange.cpp:236-253:
  * the 8 vertices, the 12 edge midpoints, the 6 face centres, the centre;
- * dim 3; element matrices on the matrix cores, one element per wavefront;
+ * dim 3; element matrices by sum factorisation, two elements per wavefront;
  * its defect is A u - b of the assembled operator). Host arrays.
  * num_elems * nv^2 < 2^31.
  * The CSR pattern holds every element coupling (rows sorted by column, zero

@@ -4,7 +4,9 @@ operator, which a copy of the matrix selects (the copy is not the
 discretisation's assembly): steps +-1, solutions and returned defects to what a
 reduction of 1e-12 leaves; several cycles, restarts, starts with entries on the
 Dirichlet DoFs, right-hand sides one after another, and an operator renewed in
-between. Breakdowns end with false and leave x unchanged."""
+between. Breakdowns end with false on both paths: with (v, r0) = 0 in the first
+step x and the defect are those of the start, with (t, t) = 0 the first half
+step stands; a defect that is not finite ends the iteration before x changes."""
 import sys
 
 import numpy as np
@@ -99,6 +101,9 @@ def test_limits_and_non_finite_defects():
     bad[3] = np.nan
     assert not S.apply(u.Vector(N), u.Vector(values=bad))
     assert S.steps() <= 1
+    x, r = u.Vector(values=np.full(N, 0.5)), u.Vector(values=bad)
+    assert not S.apply_return_defect(x, r)
+    assert np.all(x.numpy() == 0.5) and np.isnan(r.numpy()).any() and S.steps() == 0
 
 
 def test_precision_set_after_init():
@@ -111,3 +116,44 @@ def test_precision_set_after_init():
     r = subprocess.run([client, "precision"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.count("equal") == 4
+
+
+@pytest.mark.parametrize("graphs", [True, False])
+@pytest.mark.parametrize("which,refs,scale", [("v.r0", 1, 1e-170), ("v.r0", 2, 1e-170), ("t.t", 0, 1e-150)])
+def test_breakdowns(which, refs, scale, graphs):
+    """Right-hand sides so small that a product underflows to an exact zero.
+    v.r0: (v, r0) of vectors near 1e-170. t.t: the base level's LU alone is the
+    preconditioner, so s = r - alpha A B r is rounding, 1e-16 of r, and
+    (t, t) of t = A B s is below 1e-320 where (v, r0) near 1e-300 is not; the
+    half step queued before the host has looked writes scratch only."""
+    print(f"case bicgstab breakdown {which} refs={refs} graphs={graphs}", flush=True)
+    sys.stdout.flush()
+    u = U()
+    d, A, b, rng = problem(refs, 7)
+    C = u.SparseMatrix()
+    C.set_as_copy_of(A)
+    N = d.num_dofs()
+    rhs = scale * rng.uniform(0.5, 1.5, N)
+    got = {}
+    for name, M in (("lattice", A), ("surface", C)):
+        g = u.GeometricMultiGrid(d, base_level=0, omega=0.6, graphs=graphs)
+        S = u.BiCGStab(g, max_steps=20, min_defect=0.0, reduction=0.0)
+        S.init(M)
+        for _ in range(2):                       # also with what the first left behind
+            x, r = u.Vector(N), u.Vector(values=rhs)
+            assert not S.apply_return_defect(x, r), name
+            assert S.steps() == (0 if which == "v.r0" else 1), name
+            assert np.array_equal(r.numpy(), rhs), name
+        got[name] = x.numpy()
+        # the solver is as before: an ordinary problem
+        S.set_conv_check(200, 1e-50, 1e-10)
+        y = u.Vector(N)
+        assert S.apply(y, b), name
+    if which == "v.r0":
+        assert not got["lattice"].any() and not got["surface"].any()
+    else:
+        # x = alpha B r solves the system
+        Rx = u.Vector(values=rhs)
+        A.apply_sub(Rx, u.Vector(values=got["lattice"]))
+        assert np.linalg.norm(Rx.numpy() / scale) <= 1e-12 * np.linalg.norm(rhs / scale)
+        assert np.linalg.norm((got["lattice"] - got["surface"]) / scale) <= 1e-12 * np.linalg.norm(got["surface"] / scale)

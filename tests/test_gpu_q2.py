@@ -1,5 +1,5 @@
 """Q2 hexahedron element matrices on the device (ugx_q2_hex_element_matrices,
-one element per wavefront with the FP64 matrix cores) against the oracle's
+two elements per wavefront by sum factorisation) against the oracle's
 restatement: jittered trilinear elements, boxes, a batch size that is not a
 multiple of anything, per-element and unit coefficients, the empty batch.
 Tolerance: 1e-12 relative to the largest entry of each element matrix (the

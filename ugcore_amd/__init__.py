@@ -975,10 +975,11 @@ def SaveVectorForConnectionViewer(disc, v, filename):
 
 class ElementDiscretization:
     """Element-loop assembly from caller-supplied connectivity
-    (ugx_elemdisc_*): elem_type "triangle_fv1", "tetrahedron_fv1" or
-    "hexahedron_q1"; elem_dofs [num_elems, nv] in the reference element's local
-    vertex order; dof_coords [num_dofs, dim]. The pattern, the slot of every
-    local entry and the element colouring are built on the device here."""
+    (ugx_elemdisc_*): elem_type "triangle_fv1", "tetrahedron_fv1",
+    "hexahedron_q1" or "hexahedron_q2"; elem_dofs [num_elems, nv] in the
+    reference element's local vertex order; dof_coords [num_dofs, dim]. The
+    pattern and the local entries of each of its entries (Q2: their slots and an
+    element colouring) are built on the device here."""
 
     TYPES = {"triangle_fv1": (0, 3, 2), "tetrahedron_fv1": (1, 4, 3), "hexahedron_q1": (2, 8, 3),
              "hexahedron_q2": (3, 27, 3)}

@@ -2641,11 +2641,12 @@ struct GmgImpl : public AssembledMultiGridCycle::Impl {
         }
     }
 
-    // One cycle is about 60 launches, most of them on the small coarse levels
-    // where the launch costs more than the kernel. The cycle has no host
-    // decisions and every level vector is rewritten before it is read, so it
-    // is captured once per (c, d, cd_out, partial) and replayed as one graph
-    // (kernel nodes only: the zeroing is a kernel, not a memset).
+    // One V(2,2) cycle is one launch for the coarse levels together and about
+    // six for every level above them, most of these on lattices where the launch
+    // costs more than the kernel. The cycle has no host decisions and every level
+    // vector is rewritten before it is read, so it is captured once per (c, d,
+    // cd_out, partial) and replayed as one graph (kernel nodes only: the zeroing
+    // is a kernel, not a memset).
     // FP32 levels with the fused first step can start from the caller's FP32
     // copy of the defect (rounded as the conversion would)
     bool uses_f32_defect() const override { return std::is_same<T, float>::value && first_step_fused(); }

@@ -546,8 +546,8 @@ struct Q2SlotSink {
     __device__ void fe(int a, double v) { rhs[dofs[e * 27 + a]] += v; }
 };
 
-// one colour's elements (positions pos0 .. pos0+cnt-1 of the colour order),
-// one element per wavefront
+// one colour's elements (positions pos0 .. pos0+cnt-1 of the colour order), two
+// per wavefront
 __global__ __launch_bounds__(64 * kQ2Waves, 3) void k_elem_hex_q2(int64_t ne, const int32_t* __restrict__ order,
                                                                const int32_t* __restrict__ dofs,
                                                                const double* __restrict__ coords,

@@ -94,19 +94,21 @@ int device_cus();
 // residency queries of the matrix-free kernels at lattice width W, made
 // before any cycle is captured into a graph
 int q1mf_prepare(int W);
-// whether q1mf_kernels.hip has a schedule for this lattice width: then every
-// function below applies, otherwise only q1mf_jacobi_step, q1mf_apply_sub and
-// q1mf_axpy without partial sums (the plane-by-plane kernels)
 // the coarse level's deferred last post-smoothing update sc + dinv .* sd would
 // store, with the arithmetic of k_jacobi_accumulate
 template <typename TV>
 __host__ __device__ inline TV coarse_fold(TV sc, TV dinv, TV sd) {
     return (TV)((double)sc + (double)dinv * (double)sd);
 }
+// t = P c (the coarse correction; dinv_c, sd_c: its last update folded in, or both
+// null), d -= A t, sc += t in one pass (FP32), at the widths that fit
 bool q1mf_prolong_sub_fits(int W);
 template <typename T>
 int q1mf_prolong_sub(int W, const T* cell, const T* c_coarse, const T* dinv_c, const T* sd_c, T* d, T* sc,
                      hipStream_t s);
+// whether q1mf_kernels.hip has a schedule for this lattice width: then every
+// q1mf function applies, otherwise only q1mf_jacobi_step, q1mf_apply_sub and
+// q1mf_axpy without partial sums (the plane-by-plane kernels)
 bool q1mf_fused_fits(int W);
 template <typename T>
 int q1mf_planes_jacobi_step(int W, const T* cell, const T* dinv, const T* sd_in, T* sd_out, T* sc, hipStream_t s);
@@ -169,7 +171,7 @@ template <typename T>
 int q1mf_jacobi_last(int W, const T* cell, const T* dinv, const T* sd_in, const T* sc, double* z, const double* r,
                      hipStream_t s, double* dot_partial, int* n_partial);
 // dot_partial (optional): per-block partial sums of y.x (n_partial in: capacity,
-// out: number written); needs the z-marching kernel
+// out: number written); needs q1mf_fused_fits(W)
 template <typename T>
 int q1mf_axpy(int W, const T* cell, double alpha, const T* v, double beta, const T* x, T* y, hipStream_t s,
               double* dot_partial = nullptr, int* n_partial = nullptr);
@@ -416,7 +418,7 @@ int elem_gather(int64_t nnz, const int32_t* eptr, const int32_t* src, const doub
                 const int32_t* inc_ptr, const int32_t* inc_t, const double* fe, double* vec, hipStream_t s);
 int zero_listed(int64_t n, const int32_t* idx, double* x, hipStream_t s);
 // Q2 hexahedra (27 DoFs in the local shape order of LagrangeLSFS<Hexahedron,
-// 2>): one colour, one element per wavefront (q2_kernels.hip); the
+// 2>): one colour, two elements per wavefront (q2_kernels.hip); the
 // coefficient per element (kel), per element and Gauss point (kq) or 1;
 // val (through the slots) and rhs may be null
 int elem_assemble_q2_colour(int64_t ne, const int32_t* order, const int32_t* dofs, const double* coords,
