@@ -68,9 +68,9 @@ namespace {
 // Released blocks are kept for the next buffer of about their size instead of
 // going through hipFree and hipMalloc, which map and unmap the memory: a
 // multigrid set-up allocates and frees about 60 buffers (2 GB at 128^3).
-// Renewing operator and multigrid at 128^3 on one MI355X, without and with the
-// pool: 9.9 and 3.0 ms where one problem is renewed again and again, 44.4 and
-// 3.0 ms where three are in turn.
+// Renewing operator and multigrid at 128^3 on one MI355X took 9.9 ms without the
+// pool where one problem is renewed again and again, 44.4 ms where three are in
+// turn (30 ms on another machine), and 3.0 ms with it, three in turn.
 //
 // A block released by an internal buffer may still be in use by kernels
 // queued on the library's stream: later work on that stream may have it at
